@@ -1,0 +1,61 @@
+"""Preconditioner on axes of any length against the oracle: in-register pairs,
+dense second factors (prime factors above 13), primes, and the longest axes,
+on each axis in turn."""
+import numpy as np
+import pytest
+
+from oracle import spectral
+from voxel_lmfem import materials as pm
+
+pytestmark = pytest.mark.gpu
+
+# 2 to 25: one or two small factors; 17, 19, 34 = 2*17, 37, 59*2, 61, 101, 127, 251: dense factors (odd and even);
+# 100, 125, 150, 169, 225: in-register pairs; 64, 96, 256: lengths of the four-step kernels, run through the general
+# passes; 323 = 17*19, 343 = 7*49, 512.
+LENGTHS = [2, 3, 5, 7, 9, 11, 13, 14, 17, 18, 19, 20, 21, 22, 25, 34, 37, 61, 64, 96, 100, 101, 118, 125, 127, 150, 169,
+           225, 251, 256, 323, 343, 512]
+
+
+def _check(torch, shape, h, nrhs, precisions=(("float64", 1e-11), ("float32", 5e-6))):
+    from voxel_lmfem.gpu import Cell, Preconditioner
+    print(f"case lengths shape={shape}", flush=True)
+    C = {0: dict(kind="isotropic", E=1.0, nu=0.3)}
+    field = pm.build_field(np.zeros(shape, dtype=np.int32), C)
+    cell = Cell(field, shape, h)
+    lam, mu = 2.5, 1.3
+    n = int(np.prod(shape))
+    R = np.random.default_rng(n).normal(size=(nrhs, n, 3))
+    R -= R.mean(axis=1, keepdims=True)
+    ref = np.stack([spectral.green_apply(r, shape, h, lam, mu).T for r in R])
+    r = torch.tensor(np.ascontiguousarray(R.transpose(0, 2, 1)), device="cuda")
+    for precision, tol in precisions:
+        pc = Preconditioner(cell, lam, mu, precision=precision, nrhs_max=nrhs)
+        z = pc.apply_planes(r.to(pc.dtype)).double().cpu().numpy()
+        err = np.abs(z - ref).max() / np.abs(ref).max()
+        print(f"  {precision} err {err:.2e}", flush=True)
+        assert err < tol
+        pc.close()
+    cell.close()
+
+
+@pytest.mark.parametrize("n", LENGTHS)
+def test_every_axis_length(torch_gpu, n, monkeypatch):
+    monkeypatch.setenv("VXL_FFT_FOURSTEP", "0")
+    monkeypatch.setenv("VXL_FFT_XFOURSTEP", "0")
+    h = np.array([0.7, 1.1, 0.9])
+    for shape in ((3, 5, n), (3, n, 5), (n, 5, 3)):
+        _check(torch_gpu, shape, h, 2)
+
+
+# Many columns per workgroup on all three axes at once, with partly filled last workgroups.
+@pytest.mark.parametrize("shape", [(21, 25, 18), (33, 34, 35), (37, 50, 47), (30, 118, 26)])
+def test_ragged_grids(torch_gpu, shape):
+    _check(torch_gpu, shape, np.array([1.0, 1.0, 1.5]), 2)
+
+
+# The longest axes the passes take (more than 64 KB of LDS in one workgroup).
+@pytest.mark.parametrize("shape,precision,tol", [((2, 2, 1365), "float32", 2e-5), ((1365, 2, 2), "float32", 2e-5),
+                                                 ((2, 4096, 2), "float32", 2e-5), ((2, 2, 682), "float64", 1e-10),
+                                                 ((682, 2, 2), "float64", 1e-10), ((2, 2048, 2), "float64", 1e-10)])
+def test_longest_axes(torch_gpu, shape, precision, tol):
+    _check(torch_gpu, shape, np.array([1.0, 1.0, 1.0]), 1, ((precision, tol),))

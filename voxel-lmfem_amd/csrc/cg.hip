@@ -94,12 +94,13 @@ update_r_kernel(T* r, const T* q, int64_t len, const double* alpha, double* part
 // direction slot that a system never wrote does not reach its x64.
 template <typename T, bool kAssign>
 __global__ void __launch_bounds__(kBlock)
-flush_kernel(double* x64, DirectionSet<T> d, const double* alpha, int nrhs, int64_t len) {
+flush_kernel(double* x64, DirectionSet<T> d, const double* alpha, const double* unscale, int nrhs, int64_t len) {
   const int k = blockIdx.y;
   const int64_t off = int64_t(k) * len;
+  const double us = unscale ? unscale[k] : 1.0;
   double a[kMaxDirections];
 #pragma unroll
-  for (int t = 0; t < kMaxDirections; ++t) a[t] = t < d.count ? alpha[t * nrhs + k] : 0.0;
+  for (int t = 0; t < kMaxDirections; ++t) a[t] = t < d.count ? us * alpha[t * nrhs + k] : 0.0;
   if constexpr (!kAssign) {  // no step pending for this system: x64 stays
     bool any = false;
 #pragma unroll
@@ -134,12 +135,13 @@ __device__ __forceinline__ void load4(const double* p, double (&o)[4]) {
 
 template <typename T, bool kAssign>
 __global__ void __launch_bounds__(kBlock)
-flush4_kernel(double* x64, DirectionSet<T> d, const double* alpha, int nrhs, int64_t len) {
+flush4_kernel(double* x64, DirectionSet<T> d, const double* alpha, const double* unscale, int nrhs, int64_t len) {
   const int k = blockIdx.y;
   const int64_t off = int64_t(k) * len;
+  const double us = unscale ? unscale[k] : 1.0;
   double a[kMaxDirections];
 #pragma unroll
-  for (int t = 0; t < kMaxDirections; ++t) a[t] = t < d.count ? alpha[t * nrhs + k] : 0.0;
+  for (int t = 0; t < kMaxDirections; ++t) a[t] = t < d.count ? us * alpha[t * nrhs + k] : 0.0;
   if constexpr (!kAssign) {  // no step pending for this system (converged or inactive): x64 stays
     bool any = false;
 #pragma unroll
@@ -228,16 +230,26 @@ residual_kernel(double* r, const double* f, const double* q, float* r32, int64_t
   if (threadIdx.x == 0) partial[int64_t(k) * gridDim.x + blockIdx.x] = acc;
 }
 
-// x64 += x32; x32 = 0.
+// x64 += unscale x32; x32 = 0.
 __global__ void __launch_bounds__(kBlock)
-accumulate_kernel(double* x64, float* x32, int64_t len, const int* active) {
+accumulate_kernel(double* x64, float* x32, const double* unscale, int64_t len, const int* active) {
   const int k = blockIdx.y;
   if (active && !active[k]) return;
+  const double us = unscale ? unscale[k] : 1.0;
   const int64_t off = int64_t(k) * len;
   for (int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x; i < len; i += int64_t(gridDim.x) * kBlock) {
-    x64[off + i] += double(x32[off + i]);
+    x64[off + i] = fma(us, double(x32[off + i]), x64[off + i]);
     x32[off + i] = 0.0f;
   }
+}
+
+__global__ void __launch_bounds__(kBlock)
+scaled_residual_kernel(const double* f, float* r32, const double* scale, int64_t len) {
+  const int k = blockIdx.y;
+  const double s = scale[k];
+  const int64_t off = int64_t(k) * len;
+  for (int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x; i < len; i += int64_t(gridDim.x) * kBlock)
+    r32[off + i] = float(s * f[off + i]);
 }
 
 template <typename A, typename B>
@@ -427,27 +439,27 @@ template int launch_update_r<double>(double*, const double*, int64_t, int, const
                                      hipStream_t);
 
 template <typename T>
-int launch_flush(double* x64, const DirectionSet<T>& d, const double* alpha, int nrhs, int64_t len, bool assign,
-                 hipStream_t s) {
+int launch_flush(double* x64, const DirectionSet<T>& d, const double* alpha, const double* unscale, int nrhs,
+                 int64_t len, bool assign, hipStream_t s) {
   if (d.count <= 0) return VXL_OK;
   if (d.count > kMaxDirections) return fail("too many stored search directions");
   const bool v4 = len % 4 == 0;
   const dim3 g = vgrid(v4 ? len / 4 : len, nrhs);
   if (v4 && assign)
-    hipLaunchKernelGGL((flush4_kernel<T, true>), g, dim3(kBlock), 0, s, x64, d, alpha, nrhs, len);
+    hipLaunchKernelGGL((flush4_kernel<T, true>), g, dim3(kBlock), 0, s, x64, d, alpha, unscale, nrhs, len);
   else if (v4)
-    hipLaunchKernelGGL((flush4_kernel<T, false>), g, dim3(kBlock), 0, s, x64, d, alpha, nrhs, len);
+    hipLaunchKernelGGL((flush4_kernel<T, false>), g, dim3(kBlock), 0, s, x64, d, alpha, unscale, nrhs, len);
   else if (assign)
-    hipLaunchKernelGGL((flush_kernel<T, true>), g, dim3(kBlock), 0, s, x64, d, alpha, nrhs, len);
+    hipLaunchKernelGGL((flush_kernel<T, true>), g, dim3(kBlock), 0, s, x64, d, alpha, unscale, nrhs, len);
   else
-    hipLaunchKernelGGL((flush_kernel<T, false>), g, dim3(kBlock), 0, s, x64, d, alpha, nrhs, len);
+    hipLaunchKernelGGL((flush_kernel<T, false>), g, dim3(kBlock), 0, s, x64, d, alpha, unscale, nrhs, len);
   VXL_HIP(hipGetLastError());
   return VXL_OK;
 }
-template int launch_flush<float>(double*, const DirectionSet<float>&, const double*, int, int64_t, bool,
+template int launch_flush<float>(double*, const DirectionSet<float>&, const double*, const double*, int, int64_t, bool,
                                  hipStream_t);
-template int launch_flush<double>(double*, const DirectionSet<double>&, const double*, int, int64_t, bool,
-                                  hipStream_t);
+template int launch_flush<double>(double*, const DirectionSet<double>&, const double*, const double*, int, int64_t,
+                                  bool, hipStream_t);
 
 template <typename T>
 int launch_update_xr(T* x, T* r, const T* p, const T* q, int64_t len, int nrhs, const double* alpha,
@@ -468,8 +480,15 @@ int launch_residual(double* r, const double* f, const double* q, float* r32, int
   return VXL_OK;
 }
 
-int launch_accumulate(double* x64, float* x32, int64_t len, int nrhs, const int* active, hipStream_t s) {
-  hipLaunchKernelGGL(accumulate_kernel, vgrid(len, nrhs), dim3(kBlock), 0, s, x64, x32, len, active);
+int launch_accumulate(double* x64, float* x32, const double* unscale, int64_t len, int nrhs, const int* active,
+                      hipStream_t s) {
+  hipLaunchKernelGGL(accumulate_kernel, vgrid(len, nrhs), dim3(kBlock), 0, s, x64, x32, unscale, len, active);
+  VXL_HIP(hipGetLastError());
+  return VXL_OK;
+}
+
+int launch_scaled_residual(const double* f, float* r32, const double* scale, int64_t len, int nrhs, hipStream_t s) {
+  hipLaunchKernelGGL(scaled_residual_kernel, vgrid(len, nrhs), dim3(kBlock), 0, s, f, r32, scale, len);
   VXL_HIP(hipGetLastError());
   return VXL_OK;
 }

@@ -11,20 +11,20 @@
 // (no Nk-sized coefficient cache); the k = 0 mode is removed and 1/N of the
 // inverse transform is folded in.
 //
-// Transforms are hand-written mixed-radix Stockham FFTs on LDS pencils
-// (radix 8, 4, 2, 3, 5, 7, generic odd primes <= 13, direct DFT otherwise;
-// twiddles from a host table filled with std::cos/std::sin).  Five passes per
-// apply, spectrum stored as S[r][z][y][kx][c] with the three components
-// interleaved so the z pass sees whole 3-vectors:
+// Transforms are hand-written two-step FFTs on LDS pencils: axes of 2^a and of
+// 2^a times 3 or 5 run the four-step kernels below with compile-time factors,
+// every other length the general passes of vxl_fftgen.h (twiddles from a host
+// table filled with std::cos/std::sin).  Five passes per apply, spectrum
+// stored as S[r][z][y][kx][c] with the three components interleaved so the z
+// pass sees whole 3-vectors:
 //   1. x: real-to-complex (two real rows per complex FFT), half spectrum
 //   2. y: forward complex
 //   3. z: forward complex, 3x3 Green solve, inverse complex (one pass)
 //   4. y: inverse complex
 //   5. x: complex-to-real (two rows per complex FFT)
 #include <functional>
-#include <type_traits>
 
-#include "vxl_cg.h"
+#include "vxl_fft.h"
 
 #include <algorithm>
 #include <cmath>
@@ -32,442 +32,6 @@
 
 namespace vxl {
 namespace {
-
-constexpr int kMaxStages = 12;
-constexpr int kThreads = 256;
-
-struct Plan1D {
-  int n;
-  int stages;  // 0 => direct DFT
-  int radix[kMaxStages];
-};
-
-Plan1D make_plan(int n) {
-  Plan1D p;
-  p.n = n;
-  p.stages = 0;
-  int m = n;
-  const int order[] = {8, 4, 2, 3, 5, 7, 11, 13};
-  for (int r : order) {
-    while (m % r == 0 && p.stages < kMaxStages) {
-      if (r == 8 || r == 4) {
-        // keep powers of two in 8/4/2 chunks
-      }
-      p.radix[p.stages++] = r;
-      m /= r;
-    }
-  }
-  if (m != 1) p.stages = 0;  // prime factor > 13: direct DFT
-  return p;
-}
-
-template <typename T> struct CT;
-template <> struct CT<float> { using type = float2; };
-template <> struct CT<double> { using type = double2; };
-
-
-// Spectrum storage element: the compute complex type itself, or a pair of
-// BF16 values (FP32 arithmetic, half the spectrum traffic; round to nearest
-// even on store).
-struct bf16x2 {
-  unsigned short x, y;
-};
-__device__ __forceinline__ unsigned short to_bf16(float f) {
-  const unsigned int b = __float_as_uint(f);
-  return static_cast<unsigned short>((b + 0x7FFFu + ((b >> 16) & 1u)) >> 16);
-}
-__device__ __forceinline__ float from_bf16(unsigned short h) { return __uint_as_float(static_cast<unsigned int>(h) << 16); }
-template <typename C, typename SC>
-__device__ __forceinline__ C sload(const SC* p) {
-  if constexpr (std::is_same<SC, bf16x2>::value) {
-    const bf16x2 v = *p;
-    return C{from_bf16(v.x), from_bf16(v.y)};
-  } else {
-    return *p;
-  }
-}
-template <typename C, typename SC>
-__device__ __forceinline__ void sstore(SC* p, C v) {
-  if constexpr (std::is_same<SC, bf16x2>::value) {
-    *p = bf16x2{to_bf16(v.x), to_bf16(v.y)};
-  } else {
-    *p = v;
-  }
-}
-template <typename C>
-__device__ __forceinline__ C cadd(C a, C b) { return {a.x + b.x, a.y + b.y}; }
-template <typename C>
-__device__ __forceinline__ C csub(C a, C b) { return {a.x - b.x, a.y - b.y}; }
-template <typename C>
-__device__ __forceinline__ C cmul(C a, C b) { return {a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x}; }
-template <typename C>
-__device__ __forceinline__ C cconj(C a) { return {a.x, -a.y}; }
-// multiply by -i (forward) or +i (inverse)
-template <bool INV, typename C>
-__device__ __forceinline__ C rot90(C a) { return INV ? C{-a.y, a.x} : C{a.y, -a.x}; }
-
-// In-register DFTs of size R with kernel exp(-+2 pi i / R).
-template <bool INV, typename T, typename C>
-__device__ __forceinline__ void dft2(C* v) {
-  C a = v[0], b = v[1];
-  v[0] = cadd(a, b);
-  v[1] = csub(a, b);
-}
-template <bool INV, typename T, typename C>
-__device__ __forceinline__ void dft4(C* v) {
-  C a0 = cadd(v[0], v[2]), a1 = csub(v[0], v[2]);
-  C a2 = cadd(v[1], v[3]), a3 = rot90<INV>(csub(v[1], v[3]));
-  v[0] = cadd(a0, a2);
-  v[2] = csub(a0, a2);
-  v[1] = cadd(a1, a3);
-  v[3] = csub(a1, a3);
-}
-template <bool INV, typename T, typename C>
-__device__ __forceinline__ void dft8(C* v) {
-  const T s = T(0.70710678118654752440084436210484903928);
-  C e[4] = {v[0], v[2], v[4], v[6]}, o[4] = {v[1], v[3], v[5], v[7]};
-  dft4<INV, T>(e);
-  dft4<INV, T>(o);
-  // twiddles w^k, k = 0..3, w = exp(-+ i pi/4)
-  C t1 = INV ? C{s * (o[1].x - o[1].y), s * (o[1].x + o[1].y)}
-             : C{s * (o[1].x + o[1].y), s * (o[1].y - o[1].x)};
-  C t2 = rot90<INV>(o[2]);
-  C t3 = INV ? C{-s * (o[3].x + o[3].y), s * (o[3].x - o[3].y)}
-             : C{s * (o[3].y - o[3].x), -s * (o[3].x + o[3].y)};
-  v[0] = cadd(e[0], o[0]);
-  v[4] = csub(e[0], o[0]);
-  v[1] = cadd(e[1], t1);
-  v[5] = csub(e[1], t1);
-  v[2] = cadd(e[2], t2);
-  v[6] = csub(e[2], t2);
-  v[3] = cadd(e[3], t3);
-  v[7] = csub(e[3], t3);
-}
-template <bool INV, typename T, typename C>
-__device__ __forceinline__ void dft3(C* v) {
-  const T c = T(-0.5), s = T(INV ? 0.86602540378443864676372317075293618347
-                                  : -0.86602540378443864676372317075293618347);
-  C a = cadd(v[1], v[2]), b = csub(v[1], v[2]);
-  C m = {v[0].x + c * a.x, v[0].y + c * a.y};
-  C jb = {-s * b.y, s * b.x};
-  v[0] = cadd(v[0], a);
-  v[1] = cadd(m, jb);
-  v[2] = csub(m, jb);
-}
-// Radix 5: with a1 = x1 + x4, b1 = x1 - x4, a2 = x2 + x3, b2 = x2 - x3 and
-// theta = 2 pi / 5, X1,4 = x0 + a1 cos(theta) + a2 cos(2 theta) -+ i (b1 sin(theta)
-// + b2 sin(2 theta)), X2,3 = x0 + a1 cos(2 theta) + a2 cos(theta) -+ i (b1 sin(2 theta)
-// - b2 sin(theta)) (signs of i flipped for the inverse).
-template <bool INV, typename T, typename C>
-__device__ __forceinline__ void dft5(C* v) {
-  const T c1 = T(0.30901699437494742410229341718281905886), c2 = T(-0.80901699437494742410229341718281905886);
-  const T s1 = T(0.95105651629515357211643933337938214340), s2 = T(0.58778525229247312916870595463907276860);
-  const C a1 = cadd(v[1], v[4]), b1 = csub(v[1], v[4]), a2 = cadd(v[2], v[3]), b2 = csub(v[2], v[3]);
-  const C t1 = {v[0].x + c1 * a1.x + c2 * a2.x, v[0].y + c1 * a1.y + c2 * a2.y};
-  const C t2 = {v[0].x + c2 * a1.x + c1 * a2.x, v[0].y + c2 * a1.y + c1 * a2.y};
-  const C u1 = rot90<INV>(C{s1 * b1.x + s2 * b2.x, s1 * b1.y + s2 * b2.y});
-  const C u2 = rot90<INV>(C{s2 * b1.x - s1 * b2.x, s2 * b1.y - s1 * b2.y});
-  v[0] = cadd(v[0], cadd(a1, a2));
-  v[1] = cadd(t1, u1);
-  v[4] = csub(t1, u1);
-  v[2] = cadd(t2, u2);
-  v[3] = csub(t2, u2);
-}
-// Odd prime radix R via the n-point twiddle table (w[k] = exp(-2 pi i k/n)).
-template <bool INV, int R, typename C>
-__device__ __forceinline__ void dft_prime(C* v, const C* w, int n) {
-  C out[R];
-  const int step = n / R;
-#pragma unroll
-  for (int k = 0; k < R; ++k) {
-    C acc = v[0];
-#pragma unroll
-    for (int r = 1; r < R; ++r) {
-      C tw = w[((r * k) % R) * step];
-      if (INV) tw = cconj(tw);
-      acc = cadd(acc, cmul(v[r], tw));
-    }
-    out[k] = acc;
-  }
-#pragma unroll
-  for (int k = 0; k < R; ++k) v[k] = out[k];
-}
-
-// One Stockham radix-R stage over P pencils stored column-fastest: element e
-// of pencil p lives at X[e * P + p], so consecutive threads (consecutive p)
-// touch consecutive LDS words on every read and write (no bank conflicts) and
-// tiles keep the global row order.  Butterfly j reads e = j + r n/R, applies
-// w^(r (j mod Ns) n/(Ns R)), transforms, and writes e = (j/Ns) Ns R + (j mod Ns) + r Ns.
-template <bool INV, typename T, int R>
-__device__ __forceinline__ void stockham_stage(const typename CT<T>::type* A, typename CT<T>::type* B,
-                                               int P, int n, int Ns, const typename CT<T>::type* w) {
-  using C = typename CT<T>::type;
-  const int nb = n / R;
-  const int tstep = n / (Ns * R);
-  for (int idx = threadIdx.x; idx < P * nb; idx += blockDim.x) {
-    const int j = idx / P, p = idx - j * P;
-    const int jm = j % Ns;
-    C v[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      C x = A[(j + r * nb) * P + p];
-      if (r > 0 && jm > 0) {
-        C tw = w[r * jm * tstep];
-        if (INV) tw = cconj(tw);
-        x = cmul(x, tw);
-      }
-      v[r] = x;
-    }
-    if constexpr (R == 2) dft2<INV, T>(v);
-    else if constexpr (R == 3) dft3<INV, T>(v);
-    else if constexpr (R == 4) dft4<INV, T>(v);
-    else if constexpr (R == 8) dft8<INV, T>(v);
-    else dft_prime<INV, R>(v, w, n);
-    const int base = (j / Ns) * Ns * R + jm;
-#pragma unroll
-    for (int r = 0; r < R; ++r) B[(base + r * Ns) * P + p] = v[r];
-  }
-}
-
-// Batched in-LDS FFT of P pencils of length n, column-fastest layout
-// (element e of pencil p at X[e * P + p]).  A holds the input; returns the
-// buffer (A or B) holding the output.  All threads of the block must call it.
-template <bool INV, typename T>
-__device__ typename CT<T>::type* lds_fft(typename CT<T>::type* A, typename CT<T>::type* B, int P,
-                                         const Plan1D& plan, const typename CT<T>::type* w) {
-  using C = typename CT<T>::type;
-  const int n = plan.n;
-  const int tid = threadIdx.x, nt = blockDim.x;
-  if (plan.stages == 0) {  // direct DFT
-    for (int idx = tid; idx < P * n; idx += nt) {
-      const int k = idx / P, p = idx - k * P;
-      C acc = {T(0), T(0)};
-      for (int j = 0; j < n; ++j) {
-        C tw = w[(int64_t(j) * k) % n];
-        if (INV) tw = cconj(tw);
-        acc = cadd(acc, cmul(A[j * P + p], tw));
-      }
-      B[k * P + p] = acc;
-    }
-    __syncthreads();
-    return B;
-  }
-  int Ns = 1;
-  for (int s = 0; s < plan.stages; ++s) {
-    const int R = plan.radix[s];
-    switch (R) {
-      case 2: stockham_stage<INV, T, 2>(A, B, P, n, Ns, w); break;
-      case 3: stockham_stage<INV, T, 3>(A, B, P, n, Ns, w); break;
-      case 4: stockham_stage<INV, T, 4>(A, B, P, n, Ns, w); break;
-      case 5: stockham_stage<INV, T, 5>(A, B, P, n, Ns, w); break;
-      case 7: stockham_stage<INV, T, 7>(A, B, P, n, Ns, w); break;
-      case 8: stockham_stage<INV, T, 8>(A, B, P, n, Ns, w); break;
-      case 11: stockham_stage<INV, T, 11>(A, B, P, n, Ns, w); break;
-      default: stockham_stage<INV, T, 13>(A, B, P, n, Ns, w); break;
-    }
-    __syncthreads();
-    C* t = A;
-    A = B;
-    B = t;
-    Ns *= R;
-  }
-  return A;
-}
-
-struct Axes {
-  Plan1D px, py, pz;
-};
-
-template <typename T>
-struct Tables {
-  const typename CT<T>::type* wx;
-  const typename CT<T>::type* wy;
-  const typename CT<T>::type* wz;
-  const T* gx;  // 7 x (nx/2+1): 1/m, D, v, d (FI symbol); 2 sin(t/2)/h, cos(t/2), sin(t/2) (C3D8R-HG)
-  const T* gy;
-  const T* gz;
-  T hg0;        // > 0: C3D8R-HG symbol with hourglass penalty hg0 = s(C0) / V
-};
-
-// ---- pass 1: x real-to-complex ---------------------------------------------
-// Row pair (rho, rho+1) over the flattened (z, y) row index; three complex
-// pencils per pair: c0+i c1 of row rho, c0+i c1 of row rho+1, c2(rho)+i c2(rho+1).
-template <typename T>
-__global__ void __launch_bounds__(kThreads)
-fft_x_r2c(const T* __restrict__ r, typename CT<T>::type* __restrict__ S, int nx, int64_t rows,
-          int nxh, int pairs_per_block, Axes ax, Tables<T> tb, int64_t field_stride,
-          int64_t spec_stride, const int* active) {
-  using C = typename CT<T>::type;
-  extern __shared__ double2 smem_raw[];
-  if (active && !active[blockIdx.y]) return;
-  C* A = reinterpret_cast<C*>(smem_raw);
-  const int P = 3 * pairs_per_block;
-  C* B = A + P * nx;
-  const int64_t n = rows * nx;
-  const T* f = r + int64_t(blockIdx.y) * field_stride;
-  C* out = S + int64_t(blockIdx.y) * spec_stride;
-  const int64_t pair0 = int64_t(blockIdx.x) * pairs_per_block;
-  auto fetch = [&](int64_t i) -> T { return f[i]; };
-  for (int idx = threadIdx.x; idx < pairs_per_block * nx; idx += blockDim.x) {
-    const int pp = idx / nx, x = idx % nx;
-    const int64_t rho = 2 * (pair0 + pp);
-    const bool has0 = rho < rows, has1 = rho + 1 < rows;
-    T v00 = 0, v01 = 0, v10 = 0, v11 = 0, v20 = 0, v21 = 0;
-    if (has0) {
-      v00 = fetch(rho * nx + x);
-      v01 = fetch(n + rho * nx + x);
-      v20 = fetch(2 * n + rho * nx + x);
-    }
-    if (has1) {
-      v10 = fetch((rho + 1) * nx + x);
-      v11 = fetch(n + (rho + 1) * nx + x);
-      v21 = fetch(2 * n + (rho + 1) * nx + x);
-    }
-    A[x * P + 3 * pp + 0] = C{v00, v01};
-    A[x * P + 3 * pp + 1] = C{v10, v11};
-    A[x * P + 3 * pp + 2] = C{v20, v21};
-  }
-  __syncthreads();
-  C* F = lds_fft<false, T>(A, B, P, ax.px, tb.wx);
-  for (int idx = threadIdx.x; idx < pairs_per_block * nxh; idx += blockDim.x) {
-    const int pp = idx / nxh, k = idx % nxh;
-    const int64_t rho = 2 * (pair0 + pp);
-    const int km = k == 0 ? 0 : nx - k;
-    C sp[3][2];  // [pencil][real row 0/1]
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const C a = F[k * P + 3 * pp + q];
-      const C b = cconj(F[km * P + 3 * pp + q]);
-      const C s = cadd(a, b), d = csub(a, b);
-      sp[q][0] = C{T(0.5) * s.x, T(0.5) * s.y};
-      sp[q][1] = C{T(0.5) * d.y, T(-0.5) * d.x};  // d / (2i)
-    }
-    if (rho < rows) {
-      C* o = out + (rho * nxh + k) * 3;
-      o[0] = sp[0][0];
-      o[1] = sp[0][1];
-      o[2] = sp[2][0];
-    }
-    if (rho + 1 < rows) {
-      C* o = out + ((rho + 1) * nxh + k) * 3;
-      o[0] = sp[1][0];
-      o[1] = sp[1][1];
-      o[2] = sp[2][1];
-    }
-  }
-}
-
-// ---- pass 5: x complex-to-real -----------------------------------------------
-// kDir: the output is the CG search direction p = z + beta[rhs] p_old with
-// p_old read from pin (pin == z: in place; beta = 0: p = z, p_old not read).
-template <typename T, bool kDir>
-__global__ void __launch_bounds__(kThreads)
-fft_x_c2r(const typename CT<T>::type* __restrict__ S, T* z, int nx, int64_t rows,
-          int nxh, int pairs_per_block, Axes ax, Tables<T> tb, int64_t field_stride,
-          int64_t spec_stride, const int* active, const double* beta, const T* pin) {
-  using C = typename CT<T>::type;
-  extern __shared__ double2 smem_raw[];
-  if (active && !active[blockIdx.y]) return;
-  C* A = reinterpret_cast<C*>(smem_raw);
-  const int P = 3 * pairs_per_block;
-  C* B = A + P * nx;
-  const int64_t n = rows * nx;
-  T* f = z + int64_t(blockIdx.y) * field_stride;
-  const C* in = S + int64_t(blockIdx.y) * spec_stride;
-  const int64_t pair0 = int64_t(blockIdx.x) * pairs_per_block;
-  const bool even = (nx % 2) == 0;
-  for (int idx = threadIdx.x; idx < pairs_per_block * nx; idx += blockDim.x) {
-    const int pp = idx / nx, k = idx % nx;
-    const int64_t rho = 2 * (pair0 + pp);
-    const bool mirror = k >= nxh;
-    const int kk = mirror ? nx - k : k;
-    const bool realonly = kk == 0 || (even && kk == nx / 2);
-    C x[2][3];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int64_t row = rho + h;
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        C v = {T(0), T(0)};
-        if (row < rows) v = in[(row * nxh + kk) * 3 + c];
-        if (realonly) v.y = T(0);
-        if (mirror) v = cconj(v);
-        x[h][c] = v;
-      }
-    }
-    // pencil = X0 + i X1
-    A[k * P + 3 * pp + 0] = C{x[0][0].x - x[0][1].y, x[0][0].y + x[0][1].x};
-    A[k * P + 3 * pp + 1] = C{x[1][0].x - x[1][1].y, x[1][0].y + x[1][1].x};
-    A[k * P + 3 * pp + 2] = C{x[0][2].x - x[1][2].y, x[0][2].y + x[1][2].x};
-  }
-  __syncthreads();
-  C* F = lds_fft<true, T>(A, B, P, ax.px, tb.wx);
-  const T b = kDir ? T(beta[blockIdx.y]) : T(0);
-  const bool keep = kDir && b != T(0);
-  const T* g = (pin ? pin : z) + int64_t(blockIdx.y) * field_stride;
-  auto put = [&](int64_t i, T v) { f[i] = keep ? fma(b, g[i], v) : v; };
-  for (int idx = threadIdx.x; idx < pairs_per_block * nx; idx += blockDim.x) {
-    const int pp = idx / nx, x = idx % nx;
-    const int64_t rho = 2 * (pair0 + pp);
-    const C a = F[x * P + 3 * pp + 0], bb = F[x * P + 3 * pp + 1], c = F[x * P + 3 * pp + 2];
-    if (rho < rows) {
-      put(rho * nx + x, a.x);
-      put(n + rho * nx + x, a.y);
-      put(2 * n + rho * nx + x, c.x);
-    }
-    if (rho + 1 < rows) {
-      put((rho + 1) * nx + x, bb.x);
-      put(n + (rho + 1) * nx + x, bb.y);
-      put(2 * n + (rho + 1) * nx + x, c.y);
-    }
-  }
-}
-
-// ---- pass 2/4: y complex ------------------------------------------------------
-// Plane (r, z) is ny rows x W columns (W = 3*nxh); a block transforms TJ
-// consecutive columns.
-template <bool INV, typename T>
-__global__ void __launch_bounds__(kThreads)
-fft_y(typename CT<T>::type* __restrict__ S, int ny, int nz, int W, int TJ, Axes ax, Tables<T> tb,
-      int64_t spec_stride, const int* active) {
-  using C = typename CT<T>::type;
-  extern __shared__ double2 smem_raw[];
-  if (active && !active[blockIdx.z]) return;
-  C* A = reinterpret_cast<C*>(smem_raw);
-  C* B = A + TJ * ny;
-  const int j0 = blockIdx.x * TJ;
-  const int z = blockIdx.y;
-  const int tj = min(TJ, W - j0);
-  C* plane = S + int64_t(blockIdx.z) * spec_stride + int64_t(z) * ny * W;
-  for (int idx = threadIdx.x; idx < ny * TJ; idx += blockDim.x) {
-    const int y = idx / TJ, j = idx % TJ;
-    A[y * TJ + j] = j < tj ? plane[int64_t(y) * W + j0 + j] : C{T(0), T(0)};
-  }
-  __syncthreads();
-  C* F = lds_fft<INV, T>(A, B, TJ, ax.py, tb.wy);
-  for (int idx = threadIdx.x; idx < ny * TJ; idx += blockDim.x) {
-    const int y = idx / TJ, j = idx % TJ;
-    if (j < tj) plane[int64_t(y) * W + j0 + j] = F[y * TJ + j];
-  }
-}
-
-// Reciprocal for the Green solve: the hardware estimate (<= 1 ulp) in FP32,
-// exact division in FP64.
-__device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
-__device__ __forceinline__ double rcp(double x) { return 1.0 / x; }
-
-// Per-axis factors of the Green symbol at one wavenumber: table columns 0-3
-// (1/m, D, v, d) for the FI element, columns 4-6 (S, c, s) in a, b, c for
-// C3D8R-HG.
-template <typename T>
-struct AxisF {
-  T a, b, c, d;
-};
-template <typename T>
-__device__ __forceinline__ AxisF<T> axis_factors(const T* g, int n, int k, bool hg) {
-  if (hg) return {g[4 * n + k], g[5 * n + k], g[6 * n + k], T(0)};
-  return {g[k], g[n + k], g[2 * n + k], g[3 * n + k]};
-}
 
 // Green solve at one wavevector (kx, ky, kz), in place:
 //   out = 1/(t N) [q/E - gamma (v/E) (v . q/E)],  E_i = mu sum D + (lam+mu) d_i,
@@ -557,69 +121,6 @@ __device__ __forceinline__ double green_solve(C& q0, C& q1, C& q2, const Tables<
   return green_point<T>(q0, q1, q2, X, Y, Z, lam, mu, inv_vn);
 }
 
-// ---- pass 3: z forward, Green solve, z inverse ---------------------------------
-// kDot: r . z by Parseval, sum over the half spectrum of w(kx) Re(conj(r^) z^)
-// with w = 1 at kx = 0 and kx = nyq (nx even), 2 elsewhere; z^ = G r^ already
-// carries the 1/N of the inverse transform, so the sum equals the real-space
-// r . z.  One FP64 partial per workgroup at
-// partial[(rhs * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x].
-template <typename T, bool kDot>
-__global__ void __launch_bounds__(kThreads)
-fft_z_green(typename CT<T>::type* __restrict__ S, int ny, int nz, int nxh, int TK, Axes ax,
-            Tables<T> tb, T lam, T mu, T inv_vn, int64_t spec_stride, const int* active, int nyq,
-            double* partial, const double* media, int group_rhs) {
-  using C = typename CT<T>::type;
-  extern __shared__ double2 smem_raw[];
-  __shared__ double red[kThreads / 64];
-  if (active && !active[blockIdx.z]) return;
-  if (media) {  // stacked cells: this right-hand side's reference medium
-    lam = T(media[2 * (blockIdx.z / group_rhs)]);
-    mu = T(media[2 * (blockIdx.z / group_rhs) + 1]);
-  }
-  C* A = reinterpret_cast<C*>(smem_raw);
-  const int TJ = 3 * TK;
-  C* B = A + TJ * nz;
-  const int k0 = blockIdx.x * TK;
-  const int y = blockIdx.y;
-  const int tk = min(TK, nxh - k0);
-  const int W = 3 * nxh;
-  const int64_t zstride = int64_t(ny) * W;
-  C* col = S + int64_t(blockIdx.z) * spec_stride + int64_t(y) * W + 3 * k0;
-  for (int idx = threadIdx.x; idx < nz * TJ; idx += blockDim.x) {
-    const int z = idx / TJ, j = idx % TJ;
-    A[z * TJ + j] = j < 3 * tk ? col[z * zstride + j] : C{T(0), T(0)};
-  }
-  __syncthreads();
-  C* F = lds_fft<false, T>(A, B, TJ, ax.pz, tb.wz);
-  C* G = F == A ? B : A;
-  // Green solve per (kz, ky, kx), in place in F.
-  const bool hg = tb.hg0 > T(0);
-  const AxisF<T> ay = axis_factors(tb.gy, ny, y, hg);
-  double dot = 0.0;
-  for (int idx = threadIdx.x; idx < nz * TK; idx += blockDim.x) {
-    const int kz = idx / TK, kk = idx % TK;
-    if (kk >= tk) continue;
-    const int kx = k0 + kk;
-    const double d = green_solve<T>(F[kz * TJ + 3 * kk + 0], F[kz * TJ + 3 * kk + 1], F[kz * TJ + 3 * kk + 2],
-                                    tb, axis_factors(tb.gx, nxh, kx, hg), ay, axis_factors(tb.gz, nz, kz, hg),
-                                    lam, mu, inv_vn);
-    if constexpr (kDot) dot += (kx == 0 || kx == nyq) ? d : 2.0 * d;
-  }
-  if constexpr (kDot) {
-    const double total = block_reduce_sum<kThreads>(dot, red);
-    if (threadIdx.x == 0)
-      partial[(int64_t(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x] = total;
-  } else {
-    __syncthreads();
-  }
-  C* H = lds_fft<true, T>(F, G, TJ, ax.pz, tb.wz);
-  for (int idx = threadIdx.x; idx < nz * TJ; idx += blockDim.x) {
-    const int z = idx / TJ, j = idx % TJ;
-    if (j < 3 * tk) col[z * zstride + j] = H[z * TJ + j];
-  }
-}
-
-
 // ---- four-step pencil FFTs for axes of 2^a (times 3 or 5) -----------------------
 // n = N1 * N2.  Step 1: thread t < N2 of a column holds x[t + N2 k1] (k1 < N1),
 // transforms over k1, multiplies by w_n^(j1 t) and writes to LDS; step 2:
@@ -628,97 +129,6 @@ fft_z_green(typename CT<T>::type* __restrict__ S, int ny, int nz, int nxh, int T
 // column p at L[e * TJ + p]) so every LDS access is conflict-minimal and every
 // global row segment is TJ contiguous complex values.  Twiddles come from the
 // axis table w[k] = exp(-2 pi i k / n).
-
-// cos and sin of x in [0, pi), evaluated at compile time: reduced to
-// [0, pi/4] by the quarter-turn symmetries, then Taylor series (x^2 <= 0.62,
-// 14 terms, far below double rounding).
-constexpr double kPiD = 3.14159265358979323846264338327950288;
-constexpr double taylor_cos(double x) {
-  double term = 1.0, sum = 1.0;
-  for (int i = 1; i < 15; ++i) {
-    term *= -x * x / double((2 * i - 1) * (2 * i));
-    sum += term;
-  }
-  return sum;
-}
-constexpr double taylor_sin(double x) {
-  double term = x, sum = x;
-  for (int i = 1; i < 15; ++i) {
-    term *= -x * x / double((2 * i) * (2 * i + 1));
-    sum += term;
-  }
-  return sum;
-}
-constexpr double const_cos(double x) {
-  if (x > kPiD / 2) return -const_cos(kPiD - x);
-  if (x > kPiD / 4) return taylor_sin(kPiD / 2 - x);
-  return taylor_cos(x);
-}
-constexpr double const_sin(double x) {
-  if (x > kPiD / 2) return const_sin(kPiD - x);
-  if (x > kPiD / 4) return taylor_cos(kPiD / 2 - x);
-  return taylor_sin(x);
-}
-
-// a * exp(-+2 pi i K / N) with the root a compile-time constant (0 <= K < N/2);
-// K = 0 and K = N/4 take no multiplies.
-template <int N, int K, bool INV, typename T, typename C>
-__device__ __forceinline__ C twiddle_const(C a) {
-  if constexpr (K == 0) {
-    return a;
-  } else if constexpr (4 * K == N) {
-    return rot90<INV>(a);
-  } else {
-    constexpr double ang = 2.0 * kPiD * K / N;
-    constexpr double c = const_cos(ang), sn = const_sin(ang);
-    const C tw = {T(c), T(INV ? sn : -sn)};
-    return cmul(a, tw);
-  }
-}
-
-template <int K, int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  if constexpr (K < N) {
-    f(std::integral_constant<int, K>());
-    static_for<K + 1, N>(f);
-  }
-}
-
-// In-register DFT of size N = 2^a, 3 * 2^a or 5 * 2^a (even sizes split into
-// even and odd halves, combined with compile-time roots of unity).  w and
-// wstride are not read (the four-step callers pass the axis table).
-template <int N, bool INV, typename T, typename C>
-__device__ __forceinline__ void dft_reg(C* v, const C* w, int wstride) {
-  if constexpr (N == 1) {
-    return;
-  } else if constexpr (N == 2) {
-    dft2<INV, T>(v);
-  } else if constexpr (N == 3) {
-    dft3<INV, T>(v);
-  } else if constexpr (N == 4) {
-    dft4<INV, T>(v);
-  } else if constexpr (N == 5) {
-    dft5<INV, T>(v);
-  } else if constexpr (N == 8) {
-    dft8<INV, T>(v);
-  } else {
-    static_assert(N % 2 == 0, "in-register DFT sizes are 3, 5 or 2^a times them");
-    C e[N / 2], o[N / 2];
-#pragma unroll
-    for (int k = 0; k < N / 2; ++k) {
-      e[k] = v[2 * k];
-      o[k] = v[2 * k + 1];
-    }
-    dft_reg<N / 2, INV, T>(e, w, 2 * wstride);
-    dft_reg<N / 2, INV, T>(o, w, 2 * wstride);
-    static_for<0, N / 2>([&](auto kc) {
-      constexpr int k = decltype(kc)::value;
-      const C t = twiddle_const<N, k, INV, T>(o[k]);
-      v[k] = cadd(e[k], t);
-      v[k + N / 2] = csub(e[k], t);
-    });
-  }
-}
 
 template <int N1, int N2>
 struct FourStep {
@@ -733,7 +143,7 @@ __device__ __forceinline__ void four_step_1(C* L, int p, int t, const C* w, Load
   C v[N1];
 #pragma unroll
   for (int k1 = 0; k1 < N1; ++k1) v[k1] = load(k1);  // element t + N2 k1
-  dft_reg<N1, INV, T>(v, w, N2);
+  dft_reg<N1, INV, T>(v);
 #pragma unroll
   for (int j1 = 0; j1 < N1; ++j1) {
     if (j1 > 0 && t > 0) {
@@ -751,7 +161,7 @@ __device__ __forceinline__ void four_step_2(const C* L, int p, int t, const C* w
   C u[N2];
 #pragma unroll
   for (int k2 = 0; k2 < N2; ++k2) u[k2] = L[(t * N2 + k2) * TS + p];
-  dft_reg<N2, INV, T>(u, w, N1);
+  dft_reg<N2, INV, T>(u);
 #pragma unroll
   for (int j2 = 0; j2 < N2; ++j2) store(t + N1 * j2, u[j2]);
 }
@@ -816,7 +226,11 @@ fft_y4(SC* S, const SC* src, int W, int TJ, const typename CT<T>::type* __restri
 }
 
 // Launched with a multiple of 64 threads; threads past 3 TK lanes-per-column
-// only take part in the Green loop and the reduction.  kDot as in fft_z_green.
+// only take part in the Green loop and the reduction.  kDot: r . z by Parseval, sum over the half
+// spectrum of w(kx) Re(conj(r^) z^) with w = 1 at kx = 0 and kx = nyq (nx even), 2
+// elsewhere; z^ = G r^ already carries the 1/N of the inverse transform, so the sum
+// equals the real-space r . z.  One FP64 partial per workgroup at
+// partial[(rhs * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x].
 template <typename T, int N1, int N2, bool kDot, typename SC>
 __global__ void __launch_bounds__(kThreads4)
 fft_z4_green(SC* __restrict__ S, int ny, int nxh, int TK, Tables<T> tb, T lam, T mu, T inv_vn,
@@ -867,7 +281,7 @@ fft_z4_green(SC* __restrict__ S, int ny, int nxh, int TK, Tables<T> tb, T lam, T
   if (t < N1) {
 #pragma unroll
     for (int k2 = 0; k2 < N2; ++k2) u[k2] = L[(t * N2 + k2) * TJ + p];
-    dft_reg<N2, false, T>(u, w, N1);
+    dft_reg<N2, false, T>(u);
   }
   __syncthreads();
   if (t < N1) {
@@ -912,20 +326,10 @@ fft_z4_green(SC* __restrict__ S, int ny, int nxh, int TK, Tables<T> tb, T lam, T
 // workgroup is worked by `lanes` consecutive threads (t fastest), every global
 // access is a run of consecutive floats, and no integer division by runtime
 // values remains.  Pencils 3 pp + {0, 1, 2} of row pair pp are c0 + i c1 of
-// row 2pp, of row 2pp + 1, and c2(2pp) + i c2(2pp + 1), as in fft_x_r2c.
+// row 2pp, of row 2pp + 1, and c2(2pp) + i c2(2pp + 1).
 // LDS: the N1 x N2 step-1 tile of pencil p at p * TS + j1 * (N2 + 1) + t
 // (row padding: step-2 reads run down a column), and the natural-order
 // spectrum at p * (n + 1) + e.
-template <typename T>
-struct XUpdate {
-  T* r;
-  T* x;
-  const T* p;
-  const T* q;
-  const double* alpha;
-  double* partial;
-};
-
 template <int N1, int N2>
 struct XTile {
   static constexpr int n = N1 * N2;
@@ -1014,7 +418,7 @@ fft_x4_r2c(const T* __restrict__ r, SC* __restrict__ S, int64_t rows, int PP,
         v[k1] = C{re_ok ? f[re_off + e] : T(0), im_ok ? f[im_off + e] : T(0)};
       }
     }
-    dft_reg<N1, false, T>(v, w, N2);
+    dft_reg<N1, false, T>(v);
 #pragma unroll
     for (int j1 = 0; j1 < N1; ++j1) {
       if (j1 > 0 && t > 0) v[j1] = cmul(v[j1], w[(j1 * t) % n]);
@@ -1026,7 +430,7 @@ fft_x4_r2c(const T* __restrict__ r, SC* __restrict__ S, int64_t rows, int PP,
   if (live && t < N1) {
 #pragma unroll
     for (int k2 = 0; k2 < N2; ++k2) u[k2] = T1[t * (N2 + 1) + k2];
-    dft_reg<N2, false, T>(u, w, N1);
+    dft_reg<N2, false, T>(u);
   }
   __syncthreads();
   if (live && t < N1) {
@@ -1034,7 +438,7 @@ fft_x4_r2c(const T* __restrict__ r, SC* __restrict__ S, int64_t rows, int PP,
     for (int j2 = 0; j2 < N2; ++j2) T1[t + N1 * j2] = u[j2];  // natural order X[e]
   }
   __syncthreads();
-  // Two-for-one split, as in fft_x_r2c.
+  // Two-for-one split.
   double spec_rr = 0.0;  // kSpec: sum of w(k) |R^(k)|^2 over this thread's entries
   const T spec_alpha = kSpec ? T(upd.alpha[blockIdx.y]) : T(0);
   for (int idx = threadIdx.x; idx < PP * nxh; idx += blockDim.x) {
@@ -1090,7 +494,7 @@ fft_x4_r2c(const T* __restrict__ r, SC* __restrict__ S, int64_t rows, int PP,
   }
 }
 
-// kDir as in fft_x_c2r: the output is p = z + beta[rhs] p_old, p_old from pin
+// kDir: the output is the CG search direction p = z + beta[rhs] p_old, p_old from pin
 // (pin == z: in place).
 template <typename T, int N1, int N2, bool kDir, typename SC>
 __global__ void __launch_bounds__(256)
@@ -1168,7 +572,7 @@ fft_x4_c2r(const SC* __restrict__ S, T* z, int64_t rows, int PP,
   }
   __syncthreads();
   if (live && t < N2) {
-    dft_reg<N1, true, T>(v, w, N2);
+    dft_reg<N1, true, T>(v);
 #pragma unroll
     for (int j1 = 0; j1 < N1; ++j1) {
       if (j1 > 0 && t > 0) v[j1] = cmul(v[j1], cconj(w[(j1 * t) % n]));
@@ -1180,7 +584,7 @@ fft_x4_c2r(const SC* __restrict__ S, T* z, int64_t rows, int PP,
   C u[N2];
 #pragma unroll
   for (int k2 = 0; k2 < N2; ++k2) u[k2] = X[t * (N2 + 1) + k2];
-  dft_reg<N2, true, T>(u, w, N1);
+  dft_reg<N2, true, T>(u);
   T* f = z + int64_t(blockIdx.y) * field_stride;
 #pragma unroll
   for (int j2 = 0; j2 < N2; ++j2) {
@@ -1194,17 +598,16 @@ struct PrecondImpl {
   double hg0;  // C3D8R-HG cell: hourglass penalty of the reference medium per unit volume (0: FI)
   int nx, ny, nz, nxh;
   int64_t rows;
-  Axes axes;
+  AxisPlan plan[3];  // x, y, z (general passes)
+  GenShape shape[3];
   void* tw[3];
   void* tab[3];
   void* spec;
   int64_t spec_stride;  // complex entries per RHS
   void* rhat;           // x spectrum of the CG residual (spectral-residual form), allocated on demand
-  int pairs_per_block, tj, tk;
-  size_t lds_x, lds_y, lds_z;
-  // four-step kernels for y / z axes with a factorisation (0: use the Stockham pass)
+  // four-step kernels for y / z axes with a factorisation (0: the general passes)
   int bf16;          // spectrum stored as BF16 pairs (FP32 arithmetic, four-step passes only)
-  int x4;            // nx handled by fft_x4_r2c / fft_x4_c2r (0: Stockham x passes)
+  int x4;            // nx handled by fft_x4_r2c / fft_x4_c2r (0: the general passes)
   int pp4, thr_x4;   // row pairs and threads per x4 workgroup
   size_t lds_x4;
   int y4, z4;        // axis length handled by fft_y4 / fft_z4_green
@@ -1427,6 +830,7 @@ Tables<T> tables_of(const PrecondImpl* im) {
 }
 
 constexpr size_t kMaxLds = 65536;
+constexpr size_t kMaxLdsGen = 163840 - 1024;  // general passes, longest axes: one workgroup per CU
 
 // Positive integer from the environment (tile-size overrides for sweeps), else 0.
 int env_int(const char* name) {
@@ -1445,22 +849,8 @@ int create_impl(vxl_precond* pc, PrecondImpl* im) {
   im->nz = cell->grid.nz;
   im->nxh = im->nx / 2 + 1;
   im->rows = int64_t(im->ny) * im->nz;
-  im->axes.px = make_plan(im->nx);
-  im->axes.py = make_plan(im->ny);
-  im->axes.pz = make_plan(im->nz);
-  // ~2048 complex entries per ping-pong buffer (<= 32 KB FP32): several
-  // workgroups per CU so one group's loads overlap another's LDS transforms
-  // (two row pairs per x workgroup at nx = 256, the measured optimum).
-  const int target = 2048;
-  im->pairs_per_block = std::max(1, target / (3 * im->nx));
-  if (const int v = env_int("VXL_FFT_XPAIRS")) im->pairs_per_block = v;
-  im->tj = std::max(1, std::min(3 * im->nxh, target / im->ny));
-  im->tk = std::max(1, std::min(im->nxh, target / (3 * im->nz)));
-  im->lds_x = 2 * sizeof(C) * size_t(3 * im->pairs_per_block) * im->nx;
-  im->lds_y = 2 * sizeof(C) * size_t(im->tj) * im->ny;
-  im->lds_z = 2 * sizeof(C) * size_t(3 * im->tk) * im->nz;
-  if (im->lds_x > kMaxLds || im->lds_y > kMaxLds || im->lds_z > kMaxLds)
-    return fail("grid axis too long for the LDS pencil FFT");
+  const int axis[3] = {im->nx, im->ny, im->nz};
+  for (int a = 0; a < 3; ++a) im->plan[a] = make_axis_plan<T>(axis[a]);
   {
     const int ly = four_step_lanes(im->ny), lz = four_step_lanes(im->nz);
     const char* env = std::getenv("VXL_FFT_FOURSTEP");
@@ -1498,6 +888,17 @@ int create_impl(vxl_precond* pc, PrecondImpl* im) {
       im->lds_x4 = sizeof(C) * x4_stride<T>(im->nx) * 3 * im->pp4;
       if (im->thr_x4 > 256 || im->thr_x4 % 64 != 0 || im->lds_x4 > kMaxLds) im->x4 = 0;
     }
+  }
+  const int fourstep[3] = {im->x4, im->y4, im->z4};
+  for (int a = 0; a < 3; ++a) {
+    AxisPlan& p = im->plan[a];
+    if (fourstep[a]) {
+      p.dense = 0;
+      continue;
+    }
+    im->shape[a] = a == 0 ? gen_shape_x<T>(p, env_int("VXL_FFT_XPAIRS")) : a == 1 ? gen_shape_y<T>(p) : gen_shape_z<T>(p);
+    if (im->shape[a].lds > kMaxLdsGen) return fail("grid axis too long for the LDS pencil FFT");
+    VXL_TRY(upload_dense_table<T>(p));
   }
   im->spec_stride = int64_t(im->nz) * im->ny * im->nxh * 3;
   VXL_TRY(upload_tables<T>(im, cell->h));
@@ -1546,39 +947,39 @@ int apply_stages(vxl_precond* pc, PrecondImpl* im, int nrhs, const T* r, T* z, h
   SC* S = static_cast<SC*>(im->spec);
   const int64_t fstride = 3 * int64_t(im->nx) * im->rows;
   const int64_t pairs = (im->rows + 1) / 2;
-  const unsigned bx = unsigned((pairs + im->pairs_per_block - 1) / im->pairs_per_block);
   const int W = 3 * im->nxh;
   const unsigned bx4 = im->x4 ? unsigned((pairs + im->pp4 - 1) / im->pp4) : 0u;
   if (sr) {
     if constexpr (!kFull) {
       return fail("the spectral residual needs full-precision spectrum storage");
     } else {
-      if (!im->x4 || !im->y4 || !im->rhat) return fail("the spectral residual needs the four-step x and y passes");
+      if (!im->rhat) return fail("the spectral residual has no buffer");
     }
   }
   SC* const Rh = static_cast<SC*>(im->rhat);
+  const GenX<T> gx{im->plan[0], im->shape[0], tb.wx, im->rows, fstride, im->spec_stride, active};
   if (stages & kForwardX) {
-    if (upd && !im->x4) return fail("fused CG update needs the four-step x pass");
-    bool done = false;
-    if constexpr (kFull) {
-      if (sr && upd)
-        launch_x4_r2c<T, false, SC, true>(im->x4, dim3(bx4, nrhs), im->thr_x4, im->lds_x4, s, upd->q, Rh, im->rows,
-                                          im->pp4, tb.wx, fstride, im->spec_stride, active, *upd);
-      else if (sr)
-        launch_x4_r2c<T, false, SC>(im->x4, dim3(bx4, nrhs), im->thr_x4, im->lds_x4, s, r, Rh, im->rows, im->pp4,
-                                    tb.wx, fstride, im->spec_stride, active, XUpdate<T>{});
-      done = sr;
-    }
-    if (done) {
-    } else if (upd)
+    if (!im->x4) {
+      if constexpr (!kFull)
+        return fail("BF16 spectrum storage needs power-of-two axes");
+      else
+        VXL_TRY(launch_gen_r2c<T>(gx, nrhs, r, sr ? Rh : S, upd, sr, s));
+    } else if (sr) {
+      if constexpr (kFull) {
+        if (upd)
+          launch_x4_r2c<T, false, SC, true>(im->x4, dim3(bx4, nrhs), im->thr_x4, im->lds_x4, s, upd->q, Rh, im->rows,
+                                            im->pp4, tb.wx, fstride, im->spec_stride, active, *upd);
+        else
+          launch_x4_r2c<T, false, SC>(im->x4, dim3(bx4, nrhs), im->thr_x4, im->lds_x4, s, r, Rh, im->rows, im->pp4,
+                                      tb.wx, fstride, im->spec_stride, active, XUpdate<T>{});
+      }
+    } else if (upd) {
       launch_x4_r2c<T, true, SC>(im->x4, dim3(bx4, nrhs), im->thr_x4, im->lds_x4, s, r, S, im->rows, im->pp4, tb.wx,
                              fstride, im->spec_stride, active, *upd);
-    else if (im->x4)
+    } else {
       launch_x4_r2c<T, false, SC>(im->x4, dim3(bx4, nrhs), im->thr_x4, im->lds_x4, s, r, S, im->rows, im->pp4, tb.wx,
                               fstride, im->spec_stride, active, XUpdate<T>{});
-    else if constexpr (kFull)
-      hipLaunchKernelGGL((fft_x_r2c<T>), dim3(bx, nrhs), dim3(kThreads), im->lds_x, s, r, S, im->nx, im->rows,
-                         im->nxh, im->pairs_per_block, im->axes, tb, fstride, im->spec_stride, active);
+    }
     VXL_HIP(hipGetLastError());
   }
   if (!(stages & kRest)) return VXL_OK;
@@ -1593,12 +994,9 @@ int apply_stages(vxl_precond* pc, PrecondImpl* im, int nrhs, const T* r, T* z, h
                                 im->spec_stride, active);
     } else if constexpr (!kFull) {
       return fail("BF16 spectrum storage needs power-of-two axes");
-    } else if (inverse) {
-      hipLaunchKernelGGL((fft_y<true, T>), dim3((W + im->tj - 1) / im->tj, im->nz, nrhs), dim3(kThreads),
-                         im->lds_y, s, S, im->ny, im->nz, W, im->tj, im->axes, tb, im->spec_stride, active);
     } else {
-      hipLaunchKernelGGL((fft_y<false, T>), dim3((W + im->tj - 1) / im->tj, im->nz, nrhs), dim3(kThreads),
-                         im->lds_y, s, S, im->ny, im->nz, W, im->tj, im->axes, tb, im->spec_stride, active);
+      VXL_TRY(launch_gen_y<T>(im->plan[1], im->shape[1], tb.wy, inverse, nrhs, S, inverse || !sr ? S : Rh, im->nz, W,
+                              im->spec_stride, active, s));
     }
     VXL_HIP(hipGetLastError());
     return VXL_OK;
@@ -1620,13 +1018,8 @@ int apply_stages(vxl_precond* pc, PrecondImpl* im, int nrhs, const T* r, T* z, h
       launch_z4<T, false, SC>(im->z4, g, im->thr_z4, im->lds_z4, s, S, im->ny, im->nxh, im->tk4, tb, lam, mu, inv_vn,
                           im->spec_stride, active, nyq, part, media, grhs);
   } else if constexpr (kFull) {
-    const dim3 g((im->nxh + im->tk - 1) / im->tk, im->ny, nrhs);
-    if (cg)
-      hipLaunchKernelGGL((fft_z_green<T, true>), g, dim3(kThreads), im->lds_z, s, S, im->ny, im->nz, im->nxh,
-                         im->tk, im->axes, tb, lam, mu, inv_vn, im->spec_stride, active, nyq, part, media, grhs);
-    else
-      hipLaunchKernelGGL((fft_z_green<T, false>), g, dim3(kThreads), im->lds_z, s, S, im->ny, im->nz, im->nxh,
-                         im->tk, im->axes, tb, lam, mu, inv_vn, im->spec_stride, active, nyq, part, media, grhs);
+    VXL_TRY(launch_gen_z<T>(im->plan[2], im->shape[2], tb, nrhs, S, im->ny, im->nxh, lam, mu, inv_vn, im->spec_stride,
+                            active, nyq, part, media, grhs, s));
   }
   VXL_HIP(hipGetLastError());
   if (cg) VXL_TRY(cg->mid());
@@ -1639,14 +1032,8 @@ int apply_stages(vxl_precond* pc, PrecondImpl* im, int nrhs, const T* r, T* z, h
                             fstride, im->spec_stride, active, nullptr, static_cast<const T*>(nullptr));
   else if constexpr (!kFull)
     return fail("BF16 spectrum storage needs power-of-two axes");
-  else if (cg)
-    hipLaunchKernelGGL((fft_x_c2r<T, true>), dim3(bx, nrhs), dim3(kThreads), im->lds_x, s, S, z, im->nx,
-                       im->rows, im->nxh, im->pairs_per_block, im->axes, tb, fstride, im->spec_stride, active,
-                       cg->beta, static_cast<const T*>(cg->pin));
   else
-    hipLaunchKernelGGL((fft_x_c2r<T, false>), dim3(bx, nrhs), dim3(kThreads), im->lds_x, s, S, z, im->nx,
-                       im->rows, im->nxh, im->pairs_per_block, im->axes, tb, fstride, im->spec_stride, active,
-                       nullptr, static_cast<const T*>(nullptr));
+    VXL_TRY(launch_gen_c2r<T>(gx, nrhs, S, z, cg ? cg->beta : nullptr, cg ? static_cast<const T*>(cg->pin) : nullptr, s));
   VXL_HIP(hipGetLastError());
   return VXL_OK;
 }
@@ -1667,6 +1054,7 @@ int precond_create(vxl_precond* pc) {
   auto* im = new PrecondImpl();
   im->tw[0] = im->tw[1] = im->tw[2] = nullptr;
   im->tab[0] = im->tab[1] = im->tab[2] = nullptr;
+  for (auto& p : im->plan) p.coef = nullptr;
   im->spec = nullptr;
   im->rhat = nullptr;
   pc->impl = im;
@@ -1725,22 +1113,21 @@ template int precond_cg_rest<double>(vxl_precond*, int, double*, double*, const 
 bool precond_spectral_residual_ok(const vxl_precond* pc) {
   const auto* im = static_cast<const PrecondImpl*>(pc->impl);
   const char* env = std::getenv("VXL_SPECTRAL_RESIDUAL");
-  return pc->precision == VXL_F32 && im->x4 && im->y4 && !im->bf16 && !(env && env[0] == '0');
+  return pc->precision == VXL_F32 && !im->bf16 && !(env && env[0] == '0');
 }
 
 int precond_residual_spectrum(vxl_precond* pc) {
   auto* im = static_cast<PrecondImpl*>(pc->impl);
   if (im->rhat) return VXL_OK;
-  if (!precond_spectral_residual_ok(pc)) return fail("the spectral residual needs the FP32 four-step x and y passes");
+  if (!precond_spectral_residual_ok(pc)) return fail("the spectral residual needs FP32 spectrum storage");
   VXL_HIP(dev_malloc(&im->rhat, sizeof(float2) * size_t(im->spec_stride) * pc->nrhs_max));
   return VXL_OK;
 }
 
 int precond_fused_update_blocks(const vxl_precond* pc) {
   const auto* im = static_cast<const PrecondImpl*>(pc->impl);
-  if (!im->x4) return 0;
-  const int64_t pairs = (im->rows + 1) / 2;
-  return int((pairs + im->pp4 - 1) / im->pp4);
+  const int64_t pairs = (im->rows + 1) / 2, per = im->x4 ? im->pp4 : im->shape[0].units;
+  return int((pairs + per - 1) / per);
 }
 
 bool fused_update_enabled() {
@@ -1763,8 +1150,9 @@ int precond_apply_masked(vxl_precond* pc, int nrhs, const void* r, void* z, cons
 
 int precond_rz_blocks(const vxl_precond* pc) {
   const auto* im = static_cast<const PrecondImpl*>(pc->impl);
-  const int gx = im->z4 ? (im->nxh + im->tk4 - 1) / im->tk4 : (im->nxh + im->tk - 1) / im->tk;
-  return gx * im->ny;
+  if (im->z4) return (im->nxh + im->tk4 - 1) / im->tk4 * im->ny;
+  const int64_t cols = int64_t(im->ny) * 3 * im->nxh;
+  return int((cols + im->shape[2].units - 1) / im->shape[2].units);
 }
 
 void precond_release(vxl_precond* pc) {
@@ -1774,6 +1162,7 @@ void precond_release(vxl_precond* pc) {
   for (int a = 0; a < 3; ++a) {
     if (im->tw[a]) dev_free(im->tw[a]);
     if (im->tab[a]) dev_free(im->tab[a]);
+    if (im->plan[a].coef) dev_free(im->plan[a].coef);
   }
   if (im->spec) dev_free(im->spec);
   if (im->rhat) dev_free(im->rhat);

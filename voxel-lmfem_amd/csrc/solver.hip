@@ -120,6 +120,7 @@ int free_all(vxl_solver* s) {
     if (s->pring[i]) dev_free(s->pring[i]);
   s->nslot = 0;
   if (s->hist) dev_free(s->hist);
+  if (s->rscale) dev_free(s->rscale);
   if (s->gram) dev_free(s->gram);
   if (s->partial_cert) dev_free(s->partial_cert);
   if (s->blk_partial) dev_free(s->blk_partial);
@@ -443,6 +444,8 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
 
   std::vector<int> active(R, 1), restart(R, 0), its(R, 0), nrest(R, 0);
   std::vector<double> ff(R), rr(R), rr_ref(R), res_true(R, 0.0);
+  std::vector<double> rs2(R, 1.0);  // square of the FP32 residual's scale
+  const double* rscale = nullptr;   // device scales and their inverses, when any is not 1
   for (auto& t : s->trace) t.clear();
   // Host<->device flag and scalar traffic goes through pinned staging; every
   // upload waits for the previous one so the staging area is never rewritten
@@ -498,6 +501,35 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
     }
     rr_ref[k] = ff[k];
   }
+  if (mixed) {
+    // A load whose exact fluctuation is zero has rounding noise for a
+    // right-hand side; its FP32 products p . q would fall below the normal
+    // range before the certificate is reached and the recurrence would stall.
+    // Right-hand sides far from 1 are therefore scaled by a power of two
+    // (exact), and their steps scaled back when they are added to x64.
+    std::vector<double> sc(2 * size_t(R), 1.0);
+    bool any = false;
+    for (int k = 0; k < R; ++k) {
+      if (!active[k] || !std::isfinite(ff[k])) continue;
+      const int e = std::ilogb(std::sqrt(ff[k] / double(len)));
+      if (e >= -20 && e <= 20) continue;
+      const int se = std::max(-400, std::min(400, -e));
+      sc[k] = std::ldexp(1.0, se);
+      sc[R + k] = std::ldexp(1.0, -se);
+      rs2[k] = sc[k] * sc[k];
+      rr_ref[k] = ff[k] * rs2[k];
+      any = true;
+    }
+    if (any) {
+      if (!s->rscale) VXL_HIP(dev_malloc(&s->rscale, sizeof(double) * sc.size()));
+      VXL_HIP(hipMemcpyAsync(s->rscale, sc.data(), sizeof(double) * sc.size(), hipMemcpyHostToDevice, st));
+      VXL_HIP(hipMemcpyAsync(scal + kFF * R, rr_ref.data(), sizeof(double) * R, hipMemcpyHostToDevice, st));
+      VXL_HIP(hipStreamSynchronize(st));  // sc is host memory of this block
+      rscale = s->rscale;
+      VXL_TRY(launch_scaled_residual(s->f, reinterpret_cast<float*>(r), rscale, len, R, st));
+    }
+  }
+  const double* unscale = rscale ? rscale + R : nullptr;
   VXL_TRY(upload_flags());
   // p = z = M r with rho = r.z: beta = 0 because rho_old = 0 (slots cleared).
   Steps<T> steps(s, tol, st);
@@ -531,7 +563,7 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
     DirectionSet<T> d{};
     for (size_t t = 0; t < pend.size(); ++t) d.p[t] = slots[pend[t]];
     d.count = int(pend.size());
-    VXL_TRY(launch_flush<T>(s->x64, d, s->hist, R, len, !x64_set, st));
+    VXL_TRY(launch_flush<T>(s->x64, d, s->hist, unscale, R, len, !x64_set, st));
     x64_set = true;
     pend.clear();
     return VXL_OK;
@@ -554,12 +586,12 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
     if (ring)
       VXL_TRY(flush());
     else if (mixed)
-      VXL_TRY(launch_accumulate(s->x64, reinterpret_cast<float*>(x), len, R, act, st));
+      VXL_TRY(launch_accumulate(s->x64, reinterpret_cast<float*>(x), unscale, len, R, act, st));
     // K annihilates the mean, so the zero-mean projection of x64 is left to
     // the end of the run; mixed mode needs the residual only in FP32.
     int rblocks = 0;
     VXL_TRY(launch_residual_apply(cell, R, s->x64, s->f, mixed ? reinterpret_cast<float*>(r) : nullptr,
-                                  mixed ? nullptr : s->r64, act, s->partial_cert, &rblocks, st));
+                                  mixed ? nullptr : s->r64, act, s->partial_cert, &rblocks, rscale, st));
     VXL_TRY(launch_finalize(s->partial_cert, rblocks, kOpStore, scal, R, act, nullptr, st));
     std::vector<double> t(R);
     VXL_TRY(read_slot(kTmp, t));
@@ -569,7 +601,7 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
       if (!std::isfinite(rel)) return fail("Nonfinite true residual");
       nrest[k] += 1;
       s->trace[k].push_back({-it, rel});  // negative iteration: FP64 true residual
-      rr_ref[k] = t[k];
+      rr_ref[k] = t[k] * rs2[k];
       if (rel <= tol) {
         active[k] = 0;
         res_true[k] = rel;
@@ -648,7 +680,7 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
         if (!active[k]) continue;
         if (!std::isfinite(rr[k])) return fail("Nonfinite residual in CG recursion");
         const int at = pin_stop[k] ? (base >= 0 ? base + pin_stop[k] : pin_stop[k]) : it;
-        s->trace[k].push_back({at, std::sqrt(rr[k] / ff[k])});
+        s->trace[k].push_back({at, std::sqrt(rr[k] / (ff[k] * rs2[k]))});
         its[k] = at;
         latched[k] = pin_stop[k] != 0;
         const bool drop = mixed && rr[k] < kReliable * kReliable * rr_ref[k];
@@ -843,10 +875,10 @@ int run_block_impl(vxl_solver* s, const double* macro_host, double tol, int max_
   int it = 0;
   auto certify = [&]() -> int {
     std::vector<int> mask = active;
-    if (mixed) VXL_TRY(launch_accumulate(s->x64, reinterpret_cast<float*>(s->x), len, R, act, st));
+    if (mixed) VXL_TRY(launch_accumulate(s->x64, reinterpret_cast<float*>(s->x), nullptr, len, R, act, st));
     int rblocks = 0;
     VXL_TRY(launch_residual_apply(cell, R, s->x64, s->f, mixed ? reinterpret_cast<float*>(s->r) : nullptr,
-                                  mixed ? nullptr : s->r64, act, s->partial_cert, &rblocks, st));
+                                  mixed ? nullptr : s->r64, act, s->partial_cert, &rblocks, nullptr, st));
     VXL_TRY(launch_finalize(s->partial_cert, rblocks, kOpStore, scal, R, act, nullptr, st));
     std::vector<double> t;
     VXL_TRY(read_doubles(scal + kTmp * R, R, t));

@@ -263,6 +263,7 @@ struct ApplyArgs {
   const double* f;
   float* r32;
   double* r64;
+  const double* rscale;  // optional power of two per right-hand side applied to r32
   // kFuse: systems with active[r] == 0 are skipped and u . (K u) of each
   // workgroup is written to partial[(r * chunks + chunk) * tiles + tile].
   const int* active;
@@ -718,6 +719,7 @@ apply_kernel_v2(ApplyArgs<T> a) {
   // u_node . (K u)_node; u at the node of plane z is read from LDS while that
   // plane is resident (one layer earlier) and kept in registers.
   double rr = 0.0;  // kResid: sum of r^2 over the nodes this thread writes
+  const double rscale = kResid && a.rscale ? a.rscale[bid.rhs] : 1.0;
   T pq = T(0);  // at most zchunk nodes per thread; FP64 from the block sum on
   auto node_value = [&](T (&v)[3], int buf) {
 #pragma unroll
@@ -856,7 +858,7 @@ apply_kernel_v2(ApplyArgs<T> a) {
         for (int cc = 0; cc < 3; ++cc) {
           const double v = fpre[cc] - double(acc[cc]);
           if (a.r32)
-            a.r32[base + cc * n + node] = float(v);
+            a.r32[base + cc * n + node] = float(v * rscale);
           else
             a.r64[base + cc * n + node] = v;
           rr = fma(v, v, rr);
@@ -1296,7 +1298,7 @@ int default_stencil_variant(int precision) {
 // r64, ||r||^2 partials per workgroup; systems with active == 0 are skipped.
 template <typename Idx, bool kScale>
 int launch_resid_impl(const vxl_cell* cell, int nrhs, const double* u, const double* f, float* r32, double* r64,
-                      const int* active, double* partial, int* blocks, hipStream_t s) {
+                      const int* active, double* partial, int* blocks, const double* rscale, hipStream_t s) {
   constexpr int TY = kTilesF64[0];
   using TL = Tile<32, TY>;
   ApplyArgs<double> a{};
@@ -1306,6 +1308,7 @@ int launch_resid_impl(const vxl_cell* cell, int nrhs, const double* u, const dou
   a.f = f;
   a.r32 = r32;
   a.r64 = r64;
+  a.rscale = rscale;
   a.active = active;
   a.partial = partial;
   a.rhs_stride = 3 * cell->grid.n;
@@ -1343,18 +1346,18 @@ int launch_resid_impl(const vxl_cell* cell, int nrhs, const double* u, const dou
 }
 
 int launch_residual_apply(const vxl_cell* cell, int nrhs, const double* u, const double* f, float* r32, double* r64,
-                          const int* active, double* partial, int* blocks, hipStream_t s) {
+                          const int* active, double* partial, int* blocks, const double* rscale, hipStream_t s) {
   const bool sc = cell->mat.scale != nullptr;
   switch (cell->mat.index_kind) {
     case VXL_INDEX_U8:
-      return sc ? launch_resid_impl<uint8_t, true>(cell, nrhs, u, f, r32, r64, active, partial, blocks, s)
-                : launch_resid_impl<uint8_t, false>(cell, nrhs, u, f, r32, r64, active, partial, blocks, s);
+      return sc ? launch_resid_impl<uint8_t, true>(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale, s)
+                : launch_resid_impl<uint8_t, false>(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale, s);
     case VXL_INDEX_U16:
-      return sc ? launch_resid_impl<uint16_t, true>(cell, nrhs, u, f, r32, r64, active, partial, blocks, s)
-                : launch_resid_impl<uint16_t, false>(cell, nrhs, u, f, r32, r64, active, partial, blocks, s);
+      return sc ? launch_resid_impl<uint16_t, true>(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale, s)
+                : launch_resid_impl<uint16_t, false>(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale, s);
     case VXL_INDEX_I32:
-      return sc ? launch_resid_impl<int32_t, true>(cell, nrhs, u, f, r32, r64, active, partial, blocks, s)
-                : launch_resid_impl<int32_t, false>(cell, nrhs, u, f, r32, r64, active, partial, blocks, s);
+      return sc ? launch_resid_impl<int32_t, true>(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale, s)
+                : launch_resid_impl<int32_t, false>(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale, s);
   }
   return fail("unknown material index kind");
 }

@@ -50,15 +50,20 @@ int launch_row_totals(const double* partial, int rows, int nblk, double scale, d
 int launch_stiffness_sums(const vxl_cell* cell, double* partial, int blocks, hipStream_t s);
 // x64 += sum_t alpha[t * nrhs + k] p_t for every system k (assign: x64 =
 // the sum, its old contents ignored); terms with alpha = 0 are skipped.
+// unscale (optional, one per system): the steps are unscale[k] alpha_t p_t.
 template <typename T>
-int launch_flush(double* x64, const DirectionSet<T>& d, const double* alpha, int nrhs, int64_t len, bool assign,
-                 hipStream_t s);
+int launch_flush(double* x64, const DirectionSet<T>& d, const double* alpha, const double* unscale, int nrhs,
+                 int64_t len, bool assign, hipStream_t s);
 template <typename T>
 int launch_update_xr(T* x, T* r, const T* p, const T* q, int64_t len, int nrhs, const double* alpha,
                      double* partial, const int* active, hipStream_t s);
 int launch_residual(double* r, const double* f, const double* q, float* r32, int64_t len, int nrhs,
                     double* partial, const int* active, hipStream_t s);
-int launch_accumulate(double* x64, float* x32, int64_t len, int nrhs, const int* active, hipStream_t s);
+// x64 += unscale[k] x32 (unscale may be null: 1), x32 = 0.
+int launch_accumulate(double* x64, float* x32, const double* unscale, int64_t len, int nrhs, const int* active,
+                      hipStream_t s);
+// r32 = float(scale[k] f).
+int launch_scaled_residual(const double* f, float* r32, const double* scale, int64_t len, int nrhs, hipStream_t s);
 template <typename A, typename B>
 int launch_convert(B* dst, const A* src, int64_t len, int nrhs, const int* active, hipStream_t s);
 template <typename T>
@@ -218,6 +223,9 @@ struct vxl_solver {
   int nslot;
   void* pring[vxl::kMaxDirections];
   double* hist;  // alpha_t per slot use and system, kMaxDirections x R
+  // Mixed mode: power of two each FP32 residual is scaled by and its inverse
+  // (device, 2 R; see run_impl).
+  double* rscale;
   double* gram;  // mean-stress partials and totals of the six-unit-strain path
   // Block CG (method VXL_METHOD_BLOCK_CG): Gram partials, the small R x R
   // matrices [G | alpha | beta] and ||r||^2 totals, direction flags.
