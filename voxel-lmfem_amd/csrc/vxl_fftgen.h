@@ -7,10 +7,13 @@
 //           (the very entries it read, so it also runs in place in LDS);
 //   step 2, row t < n1: entries t n2 + k2 -> DFT_n2 -> X[t + n1 j2].
 // Lanes run along columns and the `rows` of a workgroup take the rows of each
-// step in turn.  With 64 columns (kWave) every index, twiddle and dense
+// step in turn.  With 64 columns (SUB = 1) every index, twiddle and dense
 // coefficient is uniform over a wave: address arithmetic runs on the scalar
 // unit and coefficients arrive by scalar loads, so the vector unit executes
-// little beside the transform itself.  DFT_n1 and DFT_n2 are in-register
+// little beside the transform itself.  With 32 columns (SUB = 2) the two halves
+// of a wave take neighbouring rows: dense coefficients stay uniform, and
+// twiddles are two scalar loads and a select.  Fewer columns (SUB = 0, the
+// longest axes only) index per lane.  DFT_n1 and DFT_n2 are in-register
 // transforms (2 to 16; FP32 also 18, 20, 25).  An n2 that is none of these (a prime
 // factor above 13, or a product too large) is a dense transform out of LDS:
 // the row is folded to a_j = x_j + x_{n2-j}, b_j = x_j - x_{n2-j}, and a thread
@@ -42,7 +45,7 @@ constexpr bool in_register(int n) {
 }
 template <typename T>
 constexpr int kDenseOut = sizeof(T) == 4 ? 8 : 4;  // dense output pairs per thread
-constexpr size_t kGenLds = 64512;  // dynamic LDS per workgroup, at most (two workgroups share a CU's 160 KB)
+constexpr size_t kGenLds = 81408;  // dynamic LDS of a workgroup when two share a CU's 160 KB
 
 // Read-only table in the constant address space: uniform indices become
 // scalar loads.
@@ -66,11 +69,41 @@ struct GenAxis {
   const void* coef;
 };
 
-// Row of a thread (uniform over a wave of 64 columns).
-template <bool kWave>
-__device__ __forceinline__ int row_index(int lp) {
-  const int g = int(threadIdx.x) >> lp;
-  return kWave ? __builtin_amdgcn_readfirstlane(g) : g;
+// The rows a thread takes: base + half, base + half + step, ...; base is
+// uniform over a wave (SUB = 1, 2).
+template <int SUB>
+struct RowSet {
+  int base, step, half;
+  __device__ __forceinline__ explicit RowSet(int lp) : step(int(blockDim.x) >> lp), half(0) {
+    if constexpr (SUB == 0) {
+      base = int(threadIdx.x) >> lp;
+    } else {
+      base = SUB * __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+      if constexpr (SUB == 2) half = (int(threadIdx.x) >> 5) & 1;
+    }
+  }
+  // f(base row, row) for every row below n.
+  template <typename F>
+  __device__ __forceinline__ void each(int n, F&& f) const {
+    for (int tb = base; tb < n; tb += step) {
+      if constexpr (SUB == 2) {
+        if (tb + half < n) f(tb, tb + half);
+      } else {
+        f(tb, tb);
+      }
+    }
+  }
+};
+// Entry j * t of the twiddle table for row t = tb + half.  (tb + 1 may be one
+// row past the last: j (tb + 1) stays below n.)
+template <int SUB, typename C, typename T>
+__device__ __forceinline__ C twiddle_at(CPtr<T> w, int j, int tb, int half) {
+  C a = cload<C, T>(w, j * tb);
+  if constexpr (SUB == 2) {
+    const C b = cload<C, T>(w, j * (tb + 1));
+    a = C{half ? b.x : a.x, half ? b.y : a.y};
+  }
+  return a;
 }
 
 template <typename T, typename F>
@@ -86,15 +119,15 @@ __device__ __forceinline__ void with_radix(int r, F&& f) {
   }
 }
 
-// Step 1 over the rows g, g + rows, ...: load(entry), twiddled outputs to L
+// Step 1 over this thread's rows: load(entry), twiddled outputs to L
 // (row stride ps, column p).
-template <bool INV, typename T, typename C, typename Load>
-__device__ __forceinline__ void gen_step1(C* L, int ps, int p, int g, int rows, const GenAxis<T>& ax, Load load) {
+template <bool INV, int SUB, typename T, typename C, typename Load>
+__device__ __forceinline__ void gen_step1(C* L, int ps, int p, const RowSet<SUB>& rs, const GenAxis<T>& ax, Load load) {
   const CPtr<T> w = cptr<T>(ax.w);
   const int n2 = ax.n2;
   with_radix<T>(ax.n1, [&](auto rc) {
     constexpr int R = decltype(rc)::value;
-    for (int t = g; t < n2; t += rows) {
+    rs.each(n2, [&](int tb, int t) {
       C v[R];
 #pragma unroll
       for (int k = 0; k < R; ++k) v[k] = load(t + n2 * k);
@@ -102,13 +135,13 @@ __device__ __forceinline__ void gen_step1(C* L, int ps, int p, int g, int rows, 
 #pragma unroll
       for (int j = 0; j < R; ++j) {
         if (j > 0) {
-          C tw = cload<C, T>(w, j * t);
+          C tw = twiddle_at<SUB, C, T>(w, j, tb, rs.half);
           if (INV) tw = cconj(tw);
           v[j] = cmul(v[j], tw);
         }
         L[(j * n2 + t) * ps + p] = v[j];
       }
-    }
+    });
   });
 }
 
@@ -150,37 +183,48 @@ __device__ __forceinline__ void dense_group(const C* x, int ps, int k0, const Ge
   }
 }
 
+// Dense groups (row, first output) of this thread: f(tb, row, k0).  The
+// halves of a wave (SUB = 2) take two rows of the same group, so that the
+// coefficients stay uniform.
+template <typename T, int SUB, typename F>
+__device__ __forceinline__ void each_group(const RowSet<SUB>& rs, const GenAxis<T>& ax, F&& f) {
+  constexpr int K = kDenseOut<T>, S = SUB == 2 ? 2 : 1;
+  const int groups = ax.hpad / K, sets = (ax.n1 + S - 1) / S;
+  for (int i = rs.base / S; i < sets * groups; i += rs.step / S) {
+    const int tb = i / groups * S, k0 = (i - i / groups * groups) * K;
+    if (S == 1 || tb + rs.half < ax.n1) f(tb, tb + rs.half, k0);
+  }
+}
+
 // Step 2 over rows: out(t, j2, X[t + n1 j2]); reads L, calls out for every
 // output of a row after all reads of that row (in-register form only).
-template <bool INV, typename T, typename C, typename Out>
-__device__ __forceinline__ void gen_step2(const C* L, int ps, int p, int g, int rows, const GenAxis<T>& ax, Out out) {
+template <bool INV, int SUB, typename T, typename C, typename Out>
+__device__ __forceinline__ void gen_step2(const C* L, int ps, int p, const RowSet<SUB>& rs, const GenAxis<T>& ax,
+                                          Out out) {
   const int n1 = ax.n1, n2 = ax.n2;
   if (ax.dense) {
-    constexpr int K = kDenseOut<T>;
-    const int groups = ax.hpad / K;
-    for (int i = g; i < n1 * groups; i += rows) {
-      const int t = i / groups, k0 = (i - t * groups) * K;
+    each_group<T>(rs, ax, [&](int, int t, int k0) {
       dense_group<INV, T>(L + t * n2 * ps + p, ps, k0, ax, [&](int k, C v) { out(t, k, v); });
-    }
+    });
     return;
   }
   with_radix<T>(n2, [&](auto rc) {
     constexpr int R = decltype(rc)::value;
-    for (int t = g; t < n1; t += rows) {
+    rs.each(n1, [&](int, int t) {
       C u[R];
 #pragma unroll
       for (int k = 0; k < R; ++k) u[k] = L[(t * R + k) * ps + p];
       dft_reg<R, INV, T>(u);
 #pragma unroll
       for (int j = 0; j < R; ++j) out(t, j, u[j]);
-    }
+    });
   });
 }
 
 // ---- y pass -----------------------------------------------------------------------
 // Columns are numbered over all z planes (z W + j), so only the last workgroup
 // of a right-hand side has idle columns.
-template <bool INV, typename T, bool kWave>
+template <bool INV, typename T, int SUB>
 __global__ void __launch_bounds__(kGenThreads<T>, kGenWaves<T>)
 gen_y(typename CT<T>::type* S, const typename CT<T>::type* src, GenAxis<T> ax, int cols, int W, int64_t spec_stride,
       const int* active) {
@@ -189,18 +233,18 @@ gen_y(typename CT<T>::type* S, const typename CT<T>::type* src, GenAxis<T> ax, i
   const uint3 b = xcd_block3();
   if (active && !active[b.y]) return;
   C* L = reinterpret_cast<C*>(smem_raw);
-  const int P = kWave ? 64 : 1 << ax.lp, p = int(threadIdx.x) & (P - 1);
-  const int g = row_index<kWave>(ax.lp), rows = int(blockDim.x) >> ax.lp;
+  const int P = SUB ? 64 / SUB : 1 << ax.lp, p = int(threadIdx.x) & (P - 1);
+  const RowSet<SUB> rs(ax.lp);
   const int col = int(b.x) * P + p;
   const bool live = col < cols;
   const int c = live ? col : cols - 1;
   const int z = c / W, j = c - z * W;
   const int64_t off = int64_t(b.y) * spec_stride + int64_t(z) * ax.n * W + j;
   const C* in = src + off;
-  gen_step1<INV, T>(L, P, p, g, rows, ax, [&](int e) -> C { return in[e * W]; });
+  gen_step1<INV, SUB, T>(L, P, p, rs, ax, [&](int e) -> C { return in[e * W]; });
   __syncthreads();
   C* o = S + off;
-  gen_step2<INV, T>(L, P, p, g, rows, ax, [&](int t, int k, C v) {
+  gen_step2<INV, SUB, T>(L, P, p, rs, ax, [&](int t, int k, C v) {
     if (live) o[(t + ax.n1 * k) * W] = v;
   });
 }
@@ -295,7 +339,7 @@ struct GreenLane {
 
 // partial (optional): FP64 r . z of the workgroup by Parseval, weight 1 at
 // kx = 0 and kx = nyq, 2 elsewhere, at partial[rhs * gridDim.x + block].
-template <typename T, bool kDot, bool kWave>
+template <typename T, bool kDot, int SUB>
 __global__ void __launch_bounds__(kGenThreads<T>, kGenWaves<T>)
 gen_z(typename CT<T>::type* S, GenAxis<T> ax, int units, int ny, int nxh, Tables<T> tb, T lam, T mu, T inv_vn,
       int64_t spec_stride, const int* active, int nyq, double* partial, const double* media, int group_rhs) {
@@ -308,8 +352,8 @@ gen_z(typename CT<T>::type* S, GenAxis<T> ax, int units, int ny, int nxh, Tables
     lam = T(media[2 * (bk.y / group_rhs)]);
     mu = T(media[2 * (bk.y / group_rhs) + 1]);
   }
-  const int P = kWave ? 64 : 1 << ax.lp, p = int(threadIdx.x) & (P - 1);
-  const int g = row_index<kWave>(ax.lp), rows = int(blockDim.x) >> ax.lp;
+  const int P = SUB ? 64 / SUB : 1 << ax.lp, p = int(threadIdx.x) & (P - 1);
+  const RowSet<SUB> rs(ax.lp);
   const int n1 = ax.n1, n2 = ax.n2, W = 3 * nxh, cols = ny * W;
   C* L = reinterpret_cast<C*>(smem_raw);
   C* L2 = L + ax.n * P;  // dense only
@@ -330,55 +374,59 @@ gen_z(typename CT<T>::type* S, GenAxis<T> ax, int units, int ny, int nxh, Tables
   const int64_t zs = int64_t(cols);
   const CPtr<T> gz = cptr<T>(tb.gz);
   const CPtr<T> w = cptr<T>(ax.w);
-  auto zfactors = [&](int kz) -> AxisF<T> {
+  auto zload = [&](int kz) -> AxisF<T> {
     const int n = ax.n;
     if (G.hg) return {gz[4 * n + kz], gz[5 * n + kz], gz[6 * n + kz], T(0)};
     return {gz[kz], gz[n + kz], gz[2 * n + kz], gz[3 * n + kz]};
   };
+  auto zfactors = [&](int tb, int k) -> AxisF<T> {  // of entry tb + half + n1 k
+    AxisF<T> f = zload(tb + n1 * k);
+    if constexpr (SUB == 2) {
+      const AxisF<T> h = zload(min(tb + 1 + n1 * k, ax.n - 1));
+      f = {rs.half ? h.a : f.a, rs.half ? h.b : f.b, rs.half ? h.c : f.c, rs.half ? h.d : f.d};
+    }
+    return f;
+  };
   double dot = 0.0;
 
-  gen_step1<false, T>(L, P, p, g, rows, ax, [&](int e) -> C { return base[e * zs]; });
+  gen_step1<false, SUB, T>(L, P, p, rs, ax, [&](int e) -> C { return base[e * zs]; });
   __syncthreads();
   if (ax.dense) {
-    constexpr int K = kDenseOut<T>;
-    const int groups = ax.hpad / K;
-    for (int i = g; i < n1 * groups; i += rows) {
-      const int t = i / groups, k0 = (i - t * groups) * K;
+    each_group<T>(rs, ax, [&](int tb, int t, int k0) {
       dense_group<false, T>(L + t * n2 * P + p, P, k0, ax, [&](int k, C v) {
-        dot += G.solve(v, zfactors(t + n1 * k));
+        dot += G.solve(v, zfactors(tb, k));
         L2[(t * n2 + k) * P + p] = v;
       });
-    }
+    });
     __syncthreads();
-    for (int i = g; i < n1 * groups; i += rows) {
-      const int t = i / groups, k0 = (i - t * groups) * K;
+    each_group<T>(rs, ax, [&](int tb, int t, int k0) {
       dense_group<true, T>(L2 + t * n2 * P + p, P, k0, ax, [&](int m, C v) {
-        L[(t * n2 + m) * P + p] = cmul(v, cconj(cload<C, T>(w, t * m)));
+        L[(t * n2 + m) * P + p] = cmul(v, cconj(twiddle_at<SUB, C, T>(w, m, tb, rs.half)));
       });
-    }
+    });
   } else {
     with_radix<T>(n2, [&](auto rc) {
       constexpr int R = decltype(rc)::value;
-      for (int t = g; t < n1; t += rows) {
+      rs.each(n1, [&](int tb, int t) {
         C u[R];
 #pragma unroll
         for (int k = 0; k < R; ++k) u[k] = L[(t * R + k) * P + p];
         dft_reg<R, false, T>(u);
 #pragma unroll
-        for (int k = 0; k < R; ++k) dot += G.solve(u[k], zfactors(t + n1 * k));
+        for (int k = 0; k < R; ++k) dot += G.solve(u[k], zfactors(tb, k));
         dft_reg<R, true, T>(u);
 #pragma unroll
         for (int m = 0; m < R; ++m) {
-          if (m > 0) u[m] = cmul(u[m], cconj(cload<C, T>(w, t * m)));
+          if (m > 0) u[m] = cmul(u[m], cconj(twiddle_at<SUB, C, T>(w, m, tb, rs.half)));
           L[(t * R + m) * P + p] = u[m];
         }
-      }
+      });
     });
   }
   __syncthreads();
   with_radix<T>(n1, [&](auto rc) {
     constexpr int R = decltype(rc)::value;
-    for (int m = g; m < n2; m += rows) {
+    rs.each(n2, [&](int, int m) {
       C v[R];
 #pragma unroll
       for (int t = 0; t < R; ++t) v[t] = L[(t * n2 + m) * P + p];
@@ -387,7 +435,7 @@ gen_z(typename CT<T>::type* S, GenAxis<T> ax, int units, int ny, int nxh, Tables
 #pragma unroll
         for (int k = 0; k < R; ++k) base[(m + n2 * k) * zs] = v[k];
       }
-    }
+    });
   });
   if constexpr (kDot) {
     const double total = block_reduce_dyn(wk * dot, red);
@@ -432,7 +480,7 @@ __device__ __forceinline__ void fill_slots(unsigned short* slot, const GenAxis<T
     slot[k] = static_cast<unsigned short>(ax.dense ? k : (k % ax.n1) * ax.n2 + k / ax.n1);
 }
 
-template <typename T, int MODE, bool kWave>
+template <typename T, int MODE, int SUB>
 __global__ void __launch_bounds__(kGenThreads<T>, kGenWaves<T>)
 gen_r2c(const T* f, typename CT<T>::type* __restrict__ S, GenAxis<T> ax, int PB, int64_t rows_total,
         int64_t field_stride, int64_t spec_stride, const int* active, XUpdate<T> upd) {
@@ -445,8 +493,8 @@ gen_r2c(const T* f, typename CT<T>::type* __restrict__ S, GenAxis<T> ax, int PB,
   C* L = reinterpret_cast<C*>(smem_raw);
   C* F = ax.dense ? L + n * ps : L;  // spectrum after step 2
   unsigned short* slot = reinterpret_cast<unsigned short*>(L + n * ps * (ax.dense ? 2 : 1));
-  const int P = kWave ? 64 : 1 << ax.lp, p = int(threadIdx.x) & (P - 1);
-  const int g = row_index<kWave>(ax.lp), rows = int(blockDim.x) >> ax.lp;
+  const int P = SUB ? 64 / SUB : 1 << ax.lp, p = int(threadIdx.x) & (P - 1);
+  const RowSet<SUB> rs(ax.lp);
   const int64_t row0 = 2 * int64_t(blockIdx.x) * PB;
   const int have = int(min(int64_t(2 * PB), rows_total - row0));  // rows of this workgroup
   const int64_t plane = rows_total * n;
@@ -507,10 +555,10 @@ gen_r2c(const T* f, typename CT<T>::type* __restrict__ S, GenAxis<T> ax, int PB,
     }
   }
   __syncthreads();
-  if (p < NP) gen_step1<false, T>(L, ps, p, g, rows, ax, [&](int e) -> C { return L[e * ps + p]; });
+  if (p < NP) gen_step1<false, SUB, T>(L, ps, p, rs, ax, [&](int e) -> C { return L[e * ps + p]; });
   __syncthreads();
   if (p < NP)
-    gen_step2<false, T>(L, ps, p, g, rows, ax, [&](int t, int k, C v) {
+    gen_step2<false, SUB, T>(L, ps, p, rs, ax, [&](int t, int k, C v) {
       F[(ax.dense ? t + ax.n1 * k : t * ax.n2 + k) * ps + p] = v;
     });
   __syncthreads();
@@ -565,7 +613,7 @@ gen_r2c(const T* f, typename CT<T>::type* __restrict__ S, GenAxis<T> ax, int PB,
   }
 }
 
-template <typename T, bool kDir, bool kWave>
+template <typename T, bool kDir, int SUB>
 __global__ void __launch_bounds__(kGenThreads<T>, kGenWaves<T>)
 gen_c2r(const typename CT<T>::type* __restrict__ S, T* z, GenAxis<T> ax, int PB, int64_t rows_total,
         int64_t field_stride, int64_t spec_stride, const int* active, const double* beta, const T* pin) {
@@ -577,8 +625,8 @@ gen_c2r(const typename CT<T>::type* __restrict__ S, T* z, GenAxis<T> ax, int PB,
   C* L = reinterpret_cast<C*>(smem_raw);
   C* F = ax.dense ? L + n * ps : L;
   unsigned short* slot = reinterpret_cast<unsigned short*>(L + n * ps * (ax.dense ? 2 : 1));
-  const int P = kWave ? 64 : 1 << ax.lp, p = int(threadIdx.x) & (P - 1);
-  const int g = row_index<kWave>(ax.lp), rows = int(blockDim.x) >> ax.lp;
+  const int P = SUB ? 64 / SUB : 1 << ax.lp, p = int(threadIdx.x) & (P - 1);
+  const RowSet<SUB> rs(ax.lp);
   const int64_t row0 = 2 * int64_t(blockIdx.x) * PB;
   const int have = int(min(int64_t(2 * PB), rows_total - row0));
   const int64_t plane = rows_total * n;
@@ -633,10 +681,10 @@ gen_c2r(const typename CT<T>::type* __restrict__ S, T* z, GenAxis<T> ax, int PB,
     }
   }
   __syncthreads();
-  if (p < NP) gen_step1<true, T>(L, ps, p, g, rows, ax, [&](int e) -> C { return L[e * ps + p]; });
+  if (p < NP) gen_step1<true, SUB, T>(L, ps, p, rs, ax, [&](int e) -> C { return L[e * ps + p]; });
   __syncthreads();
   if (p < NP)
-    gen_step2<true, T>(L, ps, p, g, rows, ax, [&](int t, int k, C v) {
+    gen_step2<true, SUB, T>(L, ps, p, rs, ax, [&](int t, int k, C v) {
       F[(ax.dense ? t + ax.n1 * k : t * ax.n2 + k) * ps + p] = v;
     });
   __syncthreads();
@@ -673,6 +721,21 @@ gen_c2r(const typename CT<T>::type* __restrict__ S, T* z, GenAxis<T> ax, int PB,
   }
 }
 
+// Row form of a shape (see RowSet).
+inline int sub_of(const AxisPlan& p, const GenShape& sh) {
+  if (sh.P == 64) return 1;
+  return sh.P == 32 && !(p.dense && p.n1 == 1) ? 2 : 0;
+}
+#define VXL_GS(A)   \
+  do {              \
+    if (sub == 1)   \
+      VXL_G(A, 1);  \
+    else if (sub == 2) \
+      VXL_G(A, 2);  \
+    else            \
+      VXL_G(A, 0);  \
+  } while (0)
+
 template <typename T>
 GenAxis<T> axis_view(const AxisPlan& p, const GenShape& sh, const void* w) {
   GenAxis<T> a;
@@ -687,13 +750,22 @@ GenAxis<T> axis_view(const AxisPlan& p, const GenShape& sh, const void* w) {
   return a;
 }
 
-// The widest column count whose tile fits, and the row count that finishes the
+// Columns: the most of 64, 32 and 16 with which two workgroups share a CU's
+// LDS, else the most that fit one.  (118-point dense z pass, FP64: 16 columns
+// 293 us, 32 in one workgroup per CU 380 us; 150 points, FP32: 64 columns in
+// 77 KB 164 us, 32 columns 253 us.)  The row count is the one that finishes the
 // two steps in the fewest rounds.
 template <typename T>
 GenShape pick_shape(const AxisPlan& p, int widest, size_t (*lds)(const AxisPlan&, int P)) {
   GenShape s;
-  s.P = widest;
-  while (s.P > 4 && lds(p, s.P) > kGenLds) s.P /= 2;
+  s.P = 0;
+  for (size_t limit : {kGenLds, 2 * kGenLds})
+    for (int P = widest; P >= 16 && !s.P; P /= 2)
+      if (lds(p, P) <= limit) s.P = P;
+  if (!s.P) {
+    s.P = std::min(widest, 8);
+    while (s.P > 4 && lds(p, s.P) > 2 * kGenLds) s.P /= 2;
+  }
   s.lds = lds(p, s.P);
   const int most = kGenThreads<T> / s.P, step = std::max(1, 64 / s.P);
   const int work2 = p.dense ? p.n1 * (p.hpad / kDenseOut<T>) : p.n1;
@@ -811,25 +883,16 @@ int launch_gen_r2c(const GenX<T>& g, int nrhs, const T* r, typename CT<T>::type*
   const GenAxis<T> ax = axis_view<T>(g.plan, g.shape, g.w);
   const XUpdate<T> u = upd ? *upd : XUpdate<T>{};
   const T* in = upd && spec ? upd->q : r;
-  const bool wave = g.shape.P == 64;
+  const int sub = sub_of(g.plan, g.shape);
 #define VXL_G(MODE, WV)                                                                                              \
   hipLaunchKernelGGL((gen_r2c<T, MODE, WV>), grid, block, g.shape.lds, s, in, S, ax, PB, g.rows, g.field_stride,       \
                      g.spec_stride, g.active, u)
   if (!upd) {
-    if (wave)
-      VXL_G(kGenPlain, true);
-    else
-      VXL_G(kGenPlain, false);
+    VXL_GS(kGenPlain);
   } else if (spec) {
-    if (wave)
-      VXL_G(kGenSpec, true);
-    else
-      VXL_G(kGenSpec, false);
+    VXL_GS(kGenSpec);
   } else {
-    if (wave)
-      VXL_G(kGenUpd, true);
-    else
-      VXL_G(kGenUpd, false);
+    VXL_GS(kGenUpd);
   }
 #undef VXL_G
   VXL_HIP(hipGetLastError());
@@ -843,20 +906,14 @@ int launch_gen_c2r(const GenX<T>& g, int nrhs, const typename CT<T>::type* S, T*
   const int64_t pairs = (g.rows + 1) / 2;
   const dim3 grid(unsigned((pairs + PB - 1) / PB), unsigned(nrhs)), block(unsigned(g.shape.P * g.shape.rows));
   const GenAxis<T> ax = axis_view<T>(g.plan, g.shape, g.w);
-  const bool wave = g.shape.P == 64;
+  const int sub = sub_of(g.plan, g.shape);
 #define VXL_G(DIR, WV)                                                                                            \
   hipLaunchKernelGGL((gen_c2r<T, DIR, WV>), grid, block, g.shape.lds, s, S, z, ax, PB, g.rows, g.field_stride,     \
                      g.spec_stride, g.active, beta, pin)
   if (beta) {
-    if (wave)
-      VXL_G(true, true);
-    else
-      VXL_G(true, false);
+    VXL_GS(true);
   } else {
-    if (wave)
-      VXL_G(false, true);
-    else
-      VXL_G(false, false);
+    VXL_GS(false);
   }
 #undef VXL_G
   VXL_HIP(hipGetLastError());
@@ -871,19 +928,13 @@ int launch_gen_y(const AxisPlan& plan, const GenShape& sh, const typename CT<T>:
   if (cols > INT32_MAX - 64 || int64_t(plan.n) * W > INT32_MAX) return fail("grid too large for the FFT y pass");
   const dim3 grid(unsigned((cols + sh.units - 1) / sh.units), unsigned(nrhs)), block(unsigned(sh.P * sh.rows));
   const GenAxis<T> ax = axis_view<T>(plan, sh, w);
-  const bool wave = sh.P == 64;
+  const int sub = sub_of(plan, sh);
 #define VXL_G(INV, WV) \
   hipLaunchKernelGGL((gen_y<INV, T, WV>), grid, block, sh.lds, s, S, src, ax, int(cols), W, stride, active)
   if (inverse) {
-    if (wave)
-      VXL_G(true, true);
-    else
-      VXL_G(true, false);
+    VXL_GS(true);
   } else {
-    if (wave)
-      VXL_G(false, true);
-    else
-      VXL_G(false, false);
+    VXL_GS(false);
   }
 #undef VXL_G
   VXL_HIP(hipGetLastError());
@@ -898,20 +949,14 @@ int launch_gen_z(const AxisPlan& plan, const GenShape& sh, const Tables<T>& tb, 
   if (cols > INT32_MAX - 64) return fail("grid too large for the FFT z pass");
   const dim3 grid(unsigned((cols + sh.units - 1) / sh.units), unsigned(nrhs)), block(unsigned(sh.P * sh.rows));
   const GenAxis<T> ax = axis_view<T>(plan, sh, tb.wz);
-  const bool wave = sh.P == 64;
+  const int sub = sub_of(plan, sh);
 #define VXL_G(DOT, WV)                                                                                        \
   hipLaunchKernelGGL((gen_z<T, DOT, WV>), grid, block, sh.lds, s, S, ax, sh.units, ny, nxh, tb, lam, mu, inv_vn, \
                      stride, active, nyq, partial, media, group_rhs)
   if (partial) {
-    if (wave)
-      VXL_G(true, true);
-    else
-      VXL_G(true, false);
+    VXL_GS(true);
   } else {
-    if (wave)
-      VXL_G(false, true);
-    else
-      VXL_G(false, false);
+    VXL_GS(false);
   }
 #undef VXL_G
   VXL_HIP(hipGetLastError());
