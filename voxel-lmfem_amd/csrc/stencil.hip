@@ -720,7 +720,9 @@ apply_kernel_v2(ApplyArgs<T> a) {
   // plane is resident (one layer earlier) and kept in registers.
   double rr = 0.0;  // kResid: sum of r^2 over the nodes this thread writes
   const double rscale = kResid && a.rscale ? a.rscale[bid.rhs] : 1.0;
-  T pq = T(0);  // at most zchunk nodes per thread; FP64 from the block sum on
+  // p . q: each node's product in T, summed in FP64, so that the total does not
+  // depend on how the nodes are dealt to tiles and chunks.
+  double pq = 0.0;
   auto node_value = [&](T (&v)[3], int buf) {
 #pragma unroll
     for (int c = 0; c < 3; ++c) v[c] = su[buf][c][(yl + 1) * TL::PX + xl + 1];
@@ -866,7 +868,7 @@ apply_kernel_v2(ApplyArgs<T> a) {
       } else {
 #pragma unroll
         for (int cc = 0; cc < 3; ++cc) out[cc * n + node] = acc[cc];
-        if constexpr (kFuse) pq = fma(pc[2], acc[2], fma(pc[1], acc[1], fma(pc[0], acc[0], pq)));
+        if constexpr (kFuse) pq += double(fma(pc[2], acc[2], fma(pc[1], acc[1], pc[0] * acc[0])));
       }
     }
     // kPF: no barrier here.  The next layer writes the other force buffer
@@ -879,7 +881,7 @@ apply_kernel_v2(ApplyArgs<T> a) {
     if (z + 1 < z1) layer(std::integral_constant<int, 1>(), z + 1, Bf2, Ftp2, Bf, Ftp, pnB, pnA);
   }
   if constexpr (kFuse || kResid) {
-    const double total = block_reduce_sum<TL::NT>(kResid ? rr : double(pq), red);
+    const double total = block_reduce_sum<TL::NT>(kResid ? rr : pq, red);
     if (tid == 0)
       a.partial[(int64_t(bid.rhs) * gridDim.y + bid.chunk) * gridDim.x + bid.tile] = total;
   }
@@ -915,6 +917,15 @@ void apply_grid(const vxl_cell* cell, int nrhs, int& tiles_x, int& tiles, int& c
   // Enough workgroups to fill 256 CUs several times; chunks of >= zmin
   // planes (default 8: the recomputed layer per chunk stays <= 1/8).
   if (zmin <= 0) zmin = cell->zmin[std::is_same<T, double>::value ? 1 : 0];
+  // Small grids leave CUs idle at that depth, and a launch then takes as long as
+  // one chunk's march (about 1.8 us a layer): chunks shrink to two planes while
+  // all workgroups still run at once (two per CU).  Six loads, default tiles:
+  // 18 x 25 x 21 FP32 18.2 -> 7.8 us, FP64 17.8 -> 10.0; 32^3 17.1 -> 10.6 and
+  // 16.9 -> 13.9; 40-ish 19.2 -> 15.8; 64^3 and larger keep eight planes.
+  if (zmin == kDefaultChunkPlanes) {
+    const int at_once = std::max(1, 512 / (tiles * nrhs));
+    zmin = std::max(kMinChunkPlanes, std::min(zmin, (nz + at_once - 1) / at_once));
+  }
   chunks = (4096 + tiles * nrhs - 1) / (tiles * nrhs);
   chunks = std::max(1, std::min(chunks, nz / std::max(1, zmin)));
   zchunk = (nz + chunks - 1) / chunks;
