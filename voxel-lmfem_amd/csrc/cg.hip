@@ -326,10 +326,17 @@ center_copy_kernel(double* f, TR* r, const double* mean, int64_t n, double* part
 // then the scalar update selected by op.
 __global__ void __launch_bounds__(kBlock)
 finalize_kernel(const double* partial, int nblk, int op, double* scal, int nrhs, int* active,
-                int* restart, int iteration, double tol, int* stop, double* hist) {
+                int* restart, int iteration, double tol, int* stop, double* hist, int rho_in, int rho_out,
+                double* host_rr, int* host_stop) {
   const int k = blockIdx.x;
   if (active && !active[k]) {
-    if (hist && threadIdx.x == 0) hist[k] = 0.0;  // no step for an inactive system
+    if (threadIdx.x == 0) {
+      if (hist) hist[k] = 0.0;  // no step for an inactive system
+      if (host_rr) {
+        host_rr[k] = scal[kRR * nrhs + k];
+        host_stop[k] = stop[k];
+      }
+    }
     return;
   }
   double acc = 0;
@@ -356,24 +363,21 @@ finalize_kernel(const double* partial, int nblk, int op, double* scal, int nrhs,
         stop[k] = iteration;
         active[k] = 0;
       }
+      if (host_rr) {
+        host_rr[k] = acc;
+        host_stop[k] = stop[k];
+      }
       break;
     case kOpAlpha: {
       S[kPQ * nrhs + k] = acc;
-      const bool bad = !isfinite(acc) || acc <= 0.0;
-      S[kAlpha * nrhs + k] = bad ? 0.0 : S[kRho * nrhs + k] / fmax(acc, 1e-300);
+      S[kAlpha * nrhs + k] = step_alpha(S[rho_in * nrhs + k], acc);
       if (hist) hist[k] = S[kAlpha * nrhs + k];
+      if (restart) restart[k] = 0;  // consumed by the beta kernel before this step
       break;
     }
     case kOpBeta: {
-      const double rho_old = S[kRho * nrhs + k];
-      double beta = rho_old > 0.0 ? acc / rho_old : 0.0;
-      if (restart && restart[k]) {  // consumed here, so a captured block needs no host reset
-        beta = 0.0;
-        restart[k] = 0;
-      }
-      if (!isfinite(beta)) beta = 0.0;
-      S[kBeta * nrhs + k] = beta;
-      S[kRho * nrhs + k] = acc;
+      S[kBeta * nrhs + k] = step_beta(S[rho_in * nrhs + k], acc, restart && restart[k]);
+      S[rho_out * nrhs + k] = acc;
       break;
     }
   }
@@ -404,9 +408,10 @@ template int launch_dot<float, float>(const float*, const float*, int64_t, int, 
 template int launch_dot<double, double>(const double*, const double*, int64_t, int, double*, const int*, hipStream_t);
 
 int launch_finalize(const double* partial, int nblk, int op, double* scal, int nrhs, int* active,
-                    int* restart, hipStream_t s, int iteration, double tol, int* stop, double* hist) {
+                    int* restart, hipStream_t s, int iteration, double tol, int* stop, double* hist, int rho_in,
+                    int rho_out, double* host_rr, int* host_stop) {
   hipLaunchKernelGGL(finalize_kernel, dim3(nrhs), dim3(kBlock), 0, s, partial, nblk, op, scal, nrhs,
-                     active, restart, iteration, tol, stop, hist);
+                     active, restart, iteration, tol, stop, hist, rho_in, rho_out, host_rr, host_stop);
   VXL_HIP(hipGetLastError());
   return VXL_OK;
 }

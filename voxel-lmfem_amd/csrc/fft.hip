@@ -359,7 +359,12 @@ fft_x4_r2c(const T* __restrict__ r, SC* __restrict__ S, int64_t rows, int PP,
   static_assert(!kSpec || std::is_same<SC, C>::value, "the residual spectrum is stored at full precision");
   extern __shared__ double2 smem_raw[];
   __shared__ double red[4];
-  if (active && !active[blockIdx.y]) return;
+  if (active && !active[blockIdx.y]) {
+    if constexpr (kUpd || kSpec) update_skipped(upd, blockIdx.y, blockIdx.x == 0);
+    return;
+  }
+  double step = 0.0;
+  if constexpr (kUpd || kSpec) step = update_alpha(upd, blockIdx.y, blockIdx.x == 0, red);
   C* L = reinterpret_cast<C*>(smem_raw);
   const int P = 3 * PP;
   const int t = threadIdx.x % lanes, p = threadIdx.x / lanes;
@@ -377,7 +382,7 @@ fft_x4_r2c(const T* __restrict__ r, SC* __restrict__ S, int64_t rows, int PP,
   C* T1 = L + p * XT::stride;
   double rr = 0.0;
   const int64_t base = int64_t(blockIdx.y) * field_stride;
-  const T alpha = kUpd ? T(upd.alpha[blockIdx.y]) : T(0);
+  const T alpha = T(step);
   // Distinct fields: restrict lets the loads of later entries run ahead of
   // the stores of earlier ones.
   T* __restrict__ ur = kUpd ? upd.r + base : nullptr;
@@ -440,7 +445,7 @@ fft_x4_r2c(const T* __restrict__ r, SC* __restrict__ S, int64_t rows, int PP,
   __syncthreads();
   // Two-for-one split.
   double spec_rr = 0.0;  // kSpec: sum of w(k) |R^(k)|^2 over this thread's entries
-  const T spec_alpha = kSpec ? T(upd.alpha[blockIdx.y]) : T(0);
+  const T spec_alpha = T(step);
   for (int idx = threadIdx.x; idx < PP * nxh; idx += blockDim.x) {
     const int a = idx / nxh, k = idx - a * nxh;
     const int64_t rr = 2 * (int64_t(blockIdx.x) * PP + a);
@@ -500,11 +505,12 @@ template <typename T, int N1, int N2, bool kDir, typename SC>
 __global__ void __launch_bounds__(256)
 fft_x4_c2r(const SC* __restrict__ S, T* z, int64_t rows, int PP,
            const typename CT<T>::type* __restrict__ w, int64_t field_stride, int64_t spec_stride,
-           const int* active, const double* beta, const T* pin) {
+           const int* active, const double* beta, const T* pin, BetaFold fold) {
   using C = typename CT<T>::type;
   using XT = XTile<N1, N2>;
   constexpr int n = XT::n, nxh = n / 2 + 1, lanes = FourStep<N1, N2>::lanes;
   extern __shared__ double2 smem_raw[];
+  __shared__ double red[4];
   if (active && !active[blockIdx.y]) return;
   C* L = reinterpret_cast<C*>(smem_raw);
   const int P = 3 * PP;
@@ -521,7 +527,8 @@ fft_x4_c2r(const SC* __restrict__ S, T* z, int64_t rows, int PP,
   const int64_t im_off = q == 2 ? 2 * plane + (rho + 1) * n : plane + rho * n + (q == 1 ? n : 0);
   const bool re_ok = q == 1 ? rho + 1 < rows : rho < rows;
   const bool im_ok = rho + (q == 0 ? 0 : 1) < rows;
-  const T b = kDir ? T(beta[blockIdx.y]) : T(0);
+  T b = T(0);
+  if constexpr (kDir) b = T(fold.partial ? fold_beta(fold, blockIdx.y, blockIdx.x == 0, red) : beta[blockIdx.y]);
   const bool keep = kDir && b != T(0);
   T prev[2][N2];
   if (keep && live && t < N1) {
@@ -770,11 +777,11 @@ void launch_x4_r2c(int n, dim3 grid, int thr, size_t lds, hipStream_t s, const T
 template <typename T, bool kDir, typename SC>
 void launch_x4_c2r(int n, dim3 grid, int thr, size_t lds, hipStream_t s, const SC* S, T* z,
                    int64_t rows, int PP, const typename CT<T>::type* w, int64_t fstride, int64_t sstride,
-                   const int* active, const double* beta, const T* pin) {
+                   const int* active, const double* beta, const T* pin, const BetaFold& fold) {
 #define VXL_X4C(N, A, B)                                                                                      \
   case N:                                                                                                   \
     hipLaunchKernelGGL((fft_x4_c2r<T, A, B, kDir, SC>), grid, dim3(thr), lds, s, S, z, rows, PP, w, fstride, \
-                       sstride, active, beta, pin);                                                         \
+                       sstride, active, beta, pin, fold);                                                         \
     break;
   switch (n) { VXL_X4_CASES(VXL_X4C) }
 #undef VXL_X4C
@@ -926,6 +933,7 @@ struct CgHooks {
   const double* beta;
   std::function<int()> mid;
   const void* pin;  // previous search direction (nullptr: the output buffer, in place)
+  BetaFold fold;    // partial != nullptr: the last pass forms beta itself and mid() is not called
 };
 
 enum Stages { kForwardX = 1, kRest = 2, kAllStages = 3 };
@@ -1022,18 +1030,20 @@ int apply_stages(vxl_precond* pc, PrecondImpl* im, int nrhs, const T* r, T* z, h
                             active, nyq, part, media, grhs, s));
   }
   VXL_HIP(hipGetLastError());
-  if (cg) VXL_TRY(cg->mid());
+  const BetaFold fold = cg ? cg->fold : BetaFold{};
+  if (cg && !fold.partial) VXL_TRY(cg->mid());
   VXL_TRY(y_pass(true));
   if (im->x4 && cg)
     launch_x4_c2r<T, true, SC>(im->x4, dim3(bx4, nrhs), im->thr_x4, im->lds_x4, s, S, z, im->rows, im->pp4, tb.wx,
-                           fstride, im->spec_stride, active, cg->beta, static_cast<const T*>(cg->pin));
+                           fstride, im->spec_stride, active, cg->beta, static_cast<const T*>(cg->pin), fold);
   else if (im->x4)
     launch_x4_c2r<T, false, SC>(im->x4, dim3(bx4, nrhs), im->thr_x4, im->lds_x4, s, S, z, im->rows, im->pp4, tb.wx,
-                            fstride, im->spec_stride, active, nullptr, static_cast<const T*>(nullptr));
+                            fstride, im->spec_stride, active, nullptr, static_cast<const T*>(nullptr), fold);
   else if constexpr (!kFull)
     return fail("BF16 spectrum storage needs power-of-two axes");
   else
-    VXL_TRY(launch_gen_c2r<T>(gx, nrhs, S, z, cg ? cg->beta : nullptr, cg ? static_cast<const T*>(cg->pin) : nullptr, s));
+    VXL_TRY(launch_gen_c2r<T>(gx, nrhs, S, z, cg ? cg->beta : nullptr, cg ? static_cast<const T*>(cg->pin) : nullptr, fold,
+                              s));
   VXL_HIP(hipGetLastError());
   return VXL_OK;
 }
@@ -1068,47 +1078,49 @@ int precond_apply(vxl_precond* pc, int nrhs, const void* r, void* z, hipStream_t
 
 template <typename T>
 int precond_apply_cg(vxl_precond* pc, int nrhs, const T* r, T* p, double* rz_partial, const double* beta,
-                     const std::function<int()>& mid, const int* active, hipStream_t s) {
+                     const std::function<int()>& mid, const int* active, hipStream_t s, const BetaFold* fold) {
   auto* im = static_cast<PrecondImpl*>(pc->impl);
   if (nrhs < 1 || nrhs > pc->nrhs_max) return fail("precond nrhs out of range");
   if ((pc->precision == VXL_F64) != std::is_same<T, double>::value) return fail("precond precision mismatch");
-  const CgHooks cg{rz_partial, beta, mid, nullptr};
+  const CgHooks cg{rz_partial, beta, mid, nullptr, fold ? *fold : BetaFold{}};
   return apply_impl<T>(pc, im, nrhs, r, p, s, active, &cg);
 }
 template int precond_apply_cg<float>(vxl_precond*, int, const float*, float*, double*, const double*,
-                                     const std::function<int()>&, const int*, hipStream_t);
+                                     const std::function<int()>&, const int*, hipStream_t, const BetaFold*);
 template int precond_apply_cg<double>(vxl_precond*, int, const double*, double*, double*, const double*,
-                                      const std::function<int()>&, const int*, hipStream_t);
+                                      const std::function<int()>&, const int*, hipStream_t, const BetaFold*);
 
 template <typename T>
 int precond_cg_forward(vxl_precond* pc, int nrhs, T* r, T* x, const T* p, const T* q, const double* alpha,
-                       double* rr_partial, const int* active, hipStream_t s, bool sr) {
+                       double* rr_partial, const int* active, hipStream_t s, bool sr, const AlphaFold* fold) {
   auto* im = static_cast<PrecondImpl*>(pc->impl);
   if (nrhs < 1 || nrhs > pc->nrhs_max) return fail("precond nrhs out of range");
   if ((pc->precision == VXL_F64) != std::is_same<T, double>::value) return fail("precond precision mismatch");
   if (sr && (x || p)) return fail("the spectral residual takes no x update in the forward pass");
   if (!q) return apply_impl<T>(pc, im, nrhs, r, nullptr, s, active, nullptr, kForwardX, nullptr, sr);
-  const XUpdate<T> upd{r, x, p, q, alpha, rr_partial};
+  const XUpdate<T> upd{r, x, p, q, alpha, rr_partial, fold ? *fold : AlphaFold{}};
   return apply_impl<T>(pc, im, nrhs, r, nullptr, s, active, nullptr, kForwardX, &upd, sr);
 }
 template int precond_cg_forward<float>(vxl_precond*, int, float*, float*, const float*, const float*, const double*,
-                                       double*, const int*, hipStream_t, bool);
+                                       double*, const int*, hipStream_t, bool, const AlphaFold*);
 template int precond_cg_forward<double>(vxl_precond*, int, double*, double*, const double*, const double*,
-                                        const double*, double*, const int*, hipStream_t, bool);
+                                        const double*, double*, const int*, hipStream_t, bool, const AlphaFold*);
 
 template <typename T>
 int precond_cg_rest(vxl_precond* pc, int nrhs, T* p, double* rz_partial, const double* beta,
-                    const std::function<int()>& mid, const int* active, hipStream_t s, const T* p_old, bool sr) {
+                    const std::function<int()>& mid, const int* active, hipStream_t s, const T* p_old, bool sr,
+                    const BetaFold* fold) {
   auto* im = static_cast<PrecondImpl*>(pc->impl);
   if (nrhs < 1 || nrhs > pc->nrhs_max) return fail("precond nrhs out of range");
   if ((pc->precision == VXL_F64) != std::is_same<T, double>::value) return fail("precond precision mismatch");
-  const CgHooks cg{rz_partial, beta, mid, p_old};
+  const CgHooks cg{rz_partial, beta, mid, p_old, fold ? *fold : BetaFold{}};
   return apply_impl<T>(pc, im, nrhs, static_cast<const T*>(nullptr), p, s, active, &cg, kRest, nullptr, sr);
 }
 template int precond_cg_rest<float>(vxl_precond*, int, float*, double*, const double*, const std::function<int()>&,
-                                    const int*, hipStream_t, const float*, bool);
+                                    const int*, hipStream_t, const float*, bool, const BetaFold*);
 template int precond_cg_rest<double>(vxl_precond*, int, double*, double*, const double*,
-                                     const std::function<int()>&, const int*, hipStream_t, const double*, bool);
+                                     const std::function<int()>&, const int*, hipStream_t, const double*, bool,
+                                     const BetaFold*);
 
 bool precond_spectral_residual_ok(const vxl_precond* pc) {
   const auto* im = static_cast<const PrecondImpl*>(pc->impl);

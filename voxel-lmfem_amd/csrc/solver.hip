@@ -185,49 +185,67 @@ struct Steps {
     const int nrz = nblk_rz;
     hipStream_t on = st;
     form_beta = [so, nrz, on]() -> int {
-      return launch_finalize(so->partial_rz, nrz, kOpBeta, so->scal, so->R, so->active_dev, so->restart_dev, on);
+      return launch_finalize(so->partial_rz, nrz, kOpBeta, so->scal, so->R, so->active_dev, so->restart_dev, on, 0, 0.0,
+                             nullptr, nullptr, so->rho_slot, kRho + kRhoOdd - so->rho_slot);
     };
   }
+  // beta inside the last preconditioner pass, when the r . z partials are few.
+  BetaFold beta_fold() const {
+    if (nblk_rz > kFoldBlocks) return BetaFold{};
+    return BetaFold{s->partial_rz, nblk_rz, s->scal, R, s->rho_slot, kRho + kRhoOdd - s->rho_slot, s->restart_dev};
+  }
+  void rho_formed() { s->rho_slot = kRho + kRhoOdd - s->rho_slot; }
   int jacobi_step() {
     return jacobi_cg_step<T>(r, pnext, dinv, n, R, s->partial, s->jmean, s->jrz, s->scal, s->active_dev,
                              s->restart_dev, st, pcur);
   }
-  // [stencil, alpha, update, ||r||^2 with the latch at iteration `iter`]
-  int cg_update(int iter, bool& forward_done) {
+  // [stencil, alpha, update, ||r||^2 with the latch at iteration `iter`];
+  // host_rr / host_stop: pinned copies for a host check.
+  int cg_update(int iter, bool& forward_done, double* host_rr = nullptr, int* host_stop = nullptr) {
     int* act = s->active_dev;
     double* scal = s->scal;
     VXL_TRY(launch_apply_cg<T>(s->cell, R, pcur, q, act, s->partial_st, nullptr, st));
-    VXL_TRY(launch_finalize(s->partial_st, nblk_st, kOpAlpha, scal, R, act, nullptr, st, 0, 0.0, nullptr,
-                            ring ? hist_row : nullptr));
-    forward_done = false;
+    const int rho = s->rho_slot;
+    AlphaFold fold{};
+    if (ring && nblk_fx > 0 && nblk_st <= kFoldBlocks)
+      fold = AlphaFold{s->partial_st, nblk_st, scal, R, rho, hist_row, s->restart_dev};
+    else
+      VXL_TRY(launch_finalize(s->partial_st, nblk_st, kOpAlpha, scal, R, act, s->restart_dev, st, 0, 0.0, nullptr,
+                              ring ? hist_row : nullptr, rho));
+    auto norm = [&](const double* part, int blocks) -> int {
+      return launch_finalize(part, blocks, kOpRR, scal, R, act, nullptr, st, iter, tol, s->stop_dev, nullptr, rho, rho,
+                             host_rr, host_stop);
+    };
+    forward_done = nblk_fx > 0;
     if (ring && nblk_fx > 0) {  // r -= alpha q inside the preconditioner's x pass; x from the ring
       VXL_TRY(precond_cg_forward<T>(&s->pc, R, r, static_cast<T*>(nullptr), nullptr, q, scal + kAlpha * R,
-                                    s->partial_fx, act, st, sr));
-      VXL_TRY(launch_finalize(s->partial_fx, nblk_fx, kOpRR, scal, R, act, nullptr, st, iter, tol, s->stop_dev));
-      forward_done = true;
-    } else if (ring) {
-      VXL_TRY(launch_update_r<T>(r, q, len, R, scal + kAlpha * R, s->partial, act, st));
-      VXL_TRY(launch_finalize(s->partial, nblk, kOpRR, scal, R, act, nullptr, st, iter, tol, s->stop_dev));
-    } else if (nblk_fx > 0) {
-      VXL_TRY(precond_cg_forward<T>(&s->pc, R, r, x, p, q, scal + kAlpha * R, s->partial_fx, act, st));
-      VXL_TRY(launch_finalize(s->partial_fx, nblk_fx, kOpRR, scal, R, act, nullptr, st, iter, tol, s->stop_dev));
-      forward_done = true;
-    } else {
-      VXL_TRY(launch_update_xr<T>(x, r, p, q, len, R, scal + kAlpha * R, s->partial, act, st));
-      VXL_TRY(launch_finalize(s->partial, nblk, kOpRR, scal, R, act, nullptr, st, iter, tol, s->stop_dev));
+                                    s->partial_fx, act, st, sr, &fold));
+      return norm(s->partial_fx, nblk_fx);
     }
-    return VXL_OK;
+    if (ring) {
+      VXL_TRY(launch_update_r<T>(r, q, len, R, scal + kAlpha * R, s->partial, act, st));
+      return norm(s->partial, nblk);
+    }
+    if (nblk_fx > 0) {
+      VXL_TRY(precond_cg_forward<T>(&s->pc, R, r, x, p, q, scal + kAlpha * R, s->partial_fx, act, st));
+      return norm(s->partial_fx, nblk_fx);
+    }
+    VXL_TRY(launch_update_xr<T>(x, r, p, q, len, R, scal + kAlpha * R, s->partial, act, st));
+    return norm(s->partial, nblk);
   }
-  // [FFT passes of M r, beta, p = M r + beta p] (or the Jacobi step); the
-  // beta kernel consumes the restart flags on the device.
+  // [FFT passes of M r, beta, p = M r + beta p] (or the Jacobi step); beta
+  // takes the restart flags on the device and the next alpha clears them.
   int precond_step(bool forward_done) {
     if (jacobi) return jacobi_step();
     int* act = s->active_dev;
     if (!forward_done)
       VXL_TRY(precond_cg_forward<T>(&s->pc, R, r, static_cast<T*>(nullptr), nullptr, nullptr, nullptr, nullptr, act,
                                     st, sr));
-    return precond_cg_rest<T>(&s->pc, R, pnext, s->partial_rz, s->scal + kBeta * R, form_beta, act, st,
-                              pcur == pnext ? nullptr : pcur, sr);
+    const BetaFold fold = beta_fold();
+    VXL_TRY(precond_cg_rest<T>(&s->pc, R, pnext, s->partial_rz, s->scal + kBeta * R, form_beta, act, st,
+                               pcur == pnext ? nullptr : pcur, sr, &fold));
+    rho_formed();
+    return VXL_OK;
   }
 };
 
@@ -302,6 +320,16 @@ int prepare_block_graph(vxl_solver* s, double tol) {
   const bool fused = steps.nblk_fx > 0;
   int cur = 0;
   std::vector<int> pend;
+  // A block forms an even number of betas, so it leaves the r . z slot as it
+  // found it; every block starts after a multiple of kCheckStride of them.
+  const int rho_slot = s->rho_slot;
+  struct Restore {
+    vxl_solver* s;
+    int v;
+    ~Restore() { s->rho_slot = v; }
+  } restore{s, rho_slot};
+  s->rho_slot = kRho;
+  static_assert(kCheckStride % 2 == 0, "even number of betas per block");
   if (ring) {
     cur = ring_block_start(s->nslot);
     if (cur < 0) return give_up();
@@ -483,6 +511,7 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
   VXL_HIP(hipMemcpyAsync(s->macro_dev, macro_host, sizeof(double) * 6 * R, hipMemcpyHostToDevice, st));
   VXL_HIP(hipMemsetAsync(scal, 0, sizeof(double) * kNumSlots * R, st));
   VXL_HIP(hipMemsetAsync(s->stop_dev, 0, sizeof(int) * R, st));
+  s->rho_slot = kRho;
   VXL_TRY(upload_flags());
   // f = P0 rhs(E), r = f and ||f||^2 (one pass after the component means)
   VXL_TRY(launch_rhs(cell, R, s->macro_dev, s->f, s->rhs_sig, st));
@@ -573,8 +602,12 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
     VXL_TRY(steps.jacobi_step());
   else if (steps.sr)
     VXL_TRY(steps.precond_step(false));  // R^ from r, then the rest with p = z
-  else
-    VXL_TRY(precond_apply_cg<T>(&s->pc, R, r, slots[0], s->partial_rz, scal + kBeta * R, steps.form_beta, act, st));
+  else {
+    const BetaFold fold = steps.beta_fold();
+    VXL_TRY(precond_apply_cg<T>(&s->pc, R, r, slots[0], s->partial_rz, scal + kBeta * R, steps.form_beta, act, st,
+                                &fold));
+    steps.rho_formed();
+  }
   VXL_HIP(hipEventRecord(s->ev[1], st));
 
   int it = 0;
@@ -617,11 +650,12 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
     if (ring) {
       steps.pcur = slots[cur];
       steps.hist_row = s->hist + int64_t(pend.size()) * R;
-      VXL_TRY(steps.cg_update(iter, fd));
-      pend.push_back(cur);
-      return VXL_OK;
     }
-    return steps.cg_update(iter, fd);
+    // A host check follows these iterations: their norms go straight to pinned memory.
+    const bool check = iter == 1 || iter % kCheckStride == 0 || iter == max_iter;
+    VXL_TRY(steps.cg_update(iter, fd, check ? pin_scal : nullptr, check ? pin_stop : nullptr));
+    if (ring) pend.push_back(cur);
+    return VXL_OK;
   };
   auto precond_step = [&](bool fd) -> int {
     if (!ring) return steps.precond_step(fd);
@@ -644,7 +678,8 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
     if (replay) {
       VXL_TRY(block_graph());
       // The ring must be in the state the block was captured from.
-      replay = s->block_graph != nullptr && (!ring || (pend.empty() && cur == s->block_graph_cur0));
+      replay = s->block_graph != nullptr && s->rho_slot == kRho &&
+               (!ring || (pend.empty() && cur == s->block_graph_cur0));
     }
     if (replay) {
       if (s->block_graph_fused && !forward_done)  // r was replaced: form its spectrum first
@@ -671,9 +706,14 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
     }
     pending = true;
     if (it == 1 || it % kCheckStride == 0 || it == max_iter) {
-      VXL_TRY(read_slot(kRR, rr));
-      VXL_HIP(hipMemcpyAsync(pin_stop, s->stop_dev, sizeof(int) * R, hipMemcpyDeviceToHost, st));
-      VXL_HIP(hipStreamSynchronize(st));
+      if (base >= 0) {  // replayed block: its last norm is on the device only
+        VXL_TRY(read_slot(kRR, rr));
+        VXL_HIP(hipMemcpyAsync(pin_stop, s->stop_dev, sizeof(int) * R, hipMemcpyDeviceToHost, st));
+        VXL_HIP(hipStreamSynchronize(st));
+      } else {
+        VXL_HIP(hipStreamSynchronize(st));
+        rr.assign(pin_scal, pin_scal + R);
+      }
       std::vector<int> which(R, 0), latched(R, 0);
       bool anyw = false;
       for (int k = 0; k < R; ++k) {
@@ -716,7 +756,7 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
         VXL_HIP(hipMemsetAsync(s->stop_dev, 0, sizeof(int) * R, st));  // eager, never captured
       }
       if (flush_each_check) VXL_TRY(flush());
-      VXL_TRY(upload_flags());
+      if (anyw) VXL_TRY(upload_flags());  // otherwise the device flags are the host's already
       if (!any_active()) break;
     }
   }

@@ -6,7 +6,9 @@
 namespace vxl {
 
 // Device scalar slots, scal[slot * nrhs + k].
-enum ScalarSlot { kRho = 0, kPQ, kAlpha, kBeta, kRR, kFF, kTmp, kNumSlots };
+// r . z alternates between two slots (kRho + parity): a kernel that forms beta
+// in every workgroup reads the old value while one of them writes the new.
+enum ScalarSlot { kRho = 0, kRhoOdd, kPQ, kAlpha, kBeta, kRR, kFF, kTmp, kNumSlots };
 // finalize_kernel operations.
 enum FinalizeOp { kOpStore = 0, kOpRho, kOpFF, kOpRR, kOpAlpha, kOpBeta };
 
@@ -18,10 +20,66 @@ template <typename A, typename B>
 int launch_dot(const A* a, const B* b, int64_t len, int nrhs, double* partial, const int* active,
                hipStream_t s);
 // kOpRR with `stop` latches the first iteration below tol: stop[k] = iteration,
-// active[k] = 0 (on the device).
+// active[k] = 0 (on the device); host_rr / host_stop (pinned host memory,
+// optional) receive ||r||^2 and the latch of every system.  kOpAlpha reads r . z
+// from slot rho_in and clears restart (consumed by the beta before it); kOpBeta
+// reads rho_in and writes rho_out.
 int launch_finalize(const double* partial, int nblk, int op, double* scal, int nrhs, int* active,
                     int* restart, hipStream_t s, int iteration = 0, double tol = 0.0,
-                    int* stop = nullptr, double* hist = nullptr);
+                    int* stop = nullptr, double* hist = nullptr, int rho_in = kRho, int rho_out = kRho,
+                    double* host_rr = nullptr, int* host_stop = nullptr);
+// The alpha and beta updates inside the kernel that uses them: every workgroup
+// of a right-hand side sums that side's partials itself (same order, same
+// value) and its first workgroup stores the scalars.  Taken while a side has
+// at most kFoldBlocks partials: a separate one-workgroup launch costs 3.3 us
+// and a gap on grids whose passes take 5 to 10 us, the sum about 1 us.
+constexpr int kFoldBlocks = 512;
+struct AlphaFold {
+  const double* partial;  // p . q (nullptr: alpha is ready in its slot)
+  int nblk;
+  double* scal;
+  int nrhs;
+  int rho;  // slot of r . z
+  double* hist;
+  int* restart;
+};
+struct BetaFold {
+  const double* partial;  // r . z (nullptr: beta is ready in its slot)
+  int nblk;
+  double* scal;
+  int nrhs;
+  int rho_in, rho_out;
+  const int* restart;
+};
+__device__ __forceinline__ double step_alpha(double rho, double pq) {
+  const bool bad = !isfinite(pq) || pq <= 0.0;
+  return bad ? 0.0 : rho / fmax(pq, 1e-300);
+}
+__device__ __forceinline__ double step_beta(double rho_old, double rho, bool restart) {
+  const double beta = rho_old > 0.0 ? rho / rho_old : 0.0;
+  return restart || !isfinite(beta) ? 0.0 : beta;
+}
+// alpha of system k in every thread; `first`: this workgroup stores it.
+__device__ __forceinline__ double fold_alpha(const AlphaFold& f, int k, bool first, double* red) {
+  const double pq = block_total_dyn(f.partial + int64_t(k) * f.nblk, f.nblk, red);
+  const double a = step_alpha(f.scal[f.rho * f.nrhs + k], pq);
+  if (first && threadIdx.x == 0) {
+    f.scal[kPQ * f.nrhs + k] = pq;
+    f.scal[kAlpha * f.nrhs + k] = a;
+    if (f.hist) f.hist[k] = a;
+    if (f.restart) f.restart[k] = 0;
+  }
+  return a;
+}
+__device__ __forceinline__ double fold_beta(const BetaFold& f, int k, bool first, double* red) {
+  const double rho = block_total_dyn(f.partial + int64_t(k) * f.nblk, f.nblk, red);
+  const double b = step_beta(f.scal[f.rho_in * f.nrhs + k], rho, f.restart && f.restart[k]);
+  if (first && threadIdx.x == 0) {
+    f.scal[kBeta * f.nrhs + k] = b;
+    f.scal[f.rho_out * f.nrhs + k] = rho;
+  }
+  return b;
+}
 // Stored search directions p_t (nrhs fields each) whose steps alpha_t are
 // still to be added to x64.
 constexpr int kMaxDirections = 16;
@@ -126,27 +184,30 @@ int precond_apply(vxl_precond* pc, int nrhs, const void* r, void* z, hipStream_t
 // are skipped.
 template <typename T>
 int precond_apply_cg(vxl_precond* pc, int nrhs, const T* r, T* p, double* rz_partial, const double* beta,
-                     const std::function<int()>& mid, const int* active, hipStream_t s);
+                     const std::function<int()>& mid, const int* active, hipStream_t s,
+                     const BetaFold* fold = nullptr);
 int precond_rz_blocks(const vxl_precond* pc);
 // The two halves of precond_apply_cg, for a caller that acts between them.
 // Forward x pass of r; with q != nullptr it first applies r -= alpha q (and
 // x += alpha p when x != nullptr) to every entry it loads and writes FP64
-// ||r||^2 partials (rr_partial[rhs * precond_fused_update_blocks + b]); that
-// form needs the four-step x pass (precond_fused_update_blocks > 0).
+// ||r||^2 partials (rr_partial[rhs * precond_fused_update_blocks + b]).  fold
+// (optional): alpha is formed inside the pass from the p . q partials.
 // sr (spectral residual, precond_residual_spectrum first): the residual is
 // kept as its x spectrum R^ inside the preconditioner.  Without q the pass
 // forms R^ from r; with q it updates R^ -= alpha q^ and writes the ||r||^2
 // partials (Parseval), r is not read and x, p must be null.
 template <typename T>
 int precond_cg_forward(vxl_precond* pc, int nrhs, T* r, T* x, const T* p, const T* q, const double* alpha,
-                       double* rr_partial, const int* active, hipStream_t s, bool sr = false);
+                       double* rr_partial, const int* active, hipStream_t s, bool sr = false,
+                       const AlphaFold* fold = nullptr);
 // y, z (+ Green, r.z), mid(), y^-1 and the x inverse pass writing
 // p = z + beta p_old (p_old == nullptr: p itself, in place).  sr: the y pass
-// reads R^.
+// reads R^.  fold (optional): beta is formed inside the x pass from the r . z
+// partials, and mid() is not called.
 template <typename T>
 int precond_cg_rest(vxl_precond* pc, int nrhs, T* p, double* rz_partial, const double* beta,
                     const std::function<int()>& mid, const int* active, hipStream_t s, const T* p_old = nullptr,
-                    bool sr = false);
+                    bool sr = false, const BetaFold* fold = nullptr);
 // Whether the spectral-residual form is available (FP32 spectrum storage,
 // four-step x and y passes; VXL_SPECTRAL_RESIDUAL=0 turns it off), and the
 // allocation of its R^ buffer (nrhs_max spectra; once, outside any capture).
@@ -187,6 +248,7 @@ struct vxl_solver {
   int nblk;
   int* active_dev;
   int* restart_dev;
+  int rho_slot;  // slot of the current r . z
   int* stop_dev;
   double* macro_dev;
   double* rhs_sig;  // per-row element stresses of the RHS (nullptr: direct form)

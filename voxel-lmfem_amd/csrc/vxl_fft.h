@@ -314,7 +314,18 @@ struct XUpdate {
   const T* q;
   const double* alpha;
   double* partial;
+  AlphaFold fold;
 };
+// alpha of right-hand side k for the update forms.
+template <typename T>
+__device__ __forceinline__ double update_alpha(const XUpdate<T>& u, int k, bool first, double* red) {
+  return u.fold.partial ? fold_alpha(u.fold, k, first, red) : u.alpha[k];
+}
+// An inactive system takes no step.
+template <typename T>
+__device__ __forceinline__ void update_skipped(const XUpdate<T>& u, int k, bool first) {
+  if (u.fold.partial && u.fold.hist && first && threadIdx.x == 0) u.fold.hist[k] = 0.0;
+}
 
 
 // ---- general passes (vxl_fftgen.h) ------------------------------------------------
@@ -363,7 +374,7 @@ int launch_gen_r2c(const GenX<T>& g, int nrhs, const T* r, typename CT<T>::type*
                    hipStream_t s);
 template <typename T>
 int launch_gen_c2r(const GenX<T>& g, int nrhs, const typename CT<T>::type* S, T* z, const double* beta, const T* pin,
-                   hipStream_t s);
+                   const BetaFold& fold, hipStream_t s);
 template <typename T>
 int launch_gen_y(const AxisPlan& plan, const GenShape& sh, const typename CT<T>::type* w, bool inverse, int nrhs,
                  typename CT<T>::type* S, const typename CT<T>::type* src, int nz, int W, int64_t stride,

@@ -488,7 +488,10 @@ gen_r2c(const T* f, typename CT<T>::type* __restrict__ S, GenAxis<T> ax, int PB,
   extern __shared__ double2 smem_raw[];
   __shared__ double red[kGenThreads<T> / 64];
   const int rhs = blockIdx.y;
-  if (active && !active[rhs]) return;
+  if (active && !active[rhs]) {
+    if constexpr (MODE != kGenPlain) update_skipped(upd, rhs, blockIdx.x == 0);
+    return;
+  }
   const int n = ax.n, nxh = n / 2 + 1, NP = 3 * PB, ps = NP | 1;
   C* L = reinterpret_cast<C*>(smem_raw);
   C* F = ax.dense ? L + n * ps : L;  // spectrum after step 2
@@ -499,7 +502,8 @@ gen_r2c(const T* f, typename CT<T>::type* __restrict__ S, GenAxis<T> ax, int PB,
   const int have = int(min(int64_t(2 * PB), rows_total - row0));  // rows of this workgroup
   const int64_t plane = rows_total * n;
   const int64_t base = int64_t(rhs) * field_stride + row0 * n;
-  const T alpha = MODE != kGenPlain ? T(upd.alpha[rhs]) : T(0);
+  T alpha = T(0);
+  if constexpr (MODE != kGenPlain) alpha = T(update_alpha(upd, rhs, blockIdx.x == 0, red));
   double acc = 0.0;
   fill_slots(slot, ax);
   {
@@ -616,9 +620,11 @@ gen_r2c(const T* f, typename CT<T>::type* __restrict__ S, GenAxis<T> ax, int PB,
 template <typename T, bool kDir, int SUB>
 __global__ void __launch_bounds__(kGenThreads<T>, kGenWaves<T>)
 gen_c2r(const typename CT<T>::type* __restrict__ S, T* z, GenAxis<T> ax, int PB, int64_t rows_total,
-        int64_t field_stride, int64_t spec_stride, const int* active, const double* beta, const T* pin) {
+        int64_t field_stride, int64_t spec_stride, const int* active, const double* beta, const T* pin,
+        BetaFold fold) {
   using C = typename CT<T>::type;
   extern __shared__ double2 smem_raw[];
+  __shared__ double red[kGenThreads<T> / 64];
   const int rhs = blockIdx.y;
   if (active && !active[rhs]) return;
   const int n = ax.n, nxh = n / 2 + 1, NP = 3 * PB, ps = NP | 1;
@@ -689,7 +695,8 @@ gen_c2r(const typename CT<T>::type* __restrict__ S, T* z, GenAxis<T> ax, int PB,
     });
   __syncthreads();
   const int64_t base = int64_t(rhs) * field_stride + row0 * n;
-  const T b = kDir ? T(beta[rhs]) : T(0);
+  T b = T(0);
+  if constexpr (kDir) b = T(fold.partial ? fold_beta(fold, rhs, blockIdx.x == 0, red) : beta[rhs]);
   const bool keep = kDir && b != T(0);
   const T* prev = pin ? pin : z;
   constexpr int U = 4;
@@ -901,7 +908,7 @@ int launch_gen_r2c(const GenX<T>& g, int nrhs, const T* r, typename CT<T>::type*
 
 template <typename T>
 int launch_gen_c2r(const GenX<T>& g, int nrhs, const typename CT<T>::type* S, T* z, const double* beta, const T* pin,
-                   hipStream_t s) {
+                   const BetaFold& fold, hipStream_t s) {
   const int PB = g.shape.units;
   const int64_t pairs = (g.rows + 1) / 2;
   const dim3 grid(unsigned((pairs + PB - 1) / PB), unsigned(nrhs)), block(unsigned(g.shape.P * g.shape.rows));
@@ -909,7 +916,7 @@ int launch_gen_c2r(const GenX<T>& g, int nrhs, const typename CT<T>::type* S, T*
   const int sub = sub_of(g.plan, g.shape);
 #define VXL_G(DIR, WV)                                                                                            \
   hipLaunchKernelGGL((gen_c2r<T, DIR, WV>), grid, block, g.shape.lds, s, S, z, ax, PB, g.rows, g.field_stride,     \
-                     g.spec_stride, g.active, beta, pin)
+                     g.spec_stride, g.active, beta, pin, fold)
   if (beta) {
     VXL_GS(true);
   } else {
@@ -971,7 +978,8 @@ int launch_gen_z(const AxisPlan& plan, const GenShape& sh, const Tables<T>& tb, 
   template GenShape gen_shape_x<T>(const AxisPlan&, int);                                                             \
   template int upload_dense_table<T>(AxisPlan&);                                                                      \
   template int launch_gen_r2c<T>(const GenX<T>&, int, const T*, CT<T>::type*, const XUpdate<T>*, bool, hipStream_t);   \
-  template int launch_gen_c2r<T>(const GenX<T>&, int, const CT<T>::type*, T*, const double*, const T*, hipStream_t);   \
+  template int launch_gen_c2r<T>(const GenX<T>&, int, const CT<T>::type*, T*, const double*, const T*,                   \
+                                 const BetaFold&, hipStream_t);                                                     \
   template int launch_gen_y<T>(const AxisPlan&, const GenShape&, const CT<T>::type*, bool, int, CT<T>::type*,         \
                                const CT<T>::type*, int, int, int64_t, const int*, hipStream_t);                       \
   template int launch_gen_z<T>(const AxisPlan&, const GenShape&, const Tables<T>&, int, CT<T>::type*, int, int, T, T,  \

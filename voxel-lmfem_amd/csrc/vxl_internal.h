@@ -117,6 +117,19 @@ __device__ __forceinline__ double block_reduce_dyn(double v, double* red) {
   return s;
 }
 
+// Sum of p[0 .. n) over the workgroup, valid in every thread (fixed order;
+// red as for block_reduce_dyn).
+__device__ __forceinline__ double block_total_dyn(const double* p, int n, double* red) {
+  double acc = 0;
+  for (int b = threadIdx.x; b < n; b += blockDim.x) acc += p[b];
+  acc = block_reduce_dyn(acc, red);
+  if (threadIdx.x == 0) red[0] = acc;
+  __syncthreads();
+  acc = red[0];
+  __syncthreads();
+  return acc;
+}
+
 struct Grid {
   int nx, ny, nz;
   int64_t n;
