@@ -105,6 +105,29 @@ int vxl_local_rows(int nz, int ny, int nx, int label_bytes, const void* labels_d
                    const double* b_dev, long long stride, double* rows_dev, long long local_base, int* bad_host,
                    void* stream);
 
+/* Host passes over label and orientation arrays (no device work, at most
+ * `workers` threads; labels: C-contiguous integers of 1, 2, 4 or 8 bytes, 8
+ * bytes signed only).  They serve the input checks the reference makes on the
+ * host (src/voxel_lmfem/inputs.py:36-47).
+ * range: smallest and largest label.  mark: present[l - lo] = 1 for every label
+ * l in [lo, lo + span).  pack: out[i] = labels[i] - lo as uint8 (out_bytes 1) or
+ * uint16 (2); the labels must fit.  find_label: flat positions of `label` in
+ * ascending order, *found of them; nothing is written when they exceed
+ * `capacity`.  check_axes: copies the FP64 axis pairs of the listed voxels to
+ * out1/out2 (count x 3) and checks them `piece` voxels at a time; *code is 0,
+ * or what the first failing piece fails: 1 nonfinite, 2 a zero axis, 3
+ * collinear axes. */
+int vxl_host_label_range(const void* labels, int bytes, int is_signed, int64_t count, int workers, long long* lo,
+                         long long* hi);
+int vxl_host_label_mark(const void* labels, int bytes, int is_signed, int64_t count, int workers, long long lo,
+                        int64_t span, uint8_t* present);
+int vxl_host_label_pack(const void* labels, int bytes, int is_signed, int64_t count, int workers, long long lo,
+                        int out_bytes, void* out);
+int vxl_host_find_label(const void* labels, int bytes, int is_signed, int64_t count, int workers, long long label,
+                        int64_t capacity, int64_t* out, int64_t* found);
+int vxl_host_check_axes(const double* axis1, const double* axis2, const int64_t* voxels, int64_t count, int64_t piece,
+                        int workers, double* out1, double* out2, int* code);
+
 /* Cell: grid, voxel size and material field.
  * Replaces the operator construction of the reference's hybrid FI storage:
  *   HybridFIOperator.__init__  src/voxel_lmfem/_core/materials/hybrid_adapter.py:45-68

@@ -332,7 +332,7 @@ finalize_kernel(const double* partial, int nblk, int op, double* scal, int nrhs,
   if (active && !active[k]) {
     if (threadIdx.x == 0) {
       if (hist) hist[k] = 0.0;  // no step for an inactive system
-      if (host_rr) {
+      if (host_rr && op == kOpRR) {
         host_rr[k] = scal[kRR * nrhs + k];
         host_stop[k] = stop[k];
       }
@@ -347,6 +347,7 @@ finalize_kernel(const double* partial, int nblk, int op, double* scal, int nrhs,
   switch (op) {
     case kOpStore:
       S[kTmp * nrhs + k] = acc;
+      if (host_rr) host_rr[k] = acc;
       break;
     case kOpRho:
       S[kRho * nrhs + k] = acc;

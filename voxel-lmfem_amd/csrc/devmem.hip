@@ -30,6 +30,10 @@ std::unordered_map<void*, Block> g_live;
 std::multimap<std::pair<int, size_t>, void*> g_free;
 size_t g_cached = 0;
 
+constexpr size_t kPinnedIdle = 64;
+std::unordered_map<void*, int> g_pinned_live;        // block -> device
+std::unordered_map<int, std::vector<void*>> g_pinned_free;
+
 void release_device(int device) {  // g_mu held
   for (auto it = g_free.begin(); it != g_free.end();) {
     if (it->first.first == device) {
@@ -90,6 +94,40 @@ void dev_free(void* p) {
   g_live.erase(it);
 }
 
+hipError_t pinned_get(void** p) {
+  *p = nullptr;
+  int device = 0;
+  hipError_t e = hipGetDevice(&device);
+  if (e != hipSuccess) return e;
+  std::lock_guard<std::mutex> lock(g_mu);
+  auto& idle = g_pinned_free[device];
+  if (!idle.empty()) {
+    *p = idle.back();
+    idle.pop_back();
+  } else {
+    e = hipHostMalloc(p, kPinnedBlock);
+    if (e != hipSuccess) {
+      *p = nullptr;
+      return e;
+    }
+  }
+  g_pinned_live[*p] = device;
+  return hipSuccess;
+}
+
+void pinned_put(void* p) {
+  if (!p) return;
+  std::lock_guard<std::mutex> lock(g_mu);
+  auto it = g_pinned_live.find(p);
+  if (it == g_pinned_live.end()) return;
+  auto& idle = g_pinned_free[it->second];
+  g_pinned_live.erase(it);
+  if (idle.size() < kPinnedIdle)
+    idle.push_back(p);
+  else
+    (void)hipHostFree(p);
+}
+
 size_t cached_bytes() {
   std::lock_guard<std::mutex> lock(g_mu);
   return g_cached;
@@ -103,6 +141,11 @@ void release_cached() {
     (void)hipSetDevice(kv.first.first);
     (void)hipFree(kv.second);
   }
+  for (auto& kv : g_pinned_free) {
+    (void)hipSetDevice(kv.first);
+    for (void* p : kv.second) (void)hipHostFree(p);
+  }
+  g_pinned_free.clear();
   (void)hipSetDevice(cur);
   g_free.clear();
   g_cached = 0;

@@ -607,6 +607,7 @@ struct PrecondImpl {
   int64_t rows;
   AxisPlan plan[3];  // x, y, z (general passes)
   GenShape shape[3];
+  void* tables;      // one allocation; tw, tab and the plans' coefficients point into it
   void* tw[3];
   void* tab[3];
   void* spec;
@@ -787,9 +788,19 @@ void launch_x4_c2r(int n, dim3 grid, int thr, size_t lds, hipStream_t s, const S
 #undef VXL_X4C
 }
 
+// Twiddles, Green factors and dense coefficients of the three axes, in one
+// allocation filled by one copy.
 template <typename T>
 int upload_tables(PrecondImpl* im, const double h[3]) {
   using C = typename CT<T>::type;
+  std::vector<T> all;
+  size_t at_w[3], at_tab[3], at_coef[3];
+  auto put = [&](const T* v, size_t n) {  // each table on a 64-byte boundary
+    const size_t at = (all.size() + 15) / 16 * 16;
+    all.resize(at);
+    all.insert(all.end(), v, v + n);
+    return at;
+  };
   const int ns[3] = {im->nx, im->ny, im->nz};
   const int counts[3] = {im->nxh, im->ny, im->nz};
   for (int a = 0; a < 3; ++a) {
@@ -799,8 +810,7 @@ int upload_tables(PrecondImpl* im, const double h[3]) {
       const double ang = 2.0 * M_PI * double(k) / double(n);
       w[k] = C{T(std::cos(ang)), T(-std::sin(ang))};
     }
-    VXL_HIP(dev_malloc(&im->tw[a], sizeof(C) * n));
-    VXL_HIP(hipMemcpy(im->tw[a], w.data(), sizeof(C) * n, hipMemcpyHostToDevice));
+    at_w[a] = put(reinterpret_cast<const T*>(w.data()), 2 * size_t(n));
     const int cnt = counts[a];
     std::vector<T> tab(7 * size_t(cnt));
     for (int k = 0; k < cnt; ++k) {
@@ -816,8 +826,17 @@ int upload_tables(PrecondImpl* im, const double h[3]) {
       tab[5 * cnt + k] = T(std::cos(0.5 * th));
       tab[6 * cnt + k] = T(sh);
     }
-    VXL_HIP(dev_malloc(&im->tab[a], sizeof(T) * tab.size()));
-    VXL_HIP(hipMemcpy(im->tab[a], tab.data(), sizeof(T) * tab.size(), hipMemcpyHostToDevice));
+    at_tab[a] = put(tab.data(), tab.size());
+    const std::vector<T> coef = dense_table<T>(im->plan[a]);
+    at_coef[a] = coef.empty() ? SIZE_MAX : put(coef.data(), coef.size());
+  }
+  VXL_HIP(dev_malloc(&im->tables, sizeof(T) * all.size()));
+  VXL_HIP(hipMemcpy(im->tables, all.data(), sizeof(T) * all.size(), hipMemcpyHostToDevice));
+  T* base = static_cast<T*>(im->tables);
+  for (int a = 0; a < 3; ++a) {
+    im->tw[a] = base + at_w[a];
+    im->tab[a] = base + at_tab[a];
+    im->plan[a].coef = at_coef[a] == SIZE_MAX ? nullptr : base + at_coef[a];
   }
   return VXL_OK;
 }
@@ -905,7 +924,6 @@ int create_impl(vxl_precond* pc, PrecondImpl* im) {
     }
     im->shape[a] = a == 0 ? gen_shape_x<T>(p, env_int("VXL_FFT_XPAIRS")) : a == 1 ? gen_shape_y<T>(p) : gen_shape_z<T>(p);
     if (im->shape[a].lds > kMaxLdsGen) return fail("grid axis too long for the LDS pencil FFT");
-    VXL_TRY(upload_dense_table<T>(p));
   }
   im->spec_stride = int64_t(im->nz) * im->ny * im->nxh * 3;
   VXL_TRY(upload_tables<T>(im, cell->h));
@@ -1062,6 +1080,7 @@ int apply_impl(vxl_precond* pc, PrecondImpl* im, int nrhs, const T* r, T* z, hip
 
 int precond_create(vxl_precond* pc) {
   auto* im = new PrecondImpl();
+  im->tables = nullptr;
   im->tw[0] = im->tw[1] = im->tw[2] = nullptr;
   im->tab[0] = im->tab[1] = im->tab[2] = nullptr;
   for (auto& p : im->plan) p.coef = nullptr;
@@ -1171,11 +1190,7 @@ void precond_release(vxl_precond* pc) {
   auto* im = static_cast<PrecondImpl*>(pc->impl);
   if (!im) return;
   (void)hipStreamSynchronize(pc->cell->stream);
-  for (int a = 0; a < 3; ++a) {
-    if (im->tw[a]) dev_free(im->tw[a]);
-    if (im->tab[a]) dev_free(im->tab[a]);
-    if (im->plan[a].coef) dev_free(im->plan[a].coef);
-  }
+  if (im->tables) dev_free(im->tables);
   if (im->spec) dev_free(im->spec);
   if (im->rhat) dev_free(im->rhat);
   delete im;

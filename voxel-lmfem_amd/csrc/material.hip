@@ -230,10 +230,12 @@ int label_rows(int nz, int ny, int nx, int label_bytes, const void* labels_dev, 
     }
 #undef VXL_LR
     VXL_HIP(hipGetLastError());
-    VXL_HIP(hipMemcpyAsync(present_host, present, sizeof(int) * span, hipMemcpyDeviceToHost, s));
-    VXL_HIP(hipMemcpyAsync(undefined_host, undefined, sizeof(int), hipMemcpyDeviceToHost, s));
-    VXL_HIP(hipMemcpyAsync(samples_host, samples, sizeof(int) * nsamp, hipMemcpyDeviceToHost, s));
+    std::vector<int> back(size_t(span) + 1 + nsamp);  // present | undefined | samples
+    VXL_HIP(hipMemcpyAsync(back.data(), present, sizeof(int) * back.size(), hipMemcpyDeviceToHost, s));
     VXL_HIP(hipStreamSynchronize(s));
+    std::copy(back.begin(), back.begin() + span, present_host);
+    *undefined_host = back[span];
+    std::copy(back.begin() + span + 1, back.end(), samples_host);
     return VXL_OK;
   };
   rc = body();

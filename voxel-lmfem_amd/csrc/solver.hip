@@ -103,8 +103,8 @@ int free_all(vxl_solver* s) {
   s->block_graph = nullptr;
   if (s->capture_stream) (void)hipStreamDestroy(s->capture_stream);
   s->capture_stream = nullptr;
-  double* bufs[] = {s->f, s->x64, s->r64, s->q64, s->scal, s->partial, s->macro_dev,
-                    s->stress_partial, s->ch_dev, s->partial_st, s->partial_rz, s->rhs_sig, s->partial_fx,
+  double* bufs[] = {s->f, s->x64, s->r64, s->q64, s->partial, s->stress_partial,
+                     s->ch_dev, s->partial_st, s->partial_rz, s->rhs_sig, s->partial_fx,
                     s->dinv64, s->jmean, s->jrz, s->media};
   for (double* b : bufs)
     if (b) dev_free(b);
@@ -128,15 +128,27 @@ int free_all(vxl_solver* s) {
   if (s->blk_keep) dev_free(s->blk_keep);
   s->blk_partial = s->blk_small = nullptr;
   s->blk_keep = nullptr;
-  if (s->active_dev) dev_free(s->active_dev);
-  if (s->restart_dev) dev_free(s->restart_dev);
-  if (s->stop_dev) dev_free(s->stop_dev);
+  if (s->ctl) dev_free(s->ctl);
   if (s->pc_ready) precond_release(&s->pc);
   for (auto& e : s->ev)
     if (e) (void)hipEventDestroy(e);
   if (s->flag_ev) (void)hipEventDestroy(s->flag_ev);
-  if (s->pinned_flags) (void)hipHostFree(s->pinned_flags);
-  if (s->pinned_scal) (void)hipHostFree(s->pinned_scal);
+  pinned_put(s->pinned);
+  return VXL_OK;
+}
+
+// Scalars and latches zero, macro strains, every system active: one copy.
+int upload_control(vxl_solver* s, const double* macro_host, hipStream_t st) {
+  const int R = s->R;
+  VXL_HIP(hipEventSynchronize(s->flag_ev));
+  double* image = static_cast<double*>(s->pinned);
+  std::fill(image, image + kNumSlots * R, 0.0);
+  std::copy(macro_host, macro_host + 6 * R, image + kNumSlots * R);
+  int* flags = reinterpret_cast<int*>(image + (kNumSlots + 6) * R);
+  std::fill(flags, flags + R, 1);
+  std::fill(flags + R, flags + 3 * R, 0);
+  VXL_HIP(hipMemcpyAsync(s->ctl, image, s->ctl_bytes, hipMemcpyHostToDevice, st));
+  VXL_HIP(hipEventRecord(s->flag_ev, st));
   return VXL_OK;
 }
 
@@ -389,19 +401,15 @@ int prepare_block_graph(vxl_solver* s, double tol) {
 // projection only for returned fields; B0 and the zero-mean RHS both
 // annihilate constants), outputs, per-phase times.  Systems that never started
 // (zero RHS) keep x64 = 0.
-template <typename Upload>
 int finish_run(vxl_solver* s, const double* macro_host, double* ch_host, int* iterations, int* restarts,
                double* residuals, double* u_out, const std::vector<int>& its, const std::vector<int>& nrest,
-               const std::vector<double>& res_true, bool converged, Upload&& upload_flags,
-               std::vector<int>& active) {
+               const std::vector<double>& res_true, bool converged) {
   vxl_cell* cell = s->cell;
   hipStream_t st = cell->stream;
   const int R = s->R;
   const int64_t len = s->len;
   const int64_t n = cell->grid.n;
   double* partial = s->partial;
-  std::fill(active.begin(), active.end(), 1);
-  VXL_TRY(upload_flags());
   if (u_out) VXL_TRY(launch_project_zero_mean(s->x64, n, R, partial, nullptr, st));
   // Six unit strains: <sigma_i>(e_k) = <C>_ik - f_i . u_k / |Omega| (f_i = -sum_e
   // V B0^T C_e e_i, the RHS of load i), two streaming passes instead of the
@@ -487,8 +495,7 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
       pin_flags[k] = active[k];
       pin_flags[R + k] = restart[k];
     }
-    VXL_HIP(hipMemcpyAsync(act, pin_flags, sizeof(int) * R, hipMemcpyHostToDevice, st));
-    VXL_HIP(hipMemcpyAsync(s->restart_dev, pin_flags + R, sizeof(int) * R, hipMemcpyHostToDevice, st));
+    VXL_HIP(hipMemcpyAsync(act, pin_flags, sizeof(int) * 2 * R, hipMemcpyHostToDevice, st));  // active, restart
     VXL_HIP(hipEventRecord(s->flag_ev, st));
     return VXL_OK;
   };
@@ -508,11 +515,8 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
   auto any_active = [&]() { return std::any_of(active.begin(), active.end(), [](int a) { return a; }); };
 
   VXL_HIP(hipEventRecord(s->ev[0], st));
-  VXL_HIP(hipMemcpyAsync(s->macro_dev, macro_host, sizeof(double) * 6 * R, hipMemcpyHostToDevice, st));
-  VXL_HIP(hipMemsetAsync(scal, 0, sizeof(double) * kNumSlots * R, st));
-  VXL_HIP(hipMemsetAsync(s->stop_dev, 0, sizeof(int) * R, st));
+  VXL_TRY(upload_control(s, macro_host, st));
   s->rho_slot = kRho;
-  VXL_TRY(upload_flags());
   // f = P0 rhs(E), r = f and ||f||^2 (one pass after the component means)
   VXL_TRY(launch_rhs(cell, R, s->macro_dev, s->f, s->rhs_sig, st));
   int nblk_ff = 0;
@@ -559,7 +563,7 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
     }
   }
   const double* unscale = rscale ? rscale + R : nullptr;
-  VXL_TRY(upload_flags());
+  if (std::count(active.begin(), active.end(), 1) != R) VXL_TRY(upload_flags());
   // p = z = M r with rho = r.z: beta = 0 because rho_old = 0 (slots cleared).
   Steps<T> steps(s, tol, st);
   const bool jacobi = steps.jacobi;
@@ -625,9 +629,10 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
     int rblocks = 0;
     VXL_TRY(launch_residual_apply(cell, R, s->x64, s->f, mixed ? reinterpret_cast<float*>(r) : nullptr,
                                   mixed ? nullptr : s->r64, act, s->partial_cert, &rblocks, rscale, st));
-    VXL_TRY(launch_finalize(s->partial_cert, rblocks, kOpStore, scal, R, act, nullptr, st));
-    std::vector<double> t(R);
-    VXL_TRY(read_slot(kTmp, t));
+    VXL_TRY(launch_finalize(s->partial_cert, rblocks, kOpStore, scal, R, act, nullptr, st, 0, 0.0, nullptr, nullptr,
+                            kRho, kRho, pin_scal));
+    VXL_HIP(hipStreamSynchronize(st));
+    const std::vector<double> t(pin_scal, pin_scal + R);
     for (int k = 0; k < R; ++k) {
       if (!mask[k]) continue;
       const double rel = std::sqrt(t[k] / ff[k]);
@@ -763,7 +768,7 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
   VXL_TRY(flush());
   VXL_HIP(hipEventRecord(s->ev[2], st));
   return finish_run(s, macro_host, ch_host, iterations, restarts, residuals, u_out, its, nrest, res_true,
-                    !any_active(), upload_flags, active);
+                    !any_active());
 }
 
 // ---- block CG over the load cases ---------------------------------------------
@@ -863,8 +868,7 @@ int run_block_impl(vxl_solver* s, const double* macro_host, double tol, int max_
       pin_flags[k] = active[k];
       pin_flags[R + k] = 0;
     }
-    VXL_HIP(hipMemcpyAsync(act, pin_flags, sizeof(int) * R, hipMemcpyHostToDevice, st));
-    VXL_HIP(hipMemcpyAsync(s->restart_dev, pin_flags + R, sizeof(int) * R, hipMemcpyHostToDevice, st));
+    VXL_HIP(hipMemcpyAsync(act, pin_flags, sizeof(int) * 2 * R, hipMemcpyHostToDevice, st));  // active, restart
     VXL_HIP(hipEventRecord(s->flag_ev, st));
     return VXL_OK;
   };
@@ -891,9 +895,7 @@ int run_block_impl(vxl_solver* s, const double* macro_host, double tol, int max_
   };
 
   VXL_HIP(hipEventRecord(s->ev[0], st));
-  VXL_HIP(hipMemcpyAsync(s->macro_dev, macro_host, sizeof(double) * 6 * R, hipMemcpyHostToDevice, st));
-  VXL_HIP(hipMemsetAsync(scal, 0, sizeof(double) * kNumSlots * R, st));
-  VXL_TRY(upload_flags());
+  VXL_TRY(upload_control(s, macro_host, st));
   VXL_TRY(launch_rhs(cell, R, s->macro_dev, s->f, s->rhs_sig, st));
   int nblk_ff = 0;
   VXL_TRY(launch_center_copy<T>(s->f, r, n, R, partial, &nblk_ff, st));
@@ -990,7 +992,7 @@ int run_block_impl(vxl_solver* s, const double* macro_host, double tol, int max_
     // x64 is X itself; nothing to flush.
   }
   return finish_run(s, macro_host, ch_host, iterations, restarts, residuals, u_out, its, nrest, res_true,
-                    !any_active(), upload_flags, active);
+                    !any_active());
 }
 
 }  // namespace
@@ -1045,18 +1047,24 @@ int solver_create(vxl_solver* s) {
     const int st_blocks = apply_cg_blocks_max(cell, R, s->mode == VXL_SOLVE_MIXED ? VXL_F32 : VXL_F64);
     VXL_HIP(dev_malloc(&s->partial_st, sizeof(double) * size_t(st_blocks) * R));
   }
-  VXL_HIP(dev_malloc(&s->scal, sizeof(double) * kNumSlots * R));
-  VXL_HIP(dev_malloc(&s->active_dev, sizeof(int) * R));
-  VXL_HIP(dev_malloc(&s->restart_dev, sizeof(int) * R));
-  VXL_HIP(dev_malloc(&s->macro_dev, sizeof(double) * 6 * R));
+  s->ctl_bytes = sizeof(double) * (kNumSlots + 6) * R + sizeof(int) * 3 * R;
+  VXL_HIP(dev_malloc(&s->ctl, s->ctl_bytes));
+  s->scal = static_cast<double*>(s->ctl);
+  s->macro_dev = s->scal + kNumSlots * R;
+  s->active_dev = reinterpret_cast<int*>(s->macro_dev + 6 * R);
+  s->restart_dev = s->active_dev + R;
+  s->stop_dev = s->restart_dev + R;
   if (const int64_t ns = rhs_scratch_size(cell, R)) VXL_HIP(dev_malloc(&s->rhs_sig, sizeof(double) * size_t(ns)));
   VXL_HIP(dev_malloc(&s->stress_partial, sizeof(double) * size_t(stress_partial_size(cell, R))));
   VXL_HIP(dev_malloc(&s->ch_dev, sizeof(double) * 6 * R));
   for (auto& e : s->ev) VXL_HIP(hipEventCreate(&e));
   VXL_HIP(hipEventCreate(&s->flag_ev));
-  VXL_HIP(hipHostMalloc(reinterpret_cast<void**>(&s->pinned_flags), sizeof(int) * 3 * R));
-  VXL_HIP(dev_malloc(&s->stop_dev, sizeof(int) * R));
-  VXL_HIP(hipHostMalloc(reinterpret_cast<void**>(&s->pinned_scal), sizeof(double) * R));
+  // Pinned block: image of the control block, R scalars, 3 R flags.
+  if (s->ctl_bytes + sizeof(double) * (R + 1) + sizeof(int) * 3 * R > kPinnedBlock)
+    return fail("too many load cases for the pinned control block");
+  VXL_HIP(pinned_get(&s->pinned));
+  s->pinned_scal = static_cast<double*>(s->pinned) + (s->ctl_bytes + 7) / 8;
+  s->pinned_flags = reinterpret_cast<int*>(s->pinned_scal + R);
   s->trace.assign(R, {});
   s->pc.cell = cell;
   s->pc.precision = s->mode == VXL_SOLVE_MIXED ? VXL_F32 : VXL_F64;

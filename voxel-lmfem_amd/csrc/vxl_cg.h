@@ -257,6 +257,13 @@ struct vxl_solver {
   hipEvent_t ev[4];
   double ms[3];
   hipEvent_t flag_ev;
+  // Control block: scalars, macro strains and flags in one device allocation
+  // (scal, macro_dev, active_dev, restart_dev and stop_dev point into it), set
+  // up by one copy from its pinned image; pinned_flags and pinned_scal point
+  // into the same pinned block.
+  void* ctl;
+  size_t ctl_bytes;
+  void* pinned;
   int* pinned_flags;
   double* pinned_scal;
   // Instantiated graph of one block between host checks: the preconditioner

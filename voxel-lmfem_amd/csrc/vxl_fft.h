@@ -342,13 +342,16 @@ struct AxisPlan {
   int n, n1, n2;
   int dense;    // n2 runs as a dense transform
   int hpad;     // dense: outputs 0 .. n2/2 padded to whole output groups
-  void* coef;   // dense: cos and sin of 2 pi j k / n2, device (see upload_dense_table)
+  void* coef;   // dense: cos and sin of 2 pi j k / n2, device (see dense_table)
 };
 template <typename T>
 AxisPlan make_axis_plan(int n);
-// Fills plan.coef (nothing to do unless dense).
+// Padded output count of a dense plan (0 otherwise), and its coefficient table
+// (empty otherwise; needs plan.hpad).
 template <typename T>
-int upload_dense_table(AxisPlan& plan);
+int dense_pad(const AxisPlan& plan);
+template <typename T>
+std::vector<T> dense_table(const AxisPlan& plan);
 
 // Workgroup shape of a general pass: P columns (pencils) x `rows` threads.
 struct GenShape {

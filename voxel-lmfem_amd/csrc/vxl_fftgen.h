@@ -818,6 +818,7 @@ AxisPlan make_axis_plan(int n) {
       p.n2 = b;
     }
   }
+  p.hpad = dense_pad<T>(p);
   return p;
 }
 
@@ -853,15 +854,15 @@ GenShape gen_shape_x(const AxisPlan& plan, int pairs_wanted) {
 }
 
 template <typename T>
-int upload_dense_table(AxisPlan& plan) {
-  plan.coef = nullptr;
-  if (!plan.dense) {
-    plan.hpad = 0;
-    return VXL_OK;
-  }
+int dense_pad(const AxisPlan& plan) {
   constexpr int K = kDenseOut<T>;
+  return plan.dense ? (plan.n2 / 2 + 1 + K - 1) / K * K : 0;
+}
+
+template <typename T>
+std::vector<T> dense_table(const AxisPlan& plan) {
+  if (!plan.dense) return {};
   const int n2 = plan.n2, h = (n2 - 1) / 2;
-  plan.hpad = (n2 / 2 + 1 + K - 1) / K * K;
   std::vector<double> c(n2), s(n2);
   for (int k = 0; k < n2; ++k) {
     const double ang = 2.0 * M_PI * double(k) / double(n2);
@@ -876,9 +877,7 @@ int upload_dense_table(AxisPlan& plan) {
       o[0] = T(c[m]);
       o[1] = T(s[m]);
     }
-  VXL_HIP(dev_malloc(&plan.coef, sizeof(T) * tab.size()));
-  VXL_HIP(hipMemcpy(plan.coef, tab.data(), sizeof(T) * tab.size(), hipMemcpyHostToDevice));
-  return VXL_OK;
+  return tab;
 }
 
 template <typename T>
@@ -976,7 +975,8 @@ int launch_gen_z(const AxisPlan& plan, const GenShape& sh, const Tables<T>& tb, 
   template GenShape gen_shape_y<T>(const AxisPlan&);                                                                  \
   template GenShape gen_shape_z<T>(const AxisPlan&);                                                                  \
   template GenShape gen_shape_x<T>(const AxisPlan&, int);                                                             \
-  template int upload_dense_table<T>(AxisPlan&);                                                                      \
+  template int dense_pad<T>(const AxisPlan&);                                                                         \
+  template std::vector<T> dense_table<T>(const AxisPlan&);                                                            \
   template int launch_gen_r2c<T>(const GenX<T>&, int, const T*, CT<T>::type*, const XUpdate<T>*, bool, hipStream_t);   \
   template int launch_gen_c2r<T>(const GenX<T>&, int, const CT<T>::type*, T*, const double*, const T*,                   \
                                  const BetaFold&, hipStream_t);                                                     \

@@ -100,6 +100,12 @@ hipError_t dev_malloc(T** p, size_t bytes) {
   return dev_malloc(reinterpret_cast<void**>(p), bytes);
 }
 void dev_free(void* p);
+// Pinned host blocks of kPinnedBlock bytes from a pool of at most 64 idle blocks
+// per device (released with the allocation cache); the owner synchronises the
+// streams that use a block before it puts it back.
+constexpr size_t kPinnedBlock = 16384;
+hipError_t pinned_get(void** p);
+void pinned_put(void* p);
 size_t cached_bytes();
 void release_cached();
 

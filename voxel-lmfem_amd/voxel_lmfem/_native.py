@@ -30,6 +30,7 @@ _DP = ctypes.POINTER(ctypes.c_double)
 _IP = ctypes.POINTER(ctypes.c_int)
 
 # name -> (restype, argtypes); mirrors include/vxl.h
+_L = ctypes.c_int64
 SIGNATURES = {
     "vxl_last_error": (ctypes.c_char_p, []),
     "vxl_version": (_I, []),
@@ -57,6 +58,12 @@ SIGNATURES = {
     "vxl_rhs": (_I, [_P, _I, _DP, _P]),
     "vxl_avg_stress": (_I, [_P, _I, _P, _DP, _DP]),
     "vxl_center_fields": (_I, [_P, _I, _P, _DP, _P, _P, _P]),
+    "vxl_host_label_range": (_I, [_P, _I, _I, _L, _I, ctypes.POINTER(ctypes.c_longlong),
+                                  ctypes.POINTER(ctypes.c_longlong)]),
+    "vxl_host_label_mark": (_I, [_P, _I, _I, _L, _I, ctypes.c_longlong, _L, _P]),
+    "vxl_host_label_pack": (_I, [_P, _I, _I, _L, _I, ctypes.c_longlong, _I, _P]),
+    "vxl_host_find_label": (_I, [_P, _I, _I, _L, _I, ctypes.c_longlong, _L, _P, ctypes.POINTER(ctypes.c_int64)]),
+    "vxl_host_check_axes": (_I, [_P, _P, _P, _L, _L, _I, _P, _P, _IP]),
     "vxl_energy_gradient": (_I, [_P, _I, _P, _DP, _DP, _P, _P]),
     "vxl_project_zero_mean": (_I, [_P, _I, _P]),
     "vxl_project_zero_mean_noalloc": (_I, [_P, _I, _P]),
@@ -102,6 +109,20 @@ def load():
         fn.argtypes = args
     _lib = lib
     return lib
+
+
+def host_labels(flat):
+    """(library, pointer, item bytes, signed) for the host passes over a flat
+    label array, or None when they do not take it: no library built, unsigned
+    64-bit, strided or byte-swapped labels."""
+    if (not flat.size or not flat.flags.c_contiguous or not flat.dtype.isnative or flat.dtype.kind not in "iu"
+            or (flat.dtype.kind == "u" and flat.dtype.itemsize == 8)):
+        return None
+    try:
+        lib = load()
+    except (RuntimeError, OSError):
+        return None
+    return lib, ctypes.c_void_p(flat.ctypes.data), flat.dtype.itemsize, int(flat.dtype.kind == "i")
 
 
 def check(rc, what=""):

@@ -4,19 +4,39 @@ Same accepted inputs, checks and ValueError messages as the reference's
 src/voxel_lmfem/inputs.py:16-64; per-voxel frames are validated when the
 material field is built (materials.build_field), still before any GPU work.
 """
+import ctypes
 import json
 from pathlib import Path
 
 import numpy as np
 
+from . import _native
 from . import materials as mat
 
 
 def used_labels(phase):
-    """np.unique(phase) of an integer array: counts over the label range when
-    that range is narrow (pieces counted on a thread pool), a sort otherwise.
-    Same values and dtype."""
+    """np.unique(phase) of an integer array: marks over the label range when
+    that range is narrow (one threaded host pass of the library, two for
+    labels wider than 16 bits; without it counts over pieces on a thread
+    pool), a sort otherwise.  Same values and dtype."""
     flat = phase.reshape(-1)
+    native = _native.host_labels(flat)
+    if native is not None:
+        lib, ptr, size, signed = native
+        workers = mat.host_workers()
+        if size <= 2:
+            lo, span = (-(1 << (8 * size - 1)) if signed else 0), 1 << (8 * size)
+        else:
+            a, b = ctypes.c_longlong(), ctypes.c_longlong()
+            _native.check(lib.vxl_host_label_range(ptr, size, signed, flat.size, workers, ctypes.byref(a),
+                                                   ctypes.byref(b)), "vxl_host_label_range")
+            lo, span = a.value, b.value - a.value + 1
+        if span <= (1 << 22):
+            present = np.zeros(span, dtype=np.uint8)
+            _native.check(lib.vxl_host_label_mark(ptr, size, signed, flat.size, workers, lo, span,
+                                                  present.ctypes.data), "vxl_host_label_mark")
+            return (np.flatnonzero(present) + lo).astype(phase.dtype)
+        return np.unique(flat)
     if flat.size:
         lo, hi = int(flat.min()), int(flat.max())
         if hi - lo < (1 << 22) and hi <= np.iinfo(np.int64).max:

@@ -143,7 +143,17 @@ def map_pieces(fn, length, piece=1 << 20):
 
 
 def voxels_with_label(flat, label):
-    """np.flatnonzero(flat == label), piece by piece on a thread pool."""
+    """np.flatnonzero(flat == label): a threaded host pass of the library, or
+    piece by piece on a thread pool."""
+    from . import _native
+    native = _native.host_labels(flat)
+    if native is not None:
+        import ctypes
+        lib, ptr, size, signed = native
+        out, found = np.empty(flat.size, dtype=np.int64), ctypes.c_int64()
+        _native.check(lib.vxl_host_find_label(ptr, size, signed, flat.size, host_workers(), int(label), out.size,
+                                              out.ctypes.data, ctypes.byref(found)), "vxl_host_find_label")
+        return out[:found.value].astype(np.intp)  # a copy: the pages behind the list were never touched
     parts = map_pieces(lambda a, b: np.flatnonzero(flat[a:b] == label) + a, flat.size)
     return np.concatenate(parts) if parts else np.zeros(0, dtype=np.intp)
 
@@ -222,6 +232,39 @@ def frames(orientation, shape, flat_indices):
     return _matrix_frames(_pick(_as_float(orientation), shape, (3, 3), flat_indices))
 
 
+def _native_axes(sources, shape, selections, chunk, workers, kept):
+    """The axis-pair checks of check_frames for full-grid C-ordered FP64 axes,
+    by the library's threaded host pass (the same expressions in the same
+    order, one read of the axes); fills kept and raises the first failing
+    piece's error.  False when it does not apply."""
+    import ctypes
+    from . import _native
+    full = tuple(shape) + (3,)
+    if any(s.shape != full or s.dtype != np.float64 or not s.flags.c_contiguous for s in sources):
+        return False
+    try:
+        lib = _native.load()
+    except (RuntimeError, OSError):
+        return False
+    start, total = 0, int(np.prod(shape))
+    for sel in selections:
+        if not len(sel):
+            continue
+        idx = np.ascontiguousarray(sel, dtype=np.int64)
+        if idx.min() < 0 or idx.max() >= total:
+            return False
+        part = [k[start:start + len(idx)] for k in kept]
+        code = ctypes.c_int()
+        _native.check(lib.vxl_host_check_axes(sources[0].ctypes.data, sources[1].ctypes.data, idx.ctypes.data,
+                                              len(idx), int(chunk), int(workers), part[0].ctypes.data,
+                                              part[1].ctypes.data, ctypes.byref(code)), "vxl_host_check_axes")
+        if code.value:
+            raise ValueError(("Active local-frame orientations must be finite", "Orientation axes must be nonzero",
+                              "Orientation axes must not be collinear")[code.value - 1])
+        start += len(idx)
+    return True
+
+
 def check_frames(orientation, shape, selections, chunk=65536, workers=None, keep=False):
     """Validate the frames of the selected voxels without building them.
 
@@ -248,6 +291,10 @@ def check_frames(orientation, shape, selections, chunk=65536, workers=None, keep
         return kept
     sources = ((_as_float(orientation["axis1"]), _as_float(orientation["axis2"])) if mapping
                else (_as_float(orientation),))
+    if workers is None:
+        workers = host_workers()
+    if keep and mapping and _native_axes(sources, shape, selections, chunk, workers, kept):
+        return kept
     starts = np.concatenate(([0], np.cumsum([len(p) for p in pieces])))
 
     def one(k):
@@ -260,8 +307,6 @@ def check_frames(orientation, shape, selections, chunk=65536, workers=None, keep
         if keep:
             for out, values in zip(kept, got):
                 out[starts[k]:starts[k + 1]] = values
-    if workers is None:
-        workers = host_workers()
     if workers <= 1 or len(pieces) == 1:
         for k in range(len(pieces)):
             one(k)
