@@ -125,6 +125,7 @@ int cell_create_common(vxl_cell** out, int nz, int ny, int nx, double hx, double
   c->tile_y[0] = default_stencil_tile(VXL_F32);
   c->tile_y[1] = default_stencil_tile(VXL_F64);
   c->zmin[0] = c->zmin[1] = kDefaultChunkPlanes;
+  c->ortho = 0;
   c->element = VXL_ELEMENT_FI;
   c->hg_coef = 0.1;
   c->mfma = 0;
@@ -165,7 +166,7 @@ int cell_create_common(vxl_cell** out, int nz, int ny, int nx, double hx, double
 }
 
 // 21-coefficient FP64 rows -> padded FP64 and FP32 tables; bad[0] = 1 on a
-// nonfinite coefficient.
+// nonfinite coefficient, bad[1] = 1 on a nonzero one outside the orthotropic form.
 __global__ void __launch_bounds__(256)
 pad_rows_kernel(const double* c21, int64_t rows, double* t64, float* t32, int* bad) {
   for (int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x; i < rows * kRowWidth;
@@ -174,6 +175,7 @@ pad_rows_kernel(const double* c21, int64_t rows, double* t64, float* t32, int* b
     const int k = int(i - r * kRowWidth);
     const double v = k < 21 ? c21[r * 21 + k] : 0.0;
     if (!isfinite(v)) bad[0] = 1;
+    if (k < 21 && !ortho_entry(k) && v != 0.0) bad[1] = 1;
     t64[i] = v;
     t32[i] = float(v);
   }
@@ -297,6 +299,9 @@ int vxl_cell_create(vxl_cell** out, int nz, int ny, int nx, double hx, double hy
                               for (int64_t i = 0; i < int64_t(rows) * 21; ++i)
                                 if (!std::isfinite(c21_host[i]))
                                   return fail("coefficient table contains nonfinite values");
+                              c->ortho = 1;
+                              for (int64_t i = 0; i < int64_t(rows) * 21 && c->ortho; ++i)
+                                if (!ortho_entry(int(i % 21)) && c21_host[i] != 0.0) c->ortho = 0;
                               std::vector<double> t64(size_t(rows) * kRowWidth, 0.0);
                               std::vector<float> t32(size_t(rows) * kRowWidth, 0.0f);
                               for (int r = 0; r < rows; ++r)
@@ -319,18 +324,19 @@ int vxl_cell_create_device_rows(vxl_cell** out, int nz, int ny, int nx, double h
                             [&](vxl_cell* c) -> int {
                               if (!c21_dev) return fail("index, coefficient table and rows are required");
                               DevBuf flag(c->stream);
-                              VXL_HIP(dev_malloc(&flag.p, sizeof(int)));
-                              VXL_HIP(hipMemsetAsync(flag.p, 0, sizeof(int), c->stream));
+                              VXL_HIP(dev_malloc(&flag.p, 2 * sizeof(int)));
+                              VXL_HIP(hipMemsetAsync(flag.p, 0, 2 * sizeof(int), c->stream));
                               const int64_t total = int64_t(rows) * kRowWidth;
                               const unsigned blocks = unsigned(std::min<int64_t>((total + 255) / 256, 65536));
                               hipLaunchKernelGGL(pad_rows_kernel, dim3(blocks), dim3(256), 0, c->stream, c21_dev,
                                                  int64_t(rows), static_cast<double*>(c->c64_owned),
                                                  static_cast<float*>(c->c32_owned), static_cast<int*>(flag.p));
                               VXL_HIP(hipGetLastError());
-                              int bad = 0;
-                              VXL_HIP(hipMemcpyAsync(&bad, flag.p, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+                              int bad[2] = {0, 0};
+                              VXL_HIP(hipMemcpyAsync(bad, flag.p, sizeof(bad), hipMemcpyDeviceToHost, c->stream));
                               VXL_HIP(hipStreamSynchronize(c->stream));
-                              if (bad) return fail("coefficient table contains nonfinite values");
+                              c->ortho = !bad[1];
+                              if (bad[0]) return fail("coefficient table contains nonfinite values");
                               return VXL_OK;
                             });
 }

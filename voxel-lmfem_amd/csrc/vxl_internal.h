@@ -41,6 +41,12 @@ __device__ __forceinline__ uint3 xcd_block3() {
   return make_uint3(lin % gx, (lin / gx) % gy, lin / (gx * gy));
 }
 
+// Whether C(i, j) is an entry that an orthotropic medium along the axes has;
+// k = pidx(i, j).
+__host__ __device__ constexpr bool ortho_entry(int k) {
+  return k == 0 || k == 1 || k == 2 || k == 6 || k == 7 || k == 11 || k == 15 || k == 18 || k == 20;
+}
+
 template <typename Idx>
 __device__ __forceinline__ int load_row(const void* index, int64_t v) {
   return int(static_cast<const Idx*>(index)[v]);
@@ -166,6 +172,7 @@ struct vxl_cell {
   int variant[2];  // stencil schedule per precision (VXL_F32, VXL_F64): 1, 2 or 3
   int tile_y[2];   // stencil tile height (output nodes along y; the tile is 32 wide)
   int zmin[2];     // fewest z planes per workgroup chunk (each chunk recomputes one layer)
+  int ortho;       // every row has zeros outside the normal block and the shear diagonal
   int element;     // VXL_ELEMENT_FI (2x2x2 Gauss) or VXL_ELEMENT_C3D8R_HG (one point + hourglass)
   double hg_coef;  // hourglass coefficient of the C3D8R-HG element
   // Matrix-core FP32 stencil (mfma.hip): on when mfma != 0; the dense FP16
