@@ -358,7 +358,7 @@ int launch_residual_apply(const vxl_cell* cell, int nrhs, const double* u, const
 
 int residual_apply_blocks(const vxl_cell* cell, int nrhs) {
   int tx, tiles, chunks, zc;
-  apply_grid<double, 32, kTilesF64[0]>(cell, nrhs, tx, tiles, chunks, zc, kDefaultChunkPlanes);
+  apply_grid<double, ResidTile::tx, ResidTile::ty>(cell, nrhs, tx, tiles, chunks, zc, kDefaultChunkPlanes);
   return tiles * chunks;
 }
 
@@ -382,9 +382,7 @@ bool takes_ortho(const vxl_cell* cell) {
 }
 
 template <typename T>
-constexpr int default_tile_y() {
-  return std::is_same<T, double>::value ? kTilesF64[0] : kTilesF32[0];
-}
+using DefaultTile = TileOption<T, (std::is_same<T, double>::value ? kTilesF64[0] : kTilesF32[0])>;
 
 template <typename T>
 int launch_apply_t(const vxl_cell* cell, int nrhs, const T* u, T* out, hipStream_t s) {
@@ -396,9 +394,12 @@ int launch_apply_t(const vxl_cell* cell, int nrhs, const T* u, T* out, hipStream
       });
   }
   if (cell->element == VXL_ELEMENT_C3D8R_HG)
-    return dispatch_apply<T, 32, default_tile_y<T>(), true>(cell, nrhs, u, out, s);
+    return dispatch_apply<T, DefaultTile<T>::tx, DefaultTile<T>::ty, true>(cell, nrhs, u, out, s);
   if (takes_ortho<T>(cell)) return launch_apply_ortho<T>(cell, nrhs, u, out, s, nullptr, nullptr, nullptr);
-  return with_tile<T>(cell, [&](auto ty) { return dispatch_apply<T, 32, decltype(ty)::value>(cell, nrhs, u, out, s); });
+  return with_tile<T>(cell, [&](auto t) {
+    using O = decltype(t);
+    return dispatch_apply<T, O::tx, O::ty>(cell, nrhs, u, out, s);
+  });
 }
 template <typename T>
 int launch_apply_cg_t(const vxl_cell* cell, int nrhs, const T* p, T* q, const int* active, double* partial,
@@ -411,26 +412,28 @@ int launch_apply_cg_t(const vxl_cell* cell, int nrhs, const T* p, T* q, const in
       });
   }
   if (cell->element == VXL_ELEMENT_C3D8R_HG)
-    return dispatch_apply<T, 32, default_tile_y<T>(), true>(cell, nrhs, p, q, s, active, partial, blocks);
+    return dispatch_apply<T, DefaultTile<T>::tx, DefaultTile<T>::ty, true>(cell, nrhs, p, q, s, active, partial, blocks);
   if (takes_ortho<T>(cell)) return launch_apply_ortho<T>(cell, nrhs, p, q, s, active, partial, blocks);
-  return with_tile<T>(cell, [&](auto ty) {
-    return dispatch_apply<T, 32, decltype(ty)::value>(cell, nrhs, p, q, s, active, partial, blocks);
+  return with_tile<T>(cell, [&](auto t) {
+    using O = decltype(t);
+    return dispatch_apply<T, O::tx, O::ty>(cell, nrhs, p, q, s, active, partial, blocks);
   });
 }
 template <typename T>
-int cg_blocks_t(const vxl_cell* cell, int nrhs, int zmin) {
+int cg_blocks_t(const vxl_cell* cell, int nrhs, bool most) {
   if constexpr (std::is_same<T, float>::value) {
     if (cell->mfma) return mfma_blocks(cell, nrhs);
     if (cell->frame_index)
       return frames_tile(cell, [&](auto ty) {
         int tx, tiles, chunks, zc;
-        apply_grid<T, 32, decltype(ty)::value>(cell, nrhs, tx, tiles, chunks, zc, zmin);
+        apply_grid<T, 32, decltype(ty)::value>(cell, nrhs, tx, tiles, chunks, zc, 0, most);
         return tiles * chunks;
       });
   }
-  return with_tile<T>(cell, [&](auto ty) {
+  return with_tile<T>(cell, [&](auto t) {
+    using O = decltype(t);
     int tx, tiles, chunks, zc;
-    apply_grid<T, 32, decltype(ty)::value>(cell, nrhs, tx, tiles, chunks, zc, zmin);
+    apply_grid<T, O::tx, O::ty>(cell, nrhs, tx, tiles, chunks, zc, 0, most);
     return tiles * chunks;
   });
 }
@@ -492,11 +495,11 @@ int launch_apply_cg<double>(const vxl_cell* cell, int nrhs, const double* p, dou
 }
 template <>
 int apply_cg_blocks<float>(const vxl_cell* cell, int nrhs) {
-  return cg_blocks_t<float>(cell, nrhs, 0);
+  return cg_blocks_t<float>(cell, nrhs, false);
 }
 template <>
 int apply_cg_blocks<double>(const vxl_cell* cell, int nrhs) {
-  return cg_blocks_t<double>(cell, nrhs, 0);
+  return cg_blocks_t<double>(cell, nrhs, false);
 }
 
 // Partial sums the CG form can need for any tile and chunk depth the cell may
@@ -507,7 +510,7 @@ int apply_cg_blocks_max(const vxl_cell* cell, int nrhs, int precision) {
   const bool d = precision == VXL_F64;
   for (int t = 0; t < 3; ++t) {
     probe.tile_y[d ? 1 : 0] = d ? kTilesF64[t] : kTilesF32[t];
-    const int b = d ? cg_blocks_t<double>(&probe, nrhs, kMinChunkPlanes) : cg_blocks_t<float>(&probe, nrhs, kMinChunkPlanes);
+    const int b = d ? cg_blocks_t<double>(&probe, nrhs, true) : cg_blocks_t<float>(&probe, nrhs, true);
     most = std::max(most, b);
   }
   if (!d) {  // the matrix-core form, which the cell may be switched to later

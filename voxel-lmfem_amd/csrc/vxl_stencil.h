@@ -311,6 +311,13 @@ __device__ __forceinline__ BlockId xcd_block() {
 constexpr int kTilesF32[3] = {14, 8, 6};
 constexpr int kTilesF64[3] = {6, 8, 4};
 
+// Nodes of a tile option.
+template <typename T, int OPT>
+struct TileOption {
+  static constexpr int tx = 32, ty = OPT;
+};
+using ResidTile = TileOption<double, kTilesF64[0]>;
+
 template <int TX, int TY>
 struct Tile {
   static constexpr int PX = TX + 2, PY = TY + 2, PLANE = PX * PY;
@@ -897,28 +904,46 @@ G9<T> cast_g(const ModalFactors& f) {
   return g;
 }
 
+// The launch grid: tiles and z chunks.  A chunk of `zchunk` planes marches
+// zchunk + 3 steps (the recomputed layer below and two plane loads that nothing
+// hides); workgroups run in rounds of two per CU, and a last round with at most
+// one per CU is shorter, but not half as long (six loads, default tiles: 2.2 us a
+// step with two, 1.7 with one).  The number of chunks with the least total is
+// taken, of those with at least `zmin` planes (under the default depth of 8 the
+// rule may go down to two).  Six loads, us, chunks as near eight planes as 4096
+// workgroups allow -> this rule: FP32 100 x 90 x 80 74 -> 61, 118 x 94 x 111
+// 123 -> 98, 160^3 346 -> 325, 256^3 1273 -> 1275; FP64 118 x 94 x 111 271 -> 243,
+// 160^3 700 -> 687.  One load: 160^3 FP32 59.6 -> 50.7, FP64 118 -> 110.
+// most: the largest number of chunks any depth setting can give.
 template <typename T, int TX, int TY>
 void apply_grid(const vxl_cell* cell, int nrhs, int& tiles_x, int& tiles, int& chunks, int& zchunk,
-                int zmin = 0) {
+                int zmin = 0, bool most = false) {
   const int nx = cell->grid.nx, ny = cell->grid.ny, nz = cell->grid.nz;
   tiles_x = (nx + TX - 1) / TX;
   const int tiles_y = (ny + TY - 1) / TY;
   tiles = tiles_x * tiles_y;
-  // Enough workgroups to fill 256 CUs several times; chunks of >= zmin
-  // planes (default 8: the recomputed layer per chunk stays <= 1/8).
   if (zmin <= 0) zmin = cell->zmin[std::is_same<T, double>::value ? 1 : 0];
-  // Small grids leave CUs idle at that depth, and a launch then takes as long as
-  // one chunk's march (about 1.8 us a layer): chunks shrink to two planes while
-  // all workgroups still run at once (two per CU).  Six loads, default tiles:
-  // 18 x 25 x 21 FP32 18.2 -> 7.8 us, FP64 17.8 -> 10.0; 32^3 17.1 -> 10.6 and
-  // 16.9 -> 13.9; 40-ish 19.2 -> 15.8; 64^3 and larger keep eight planes.
-  if (zmin == kDefaultChunkPlanes) {
-    const int at_once = std::max(1, 512 / (tiles * nrhs));
-    zmin = std::max(kMinChunkPlanes, std::min(zmin, (nz + at_once - 1) / at_once));
+  if (zmin == kDefaultChunkPlanes) zmin = kMinChunkPlanes;
+  const int64_t columns = int64_t(tiles) * nrhs;
+  const int limit = std::max(1, std::min(nz / kMinChunkPlanes, int((4096 + columns - 1) / columns)));
+  if (most) {
+    chunks = limit;
+    zchunk = (nz + chunks - 1) / chunks;
+    return;
   }
-  chunks = (4096 + tiles * nrhs - 1) / (tiles * nrhs);
-  chunks = std::max(1, std::min(chunks, nz / std::max(1, zmin)));
-  zchunk = (nz + chunks - 1) / chunks;
+  constexpr int kCu = 256;
+  int64_t best = -1;
+  for (int c = 1; c <= limit; ++c) {
+    const int depth = (nz + c - 1) / c;
+    if (c > 1 && depth < zmin) break;
+    const int64_t groups = columns * ((nz + depth - 1) / depth);
+    const int64_t rest = groups % (2 * kCu);
+    const int64_t cost = (depth + 3) * (4 * (groups / (2 * kCu)) + (rest == 0 ? 0 : rest <= kCu ? 3 : 4));
+    if (best < 0 || cost < best) {
+      best = cost;
+      zchunk = depth;
+    }
+  }
   chunks = (nz + zchunk - 1) / zchunk;
 }
 
@@ -992,7 +1017,7 @@ int launch_apply_impl(const vxl_cell* cell, int nrhs, const T* u, T* out, hipStr
 template <typename Idx, bool kScale, bool kOrtho = false>
 int launch_resid_impl(const vxl_cell* cell, int nrhs, const double* u, const double* f, float* r32, double* r64,
                       const int* active, double* partial, int* blocks, const double* rscale, hipStream_t s) {
-  constexpr int TX = 32, TY = kTilesF64[0];
+  constexpr int TX = ResidTile::tx, TY = ResidTile::ty;
   using TL = Tile<TX, TY>;
   ApplyArgs<double> a{};
   set_groups(a, cell, nrhs);
@@ -1049,9 +1074,9 @@ template <typename T, typename F>
 int with_tile_of(int ty, F&& f) {
   constexpr bool d = std::is_same<T, double>::value;
   const auto& list = d ? kTilesF64 : kTilesF32;
-  if (ty == list[0]) return f(std::integral_constant<int, (d ? kTilesF64[0] : kTilesF32[0])>());
-  if (ty == list[1]) return f(std::integral_constant<int, (d ? kTilesF64[1] : kTilesF32[1])>());
-  if (ty == list[2]) return f(std::integral_constant<int, (d ? kTilesF64[2] : kTilesF32[2])>());
+  if (ty == list[0]) return f(TileOption<T, (d ? kTilesF64[0] : kTilesF32[0])>());
+  if (ty == list[1]) return f(TileOption<T, (d ? kTilesF64[1] : kTilesF32[1])>());
+  if (ty == list[2]) return f(TileOption<T, (d ? kTilesF64[2] : kTilesF32[2])>());
   return fail("unsupported stencil tile height");
 }
 
