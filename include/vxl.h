@@ -173,12 +173,12 @@ int vxl_get_stencil_variant(vxl_cell* cell, int precision);
 int vxl_tune_stencil(vxl_cell* cell, int precision, int nrhs, const void* u_dev, void* out_dev, int reps,
                      int* best, double* ms3);
 /* Full stencil configuration per precision: tile height (workgroup tile of
- * 32 x tile_y output nodes; VXL_F32: 14 (default), 8 or 6; VXL_F64: 6
- * (default), 8 or 4), schedule (1-3, as above) and the fewest z planes per
- * workgroup chunk (2..64; each chunk recomputes one element layer, and
- * shallower chunks give small cells more workgroups; the default, 8, leaves
- * the depth to the launch, which may take any from 2).  Every configuration
- * computes the same element sums.  No reference counterpart (see
+ * 32 x tile_y output nodes, 16 x 14 for VXL_F64's 6; VXL_F32: 14 (default),
+ * 8 or 6; VXL_F64: 6 (default), 8 or 4), schedule (1-3, as above) and the
+ * fewest z planes per workgroup chunk (2..64; each chunk recomputes one element
+ * layer, and shallower chunks give small cells more workgroups; the default, 8,
+ * leaves the depth to the launch, which may take any from 2).  Every
+ * configuration computes the same element sums.  No reference counterpart (see
  * vxl_tune_stencil). */
 int vxl_set_stencil_config(vxl_cell* cell, int precision, int tile_y, int variant, int zmin);
 /* Element of the cell's operator: VXL_ELEMENT_FI (default; fully integrated

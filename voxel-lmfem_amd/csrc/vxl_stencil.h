@@ -311,10 +311,17 @@ __device__ __forceinline__ BlockId xcd_block() {
 constexpr int kTilesF32[3] = {14, 8, 6};
 constexpr int kTilesF64[3] = {6, 8, 4};
 
-// Nodes of a tile option.
+// Nodes of a tile option.  All are 32 wide and as high as their name but FP64's
+// default, 6, which is 16 x 14: its 17 x 15 elements fill four waves, and it
+// computes 1.14 elements per output node against 1.20 for 32 x 6 (six loads,
+// 64^3 54.9 -> 44.6 us, 100 x 90 x 80 141 -> 121, 118 x 94 x 111 243 -> 218, 192 x
+// 160 x 144 815 -> 719, 256^3 2835 -> 2682; 32^3, where 32 fits, 13.3 -> 14.0).
+// FP32 gains nothing from 16 x 14 (160^3 347 -> 344 us, 256^3
+// 1289 -> 1334).
 template <typename T, int OPT>
 struct TileOption {
-  static constexpr int tx = 32, ty = OPT;
+  static constexpr bool kSquare = std::is_same<T, double>::value && OPT == kTilesF64[0];
+  static constexpr int tx = kSquare ? 16 : 32, ty = kSquare ? 14 : OPT;
 };
 using ResidTile = TileOption<double, kTilesF64[0]>;
 
