@@ -459,7 +459,7 @@ int with_tile(const vxl_cell* cell, F&& f) {
 
 // The orthotropic form serves the FI element without a scale field (schedule
 // 3, the default; the other schedules keep the general form).  Six loads:
-// 160^3 FP32 344 -> 323 us, FP64 705 -> 645 us a launch; the sums are the same bits
+// 160^3 FP32 325 -> 307 us, FP64 676 -> 624 us a launch; the sums are the same bits
 // (only products with exact zeros are left out).
 template <typename T>
 bool takes_ortho(const vxl_cell* cell) {
