@@ -31,6 +31,7 @@
 #include <cmath>
 
 #include "vxl_fft.h"
+#include "vxl_zlanes.h"
 
 namespace vxl {
 namespace {
@@ -341,7 +342,7 @@ struct GreenLane {
 // kx = 0 and kx = nyq, 2 elsewhere, at partial[rhs * gridDim.x + block].
 template <typename T, bool kDot, int SUB>
 __global__ void __launch_bounds__(kGenThreads<T>, kGenWaves<T>)
-gen_z(typename CT<T>::type* S, GenAxis<T> ax, int units, int ny, int nxh, Tables<T> tb, T lam, T mu, T inv_vn,
+gen_z(typename CT<T>::type* S, GenAxis<T> ax, int ny, int nxh, Tables<T> tb, T lam, T mu, T inv_vn,
       int64_t spec_stride, const int* active, int nyq, double* partial, const double* media, int group_rhs) {
   using C = typename CT<T>::type;
   extern __shared__ double2 smem_raw[];
@@ -357,19 +358,18 @@ gen_z(typename CT<T>::type* S, GenAxis<T> ax, int units, int ny, int nxh, Tables
   const int n1 = ax.n1, n2 = ax.n2, W = 3 * nxh, cols = ny * W;
   C* L = reinterpret_cast<C*>(smem_raw);
   C* L2 = L + ax.n * P;  // dense only
-  const int r = P >= 16 ? p & 15 : p, used = P >= 16 ? 15 : P >= 8 ? 6 : 3;
-  const int col = int(bk.x) * units + (p >> 4) * 15 + r;
-  const bool live = r < used && col < cols;
-  const int cc = min(col, cols - 1);
+  const ZLane lane = z_lane(P, p, int(bk.x), cols);
+  const bool live = lane.live;
+  const int cc = lane.col;
   const int ky = cc / W, kx = (cc - ky * W) / 3;
   GreenLane<T> G;
-  G.c = r % 3;
+  G.c = lane.comp;
   G.hg = tb.hg0 > T(0);
   G.hg0 = tb.hg0;
   G.lam = lam;
   G.mu = mu;
   G.init(tb, nxh, ny, kx, ky, inv_vn);
-  const double wk = !live ? 0.0 : (kx == 0 || kx == nyq) ? 1.0 : 2.0;
+  const double wk = (kx == 0 || kx == nyq) ? 1.0 : 2.0;
   C* base = S + int64_t(bk.y) * spec_stride + cc;
   const int64_t zs = int64_t(cols);
   const CPtr<T> gz = cptr<T>(tb.gz);
@@ -438,7 +438,7 @@ gen_z(typename CT<T>::type* S, GenAxis<T> ax, int units, int ny, int nxh, Tables
     });
   });
   if constexpr (kDot) {
-    const double total = block_reduce_dyn(wk * dot, red);
+    const double total = block_reduce_dyn(live ? wk * dot : 0.0, red);
     if (threadIdx.x == 0) partial[int64_t(bk.y) * gridDim.x + bk.x] = total;
   }
 }
@@ -836,7 +836,7 @@ GenShape gen_shape_z(const AxisPlan& plan) {
   GenShape s = pick_shape<T>(plan, 64, [](const AxisPlan& p, int P) {
     return sizeof(typename CT<T>::type) * size_t(p.n) * P * (p.dense ? 2 : 1);
   });
-  s.units = s.P >= 16 ? s.P / 16 * 15 : s.P >= 8 ? 6 : 3;
+  s.units = z_units(s.P);
   return s;
 }
 
@@ -957,8 +957,8 @@ int launch_gen_z(const AxisPlan& plan, const GenShape& sh, const Tables<T>& tb, 
   const GenAxis<T> ax = axis_view<T>(plan, sh, tb.wz);
   const int sub = sub_of(plan, sh);
 #define VXL_G(DOT, WV)                                                                                        \
-  hipLaunchKernelGGL((gen_z<T, DOT, WV>), grid, block, sh.lds, s, S, ax, sh.units, ny, nxh, tb, lam, mu, inv_vn, \
-                     stride, active, nyq, partial, media, group_rhs)
+  hipLaunchKernelGGL((gen_z<T, DOT, WV>), grid, block, sh.lds, s, S, ax, ny, nxh, tb, lam, mu, inv_vn, stride, \
+                     active, nyq, partial, media, group_rhs)
   if (partial) {
     VXL_GS(true);
   } else {
