@@ -59,3 +59,14 @@ def test_ragged_grids(torch_gpu, shape):
                                                  ((682, 2, 2), "float64", 1e-10), ((2, 2048, 2), "float64", 1e-10)])
 def test_longest_axes(torch_gpu, shape, precision, tol):
     _check(torch_gpu, shape, np.array([1.0, 1.0, 1.0]), 1, ((precision, tol),))
+
+
+# Lengths whose factors are all small but no in-register pair: three steps (FP64, or both precisions), with 64, 32, 16
+# and fewer columns a workgroup, odd row counts and every middle factor; the last ones lie past 682 in FP64.
+@pytest.mark.parametrize("n", [27, 44, 63, 99, 147, 175, 189, 200, 216, 243, 250, 264, 270, 288, 336, 375, 392, 448, 486,
+                               500, 539, 605, 625, 675, 700, 720, 729, 1000, 1014, 1280, 1331])
+def test_three_step_lengths(torch_gpu, n):
+    h = np.array([0.7, 1.1, 0.9])
+    tols = (("float64", 1e-11), ("float32", 5e-6)) if n <= 512 else (("float64", 1e-10), ("float32", 2e-5))
+    for shape in ((3, 5, n), (3, n, 5), (n, 5, 3)):
+        _check(torch_gpu, shape, h, 2, tols)

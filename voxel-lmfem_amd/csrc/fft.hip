@@ -876,7 +876,7 @@ int create_impl(vxl_precond* pc, PrecondImpl* im) {
   im->nxh = im->nx / 2 + 1;
   im->rows = int64_t(im->ny) * im->nz;
   const int axis[3] = {im->nx, im->ny, im->nz};
-  for (int a = 0; a < 3; ++a) im->plan[a] = make_axis_plan<T>(axis[a]);
+  for (int a = 0; a < 3; ++a) im->plan[a] = make_axis_plan<T>(axis[a], a == 2);
   {
     const int ly = four_step_lanes(im->ny), lz = four_step_lanes(im->nz);
     const char* env = std::getenv("VXL_FFT_FOURSTEP");

@@ -336,16 +336,17 @@ __device__ __forceinline__ void update_skipped(const XUpdate<T>& u, int k, bool 
 
 // ---- general passes (vxl_fftgen.h) ------------------------------------------------
 // An axis of n = n1 * n2: n1 is transformed in registers; n2 in registers too,
-// or, when it is no in-register size (a prime factor above 13, or a product
-// too large), as a dense transform out of LDS.
+// or in two such steps of na and nb, or, when it has no in-register factors (a
+// prime factor above 13), as a dense transform out of LDS.
 struct AxisPlan {
   int n, n1, n2;
+  int na, nb;   // three-step: n2 = na * nb; otherwise 0
   int dense;    // n2 runs as a dense transform
   int hpad;     // dense: outputs 0 .. n2/2 padded to whole output groups
   void* coef;   // dense: cos and sin of 2 pi j k / n2, device (see dense_table)
 };
 template <typename T>
-AxisPlan make_axis_plan(int n);
+AxisPlan make_axis_plan(int n, bool z);  // z: for the z pass
 // Padded output count of a dense plan (0 otherwise), and its coefficient table
 // (empty otherwise; needs plan.hpad).
 template <typename T>

@@ -18,7 +18,8 @@
 // factor above 13, or a product too large) is a dense transform out of LDS:
 // the row is folded to a_j = x_j + x_{n2-j}, b_j = x_j - x_{n2-j}, and a thread
 // forms kDenseOut output pairs X_k, X_{n2-k} from the cos and sin sums, n2 - 1
-// multiply-adds per output.
+// multiply-adds per output.  Where n2 = na * nb has in-register factors, step 2
+// is instead two steps of its own (kThree, gen_mid and gen_step3), in place.
 //
 // Measured, FP32, six loads, against mixed-radix Stockham passes with runtime
 // strides (and a direct DFT for prime factors above 13): 111 x 94 x 118 (3 * 37,
@@ -46,6 +47,8 @@ constexpr bool in_register(int n) {
 }
 template <typename T>
 constexpr int kDenseOut = sizeof(T) == 4 ? 8 : 4;  // dense output pairs per thread
+constexpr int kMidMost = 13;  // largest middle factor of a three-step axis; its other factors:
+constexpr bool three_step(int n) { return (n >= 1 && n <= 16) || n == 25; }
 constexpr size_t kGenLds = 81408;  // dynamic LDS of a workgroup when two share a CU's 160 KB
 
 // Read-only table in the constant address space: uniform indices become
@@ -65,6 +68,7 @@ __device__ __forceinline__ C cload(CPtr<T> p, int i) {
 template <typename T>
 struct GenAxis {
   int n, n1, n2, dense, hpad;
+  int na, nb;  // three-step: n2 = na * nb
   int lp;  // log2 of the column count
   const void* w;
   const void* coef;
@@ -107,12 +111,23 @@ __device__ __forceinline__ C twiddle_at(CPtr<T> w, int j, int tb, int half) {
   return a;
 }
 
-template <typename T, typename F>
+// Rows of two neighbouring twiddle entries i0 (base row) and i1 (the row after it).
+template <int SUB, typename C, typename T>
+__device__ __forceinline__ C twiddle_pair(CPtr<T> w, int i0, int i1, int half) {
+  C a = cload<C, T>(w, i0);
+  if constexpr (SUB == 2) {
+    const C b = cload<C, T>(w, i1);
+    a = C{half ? b.x : a.x, half ? b.y : a.y};
+  }
+  return a;
+}
+
+template <typename T, bool kThree = false, int MOST = 25, typename F>
 __device__ __forceinline__ void with_radix(int r, F&& f) {
   switch (r) {
 #define VXL_R(R) \
   case R:        \
-    if constexpr (in_register<T>(R)) f(std::integral_constant<int, R>()); \
+    if constexpr (R <= MOST && (kThree ? three_step(R) : in_register<T>(R))) f(std::integral_constant<int, R>()); \
     break;
     VXL_R(1) VXL_R(2) VXL_R(3) VXL_R(4) VXL_R(5) VXL_R(6) VXL_R(7) VXL_R(8) VXL_R(9) VXL_R(10) VXL_R(11) VXL_R(12)
     VXL_R(13) VXL_R(14) VXL_R(15) VXL_R(16) VXL_R(18) VXL_R(20) VXL_R(25)
@@ -122,11 +137,11 @@ __device__ __forceinline__ void with_radix(int r, F&& f) {
 
 // Step 1 over this thread's rows: load(entry), twiddled outputs to L
 // (row stride ps, column p).
-template <bool INV, int SUB, typename T, typename C, typename Load>
+template <bool INV, int SUB, bool kThree, typename T, typename C, typename Load>
 __device__ __forceinline__ void gen_step1(C* L, int ps, int p, const RowSet<SUB>& rs, const GenAxis<T>& ax, Load load) {
   const CPtr<T> w = cptr<T>(ax.w);
   const int n2 = ax.n2;
-  with_radix<T>(ax.n1, [&](auto rc) {
+  with_radix<T, kThree>(ax.n1, [&](auto rc) {
     constexpr int R = decltype(rc)::value;
     rs.each(n2, [&](int tb, int t) {
       C v[R];
@@ -222,10 +237,85 @@ __device__ __forceinline__ void gen_step2(const C* L, int ps, int p, const RowSe
   });
 }
 
+// The two steps of a three-step axis that replace step 2: with n2 = na nb, row
+// (t, s) of the middle step takes the entries t n2 + s + nb k (s < nb), row (t, s)
+// of the last one t n2 + s nb + k (s < na), whose outputs are X[t + n1 (s + na j)].
+// Both write the entries they read.  back: the middle step of the transform run
+// backwards (z pass), DFT_na^-1 and then the twiddle that step 1 multiplied by.
+template <bool INV, bool BACK, int SUB, typename T, typename C>
+__device__ __forceinline__ void gen_mid(C* L, int ps, int p, const RowSet<SUB>& rs, const GenAxis<T>& ax) {
+  const CPtr<T> w = cptr<T>(ax.w);
+  const int n1 = ax.n1, n2 = ax.n2, nb = ax.nb;
+  with_radix<T, true, kMidMost>(ax.na, [&](auto rc) {
+    constexpr int R = decltype(rc)::value;
+    rs.each(n1 * nb, [&](int rb, int r) {
+      const int t0 = rb / nb, s0 = rb - t0 * nb;
+      // Twiddle entry of output j: first + j step.
+      const int f0 = BACK ? t0 * s0 : 0, d0 = BACK ? t0 * nb : n1 * s0;
+      int f1 = f0, d1 = d0, at = t0 * n2 + s0;
+      if constexpr (SUB == 2) {
+        const bool wrap = s0 + 1 == nb;
+        const int t1 = wrap ? t0 + 1 : t0, s1 = wrap ? 0 : s0 + 1;
+        f1 = BACK ? t1 * s1 : 0;
+        d1 = BACK ? t1 * nb : n1 * s1;
+        at = rs.half ? t1 * n2 + s1 : at;
+      }
+      C* x = L + at * ps + p;
+      const int stride = nb * ps;
+      C v[R];
+#pragma unroll
+      for (int k = 0; k < R; ++k) v[k] = x[k * stride];
+      dft_reg<R, INV, T>(v);
+#pragma unroll
+      for (int j = 0; j < R; ++j) {
+        if (BACK || j > 0) {
+          C tw = twiddle_pair<SUB, C, T>(w, f0 + j * d0, f1 + j * d1, rs.half);
+          if (INV) tw = cconj(tw);
+          v[j] = cmul(v[j], tw);
+        }
+        x[j * stride] = v[j];
+      }
+    });
+  });
+}
+// Row (t, s) of the last step, first entry `at`: f(radix, base t, base s, t, s, at).
+template <int SUB, typename T, typename F>
+__device__ __forceinline__ void each_last(const RowSet<SUB>& rs, const GenAxis<T>& ax, F&& f) {
+  const int na = ax.na, n2 = ax.n2, nb = ax.nb;
+  with_radix<T, true>(nb, [&](auto rc) {
+    rs.each(ax.n1 * na, [&](int rb, int r) {
+      const int t0 = rb / na, s0 = rb - t0 * na;
+      int t1 = t0, s1 = s0;
+      if constexpr (SUB == 2) {
+        const bool wrap = s0 + 1 == na;
+        t1 = wrap ? t0 + 1 : t0;
+        s1 = wrap ? 0 : s0 + 1;
+      }
+      f(rc, t0, s0, t1, s1, rs.half ? t1 * n2 + s1 * nb : t0 * n2 + s0 * nb);
+    });
+  });
+}
+// out(k, entry, X[k]): output k and the entry of L it was read from.
+template <bool INV, int SUB, typename T, typename C, typename Out>
+__device__ __forceinline__ void gen_step3(const C* L, int ps, int p, const RowSet<SUB>& rs, const GenAxis<T>& ax,
+                                          Out out) {
+  const int n1 = ax.n1, na = ax.na;
+  each_last<SUB, T>(rs, ax, [&](auto rc, int t0, int s0, int t1, int s1, int at) {
+    constexpr int R = decltype(rc)::value;
+    const int k0 = rs.half ? t1 + n1 * s1 : t0 + n1 * s0;
+    C u[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) u[k] = L[(at + k) * ps + p];
+    dft_reg<R, INV, T>(u);
+#pragma unroll
+    for (int j = 0; j < R; ++j) out(k0 + n1 * na * j, at + j, u[j]);
+  });
+}
+
 // ---- y pass -----------------------------------------------------------------------
 // Columns are numbered over all z planes (z W + j), so only the last workgroup
 // of a right-hand side has idle columns.
-template <bool INV, typename T, int SUB>
+template <bool INV, typename T, int SUB, bool kThree>
 __global__ void __launch_bounds__(kGenThreads<T>, kGenWaves<T>)
 gen_y(typename CT<T>::type* S, const typename CT<T>::type* src, GenAxis<T> ax, int cols, int W, int64_t spec_stride,
       const int* active) {
@@ -242,12 +332,20 @@ gen_y(typename CT<T>::type* S, const typename CT<T>::type* src, GenAxis<T> ax, i
   const int z = c / W, j = c - z * W;
   const int64_t off = int64_t(b.y) * spec_stride + int64_t(z) * ax.n * W + j;
   const C* in = src + off;
-  gen_step1<INV, SUB, T>(L, P, p, rs, ax, [&](int e) -> C { return in[e * W]; });
+  gen_step1<INV, SUB, kThree, T>(L, P, p, rs, ax, [&](int e) -> C { return in[e * W]; });
   __syncthreads();
   C* o = S + off;
-  gen_step2<INV, SUB, T>(L, P, p, rs, ax, [&](int t, int k, C v) {
-    if (live) o[(t + ax.n1 * k) * W] = v;
-  });
+  if constexpr (kThree) {
+    gen_mid<INV, false, SUB, T>(L, P, p, rs, ax);
+    __syncthreads();
+    gen_step3<INV, SUB, T>(L, P, p, rs, ax, [&](int k, int, C v) {
+      if (live) o[k * W] = v;
+    });
+  } else {
+    gen_step2<INV, SUB, T>(L, P, p, rs, ax, [&](int t, int k, C v) {
+      if (live) o[(t + ax.n1 * k) * W] = v;
+    });
+  }
 }
 
 // ---- z pass with the Green solve -----------------------------------------------------
@@ -340,7 +438,7 @@ struct GreenLane {
 
 // partial (optional): FP64 r . z of the workgroup by Parseval, weight 1 at
 // kx = 0 and kx = nyq, 2 elsewhere, at partial[rhs * gridDim.x + block].
-template <typename T, bool kDot, int SUB>
+template <typename T, bool kDot, int SUB, bool kThree>
 __global__ void __launch_bounds__(kGenThreads<T>, kGenWaves<T>)
 gen_z(typename CT<T>::type* S, GenAxis<T> ax, int ny, int nxh, Tables<T> tb, T lam, T mu, T inv_vn,
       int64_t spec_stride, const int* active, int nyq, double* partial, const double* media, int group_rhs) {
@@ -379,22 +477,43 @@ gen_z(typename CT<T>::type* S, GenAxis<T> ax, int ny, int nxh, Tables<T> tb, T l
     if (G.hg) return {gz[4 * n + kz], gz[5 * n + kz], gz[6 * n + kz], T(0)};
     return {gz[kz], gz[n + kz], gz[2 * n + kz], gz[3 * n + kz]};
   };
-  auto zfactors = [&](int tb, int k) -> AxisF<T> {  // of entry tb + half + n1 k
-    AxisF<T> f = zload(tb + n1 * k);
+  auto zfactors = [&](int e0, int e1) -> AxisF<T> {  // of entry e0 (base row) or e1 (the row after it)
+    AxisF<T> f = zload(e0);
     if constexpr (SUB == 2) {
-      const AxisF<T> h = zload(min(tb + 1 + n1 * k, ax.n - 1));
+      const AxisF<T> h = zload(min(e1, ax.n - 1));
       f = {rs.half ? h.a : f.a, rs.half ? h.b : f.b, rs.half ? h.c : f.c, rs.half ? h.d : f.d};
     }
     return f;
   };
   double dot = 0.0;
 
-  gen_step1<false, SUB, T>(L, P, p, rs, ax, [&](int e) -> C { return base[e * zs]; });
+  gen_step1<false, SUB, kThree, T>(L, P, p, rs, ax, [&](int e) -> C { return base[e * zs]; });
   __syncthreads();
-  if (ax.dense) {
+  if constexpr (kThree) {
+    gen_mid<false, false, SUB, T>(L, P, p, rs, ax);
+    __syncthreads();
+    each_last<SUB, T>(rs, ax, [&](auto rc, int t0, int s0, int t1, int s1, int at) {
+      constexpr int R = decltype(rc)::value;
+      const int e0 = t0 + n1 * s0, e1 = t1 + n1 * s1, step = n1 * ax.na;
+      C u[R];
+#pragma unroll
+      for (int k = 0; k < R; ++k) u[k] = L[(at + k) * P + p];
+      dft_reg<R, false, T>(u);
+#pragma unroll
+      for (int j = 0; j < R; ++j) dot += G.solve(u[j], zfactors(e0 + step * j, e1 + step * j));
+      dft_reg<R, true, T>(u);
+#pragma unroll
+      for (int m = 0; m < R; ++m) {
+        if (m > 0) u[m] = cmul(u[m], cconj(twiddle_pair<SUB, C, T>(w, n1 * m * s0, n1 * m * s1, rs.half)));
+        L[(at + m) * P + p] = u[m];
+      }
+    });
+    __syncthreads();
+    gen_mid<true, true, SUB, T>(L, P, p, rs, ax);
+  } else if (ax.dense) {
     each_group<T>(rs, ax, [&](int tb, int t, int k0) {
       dense_group<false, T>(L + t * n2 * P + p, P, k0, ax, [&](int k, C v) {
-        dot += G.solve(v, zfactors(tb, k));
+        dot += G.solve(v, zfactors(tb + n1 * k, tb + 1 + n1 * k));
         L2[(t * n2 + k) * P + p] = v;
       });
     });
@@ -413,7 +532,7 @@ gen_z(typename CT<T>::type* S, GenAxis<T> ax, int ny, int nxh, Tables<T> tb, T l
         for (int k = 0; k < R; ++k) u[k] = L[(t * R + k) * P + p];
         dft_reg<R, false, T>(u);
 #pragma unroll
-        for (int k = 0; k < R; ++k) dot += G.solve(u[k], zfactors(tb, k));
+        for (int k = 0; k < R; ++k) dot += G.solve(u[k], zfactors(tb + n1 * k, tb + 1 + n1 * k));
         dft_reg<R, true, T>(u);
 #pragma unroll
         for (int m = 0; m < R; ++m) {
@@ -424,7 +543,7 @@ gen_z(typename CT<T>::type* S, GenAxis<T> ax, int ny, int nxh, Tables<T> tb, T l
     });
   }
   __syncthreads();
-  with_radix<T>(n1, [&](auto rc) {
+  with_radix<T, kThree>(n1, [&](auto rc) {
     constexpr int R = decltype(rc)::value;
     rs.each(n2, [&](int, int m) {
       C v[R];
@@ -473,14 +592,36 @@ struct RowWalk {
 enum GenXMode { kGenPlain = 0, kGenUpd = 1, kGenSpec = 2 };
 
 // The slot of output entry k after step 2: natural order for the dense form
-// (second buffer), otherwise (k % n1) n2 + k / n1 (in place).
-template <typename T>
+// (second buffer), otherwise in place, (k % n1) n2 + q with q = k / n1, or
+// (q % na) nb + q / na in place of q (three-step).
+template <bool kThree, typename T>
 __device__ __forceinline__ void fill_slots(unsigned short* slot, const GenAxis<T>& ax) {
-  for (int k = threadIdx.x; k < ax.n; k += blockDim.x)
-    slot[k] = static_cast<unsigned short>(ax.dense ? k : (k % ax.n1) * ax.n2 + k / ax.n1);
+  for (int k = threadIdx.x; k < ax.n; k += blockDim.x) {
+    const int q = k / ax.n1, t = k - q * ax.n1;
+    slot[k] = static_cast<unsigned short>(kThree     ? t * ax.n2 + (q % ax.na) * ax.nb + q / ax.na
+                                          : ax.dense ? k
+                                                     : t * ax.n2 + q);
+  }
+}
+// Both steps of an x pass on the pencils of L; every output at its slot of F.
+template <bool INV, bool kThree, int SUB, typename T, typename C>
+__device__ __forceinline__ void x_steps(C* L, C* F, int ps, int p, int NP, const RowSet<SUB>& rs,
+                                        const GenAxis<T>& ax) {
+  if (p < NP)
+    gen_step1<INV, SUB, kThree, T>(L, ps, p, rs, ax, [&](int e) -> C { return L[e * ps + p]; });
+  __syncthreads();
+  if constexpr (kThree) {
+    if (p < NP) gen_mid<INV, false, SUB, T>(L, ps, p, rs, ax);
+    __syncthreads();
+    if (p < NP) gen_step3<INV, SUB, T>(L, ps, p, rs, ax, [&](int, int at, C v) { L[at * ps + p] = v; });
+  } else if (p < NP) {
+    gen_step2<INV, SUB, T>(L, ps, p, rs, ax, [&](int t, int k, C v) {
+      F[(ax.dense ? t + ax.n1 * k : t * ax.n2 + k) * ps + p] = v;
+    });
+  }
 }
 
-template <typename T, int MODE, int SUB>
+template <typename T, int MODE, int SUB, bool kThree>
 __global__ void __launch_bounds__(kGenThreads<T>, kGenWaves<T>)
 gen_r2c(const T* f, typename CT<T>::type* __restrict__ S, GenAxis<T> ax, int PB, int64_t rows_total,
         int64_t field_stride, int64_t spec_stride, const int* active, XUpdate<T> upd) {
@@ -505,7 +646,7 @@ gen_r2c(const T* f, typename CT<T>::type* __restrict__ S, GenAxis<T> ax, int PB,
   T alpha = T(0);
   if constexpr (MODE != kGenPlain) alpha = T(update_alpha(upd, rhs, blockIdx.x == 0, red));
   double acc = 0.0;
-  fill_slots(slot, ax);
+  fill_slots<kThree>(slot, ax);
   {
     constexpr int U = MODE == kGenUpd ? 2 : 4;
     RowWalk it(n);
@@ -559,12 +700,7 @@ gen_r2c(const T* f, typename CT<T>::type* __restrict__ S, GenAxis<T> ax, int PB,
     }
   }
   __syncthreads();
-  if (p < NP) gen_step1<false, SUB, T>(L, ps, p, rs, ax, [&](int e) -> C { return L[e * ps + p]; });
-  __syncthreads();
-  if (p < NP)
-    gen_step2<false, SUB, T>(L, ps, p, rs, ax, [&](int t, int k, C v) {
-      F[(ax.dense ? t + ax.n1 * k : t * ax.n2 + k) * ps + p] = v;
-    });
+  x_steps<false, kThree, SUB, T>(L, F, ps, p, NP, rs, ax);
   __syncthreads();
   // Two-for-one split over (pair, k), lanes along k.
   C* out = S + int64_t(rhs) * spec_stride + row0 * nxh * 3;
@@ -617,7 +753,7 @@ gen_r2c(const T* f, typename CT<T>::type* __restrict__ S, GenAxis<T> ax, int PB,
   }
 }
 
-template <typename T, bool kDir, int SUB>
+template <typename T, bool kDir, int SUB, bool kThree>
 __global__ void __launch_bounds__(kGenThreads<T>, kGenWaves<T>)
 gen_c2r(const typename CT<T>::type* __restrict__ S, T* z, GenAxis<T> ax, int PB, int64_t rows_total,
         int64_t field_stride, int64_t spec_stride, const int* active, const double* beta, const T* pin,
@@ -636,7 +772,7 @@ gen_c2r(const typename CT<T>::type* __restrict__ S, T* z, GenAxis<T> ax, int PB,
   const int64_t row0 = 2 * int64_t(blockIdx.x) * PB;
   const int have = int(min(int64_t(2 * PB), rows_total - row0));
   const int64_t plane = rows_total * n;
-  fill_slots(slot, ax);
+  fill_slots<kThree>(slot, ax);
   // Hermitian extension and packing, lanes along k: each stored coefficient is
   // read once and fills entry k and, conjugated, its mirror n - k.
   const C* in = S + int64_t(rhs) * spec_stride + row0 * nxh * 3;
@@ -687,12 +823,7 @@ gen_c2r(const typename CT<T>::type* __restrict__ S, T* z, GenAxis<T> ax, int PB,
     }
   }
   __syncthreads();
-  if (p < NP) gen_step1<true, SUB, T>(L, ps, p, rs, ax, [&](int e) -> C { return L[e * ps + p]; });
-  __syncthreads();
-  if (p < NP)
-    gen_step2<true, SUB, T>(L, ps, p, rs, ax, [&](int t, int k, C v) {
-      F[(ax.dense ? t + ax.n1 * k : t * ax.n2 + k) * ps + p] = v;
-    });
+  x_steps<true, kThree, SUB, T>(L, F, ps, p, NP, rs, ax);
   __syncthreads();
   const int64_t base = int64_t(rhs) * field_stride + row0 * n;
   T b = T(0);
@@ -733,14 +864,21 @@ inline int sub_of(const AxisPlan& p, const GenShape& sh) {
   if (sh.P == 64) return 1;
   return sh.P == 32 && !(p.dense && p.n1 == 1) ? 2 : 0;
 }
-#define VXL_GS(A)   \
-  do {              \
-    if (sub == 1)   \
-      VXL_G(A, 1);  \
-    else if (sub == 2) \
-      VXL_G(A, 2);  \
-    else            \
-      VXL_G(A, 0);  \
+#define VXL_GT(A, K3)     \
+  do {                    \
+    if (sub == 1)         \
+      VXL_G(A, 1, K3);    \
+    else if (sub == 2)    \
+      VXL_G(A, 2, K3);    \
+    else                  \
+      VXL_G(A, 0, K3);    \
+  } while (0)
+#define VXL_GS(A)         \
+  do {                    \
+    if (ax.nb)            \
+      VXL_GT(A, true);    \
+    else                  \
+      VXL_GT(A, false);   \
   } while (0)
 
 template <typename T>
@@ -750,6 +888,8 @@ GenAxis<T> axis_view(const AxisPlan& p, const GenShape& sh, const void* w) {
   a.n1 = p.n1;
   a.n2 = p.n2;
   a.dense = p.dense;
+  a.na = p.na;
+  a.nb = p.nb;
   a.hpad = p.hpad;
   a.lp = 31 - __builtin_clz(unsigned(sh.P));
   a.w = w;
@@ -780,7 +920,11 @@ GenShape pick_shape(const AxisPlan& p, int widest, size_t (*lds)(const AxisPlan&
   int64_t best = INT64_MAX;
   s.rows = step;
   for (int r = step; r <= most; r += step) {
-    const int64_t c = int64_t((p.n2 + r - 1) / r) * 4 * p.n1 + int64_t((work2 + r - 1) / r) * cost2;
+    int64_t c = int64_t((p.n2 + r - 1) / r) * 4 * p.n1;
+    if (p.nb)
+      c += int64_t((p.n1 * p.nb + r - 1) / r) * 4 * p.na + int64_t((p.n1 * p.na + r - 1) / r) * 4 * p.nb;
+    else
+      c += int64_t((work2 + r - 1) / r) * cost2;
     if (c < best) {
       best = c;
       s.rows = r;
@@ -792,10 +936,17 @@ GenShape pick_shape(const AxisPlan& p, int widest, size_t (*lds)(const AxisPlan&
 }  // namespace
 
 // n = n1 * n2 with both factors in-register sizes and the larger one as small
-// as possible; otherwise the largest in-register n1, which leaves the
-// smallest dense n2 (its cost grows with n2).
+// as possible; else n = n1 * na * nb likewise, na the smallest; otherwise the
+// largest in-register n1, which leaves the smallest dense n2 (its cost grows with n2).
+// Six loads, one such axis among 64-point ones, apply, us, mixed-radix Stockham passes
+// (in use before these) / dense second factor / three steps: FP32 480 points z 526 /
+// 538 / 340, x 384 / 460 / 297; FP64 480 z 931 / 1003 / 747, x 798 / 958 / 764, 625 x
+// 1239 / 1953 / 1090.
+// z: the z pass keeps factors above 16 (FP32) only while 32 columns fit.  With 16 its
+// lanes index on their own, and wide factors spill there: 320 points as 16 * 20 take
+// 389 us, as 4 * 8 * 10 237 (301 by the Stockham passes).
 template <typename T>
-AxisPlan make_axis_plan(int n) {
+AxisPlan make_axis_plan(int n, bool z) {
   AxisPlan p{};
   p.n = n;
   p.n1 = 1;
@@ -817,6 +968,20 @@ AxisPlan make_axis_plan(int n) {
       p.n1 = a;
       p.n2 = b;
     }
+  }
+  if (p.dense || (z && best > 16 && sizeof(typename CT<T>::type) * n * 32 > kGenLds)) {
+    int most = 26;
+    for (int m = 2; m <= kMidMost; ++m)
+      for (int b = m; m * b * b <= n; ++b) {
+        const int a = n / (m * b);
+        if (a * m * b != n || a >= most || !three_step(a) || !three_step(b)) continue;
+        most = a;
+        p.n1 = a;
+        p.n2 = m * b;
+        p.na = m;
+        p.nb = b;
+        p.dense = 0;
+      }
   }
   p.hpad = dense_pad<T>(p);
   return p;
@@ -890,8 +1055,8 @@ int launch_gen_r2c(const GenX<T>& g, int nrhs, const T* r, typename CT<T>::type*
   const XUpdate<T> u = upd ? *upd : XUpdate<T>{};
   const T* in = upd && spec ? upd->q : r;
   const int sub = sub_of(g.plan, g.shape);
-#define VXL_G(MODE, WV)                                                                                              \
-  hipLaunchKernelGGL((gen_r2c<T, MODE, WV>), grid, block, g.shape.lds, s, in, S, ax, PB, g.rows, g.field_stride,       \
+#define VXL_G(MODE, WV, K3)                                                                                              \
+  hipLaunchKernelGGL((gen_r2c<T, MODE, WV, K3>), grid, block, g.shape.lds, s, in, S, ax, PB, g.rows, g.field_stride,       \
                      g.spec_stride, g.active, u)
   if (!upd) {
     VXL_GS(kGenPlain);
@@ -913,8 +1078,8 @@ int launch_gen_c2r(const GenX<T>& g, int nrhs, const typename CT<T>::type* S, T*
   const dim3 grid(unsigned((pairs + PB - 1) / PB), unsigned(nrhs)), block(unsigned(g.shape.P * g.shape.rows));
   const GenAxis<T> ax = axis_view<T>(g.plan, g.shape, g.w);
   const int sub = sub_of(g.plan, g.shape);
-#define VXL_G(DIR, WV)                                                                                            \
-  hipLaunchKernelGGL((gen_c2r<T, DIR, WV>), grid, block, g.shape.lds, s, S, z, ax, PB, g.rows, g.field_stride,     \
+#define VXL_G(DIR, WV, K3)                                                                                            \
+  hipLaunchKernelGGL((gen_c2r<T, DIR, WV, K3>), grid, block, g.shape.lds, s, S, z, ax, PB, g.rows, g.field_stride,     \
                      g.spec_stride, g.active, beta, pin, fold)
   if (beta) {
     VXL_GS(true);
@@ -935,8 +1100,8 @@ int launch_gen_y(const AxisPlan& plan, const GenShape& sh, const typename CT<T>:
   const dim3 grid(unsigned((cols + sh.units - 1) / sh.units), unsigned(nrhs)), block(unsigned(sh.P * sh.rows));
   const GenAxis<T> ax = axis_view<T>(plan, sh, w);
   const int sub = sub_of(plan, sh);
-#define VXL_G(INV, WV) \
-  hipLaunchKernelGGL((gen_y<INV, T, WV>), grid, block, sh.lds, s, S, src, ax, int(cols), W, stride, active)
+#define VXL_G(INV, WV, K3) \
+  hipLaunchKernelGGL((gen_y<INV, T, WV, K3>), grid, block, sh.lds, s, S, src, ax, int(cols), W, stride, active)
   if (inverse) {
     VXL_GS(true);
   } else {
@@ -956,8 +1121,8 @@ int launch_gen_z(const AxisPlan& plan, const GenShape& sh, const Tables<T>& tb, 
   const dim3 grid(unsigned((cols + sh.units - 1) / sh.units), unsigned(nrhs)), block(unsigned(sh.P * sh.rows));
   const GenAxis<T> ax = axis_view<T>(plan, sh, tb.wz);
   const int sub = sub_of(plan, sh);
-#define VXL_G(DOT, WV)                                                                                        \
-  hipLaunchKernelGGL((gen_z<T, DOT, WV>), grid, block, sh.lds, s, S, ax, ny, nxh, tb, lam, mu, inv_vn, stride, \
+#define VXL_G(DOT, WV, K3)                                                                                        \
+  hipLaunchKernelGGL((gen_z<T, DOT, WV, K3>), grid, block, sh.lds, s, S, ax, ny, nxh, tb, lam, mu, inv_vn, stride, \
                      active, nyq, partial, media, group_rhs)
   if (partial) {
     VXL_GS(true);
@@ -971,7 +1136,7 @@ int launch_gen_z(const AxisPlan& plan, const GenShape& sh, const Tables<T>& tb, 
 
 // Explicit instantiation of every launcher for one precision.
 #define VXL_FFTGEN_INSTANCES(T)                                                                                       \
-  template AxisPlan make_axis_plan<T>(int);                                                                           \
+  template AxisPlan make_axis_plan<T>(int, bool);                                                                         \
   template GenShape gen_shape_y<T>(const AxisPlan&);                                                                  \
   template GenShape gen_shape_z<T>(const AxisPlan&);                                                                  \
   template GenShape gen_shape_x<T>(const AxisPlan&, int);                                                             \
