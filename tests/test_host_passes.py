@@ -69,3 +69,18 @@ def test_axis_checks_match_the_numpy_pieces(plant, second):
         assert got == want
     else:
         assert all(np.array_equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("dtype,labels", [(np.uint8, 2), (np.uint8, 251), (np.int16, 300), (np.int32, 16384),
+                                          (np.int32, 16385), (np.int64, 100000)])
+@pytest.mark.parametrize("size", [1, 31, 32, 33, (1 << 18) - 1, (1 << 18), (1 << 19) + 5])
+def test_labels_in_no_order(dtype, labels, size):
+    """Random labels: narrow ranges (a table per piece) and wide ones (a shared
+    table), one piece and several, groups of 32 with and without a match."""
+    rng = np.random.default_rng(size + labels)
+    flat = rng.integers(0, labels, size).astype(dtype)
+    if size > 2:
+        flat[[0, -1]] = 0, labels - 1
+    assert np.array_equal(inputs.used_labels(flat.reshape(1, 1, -1)), np.unique(flat))
+    for label in {int(flat[0]), int(flat[-1]), labels // 2, labels}:
+        assert np.array_equal(pm.voxels_with_label(flat, label), np.flatnonzero(flat == label))

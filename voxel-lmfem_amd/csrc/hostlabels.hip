@@ -12,6 +12,11 @@ namespace vxl {
 namespace {
 
 constexpr int64_t kPiece = 1 << 18;  // entries per piece; fewer than two pieces run on the calling thread
+// Widest label range a piece marks in a table of its own.  Labels in no order, 8 threads:
+// 96^3 voxels of 200 labels 0.4 ms, 48^3 of 2 labels 0.09; marking a shared table
+// wherever the label changes took 7.9 and 0.8 ms (the threads write the same cache
+// lines, and the branch is a coin toss), bincount over pieces 1.8 and 0.3.
+constexpr int64_t kOwnTable = 1 << 14;
 
 // f(piece) for every piece, on at most `workers` threads.
 template <typename F>
@@ -89,18 +94,38 @@ int vxl_host_label_mark(const void* labels, int bytes, int is_signed, int64_t co
     std::atomic<bool> outside{false};
     for_pieces(pieces_of(count), workers, [&](int64_t k) {
       const int64_t a = k * kPiece, b = std::min(count, a + kPiece);
-      // Neighbouring voxels mostly share a label: the table is written where it changes.
-      L last = p[a];
-      auto mark = [&](L v) {
-        const int64_t at = int64_t(v) - int64_t(lo);
-        if (at < 0 || at >= span)
-          outside = true;
-        else
-          __atomic_store_n(present + at, uint8_t(1), __ATOMIC_RELAXED);
-      };
-      mark(last);
-      for (int64_t i = a + 1; i < b; ++i)
-        if (p[i] != last) mark(last = p[i]);
+      bool bad = false;
+      if (span <= kOwnTable) {
+        // A table of the piece's own, one store per voxel: no branch on the labels, and no
+        // cache line written by several threads, until the tables are joined.
+        uint8_t own[kOwnTable];
+        std::fill(own, own + span, uint8_t(0));
+        for (int64_t i = a; i < b; ++i) {
+          const uint64_t at = uint64_t(int64_t(p[i])) - uint64_t(lo);
+          if (at < uint64_t(span))
+            own[at] = 1;
+          else
+            bad = true;
+        }
+        for (int64_t l = 0; l < span; ++l)
+          if (own[l] && !__atomic_load_n(present + l, __ATOMIC_RELAXED))
+            __atomic_store_n(present + l, uint8_t(1), __ATOMIC_RELAXED);
+      } else {
+        // Wide ranges: the shared table, looked up where the label changes and written only
+        // where an entry is not set yet.
+        L last = p[a];
+        auto mark = [&](L v) {
+          const uint64_t at = uint64_t(int64_t(v)) - uint64_t(lo);
+          if (at >= uint64_t(span))
+            bad = true;
+          else if (!__atomic_load_n(present + at, __ATOMIC_RELAXED))
+            __atomic_store_n(present + at, uint8_t(1), __ATOMIC_RELAXED);
+        };
+        mark(last);
+        for (int64_t i = a + 1; i < b; ++i)
+          if (p[i] != last) mark(last = p[i]);
+      }
+      if (bad) outside = true;
     });
     return outside ? fail("vxl_host_label_mark: label outside the range") : VXL_OK;
   });
@@ -139,7 +164,28 @@ int vxl_host_find_label(const void* labels, int bytes, int is_signed, int64_t co
       *found = 0;
       return VXL_OK;
     }
+    // Positions of the label in [a, b) to out[o ...], which holds those up to `end`: a group of
+    // 32 without a match takes one compare in vector registers, the others write every
+    // position over the next free entry, without a branch on the labels.  Returns the next o.
+    auto collect = [&](int64_t a, int64_t b, int64_t o, int64_t end) {
+      for (int64_t g = a; g < b && o < end; g += 32) {
+        const int64_t e = std::min(b, g + 32);
+        bool any = e - g < 32;
+        if (!any)
+          for (int j = 0; j < 32; ++j) any |= p[g + j] == want;
+        if (!any) continue;
+        for (int64_t i = g; i < e && o < end; ++i) {
+          out[o] = i;
+          o += p[i] == want;
+        }
+      }
+      return o;
+    };
     const int64_t n = pieces_of(count);
+    if (n == 1 && capacity >= count) {  // room for every voxel: no count first
+      *found = collect(0, count, 0, count);
+      return VXL_OK;
+    }
     std::vector<int64_t> start(n + 1, 0);
     for_pieces(n, workers, [&](int64_t k) {
       const int64_t a = k * kPiece, b = std::min(count, a + kPiece);
@@ -149,10 +195,7 @@ int vxl_host_find_label(const void* labels, int bytes, int is_signed, int64_t co
     *found = start[n];
     if (start[n] > capacity) return VXL_OK;  // the caller asks again with room
     for_pieces(n, workers, [&](int64_t k) {
-      const int64_t a = k * kPiece, b = std::min(count, a + kPiece);
-      int64_t o = start[k];
-      for (int64_t i = a; i < b; ++i)
-        if (p[i] == want) out[o++] = i;
+      collect(k * kPiece, std::min(count, (k + 1) * kPiece), start[k], start[k + 1]);
     });
     return VXL_OK;
   });

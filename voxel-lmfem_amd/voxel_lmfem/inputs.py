@@ -17,15 +17,15 @@ from . import materials as mat
 def used_labels(phase):
     """np.unique(phase) of an integer array: marks over the label range when
     that range is narrow (one threaded host pass of the library, two for
-    labels wider than 16 bits; without it counts over pieces on a thread
+    labels wider than 8 bits; without it counts over pieces on a thread
     pool), a sort otherwise.  Same values and dtype."""
     flat = phase.reshape(-1)
     native = _native.host_labels(flat)
     if native is not None:
         lib, ptr, size, signed = native
         workers = mat.host_workers()
-        if size <= 2:
-            lo, span = (-(1 << (8 * size - 1)) if signed else 0), 1 << (8 * size)
+        if size == 1:
+            lo, span = (-128 if signed else 0), 256
         else:
             a, b = ctypes.c_longlong(), ctypes.c_longlong()
             _native.check(lib.vxl_host_label_range(ptr, size, signed, flat.size, workers, ctypes.byref(a),
