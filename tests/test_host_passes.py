@@ -84,3 +84,31 @@ def test_labels_in_no_order(dtype, labels, size):
     assert np.array_equal(inputs.used_labels(flat.reshape(1, 1, -1)), np.unique(flat))
     for label in {int(flat[0]), int(flat[-1]), labels // 2, labels}:
         assert np.array_equal(pm.voxels_with_label(flat, label), np.flatnonzero(flat == label))
+
+
+def _misaligned(a):
+    """The same array one byte past its item alignment."""
+    out = np.ndarray(a.shape, a.dtype, bytearray(a.nbytes + a.itemsize), offset=1)
+    out[...] = a
+    assert out.flags.c_contiguous and not out.flags.aligned
+    return out
+
+
+@pytest.mark.parametrize("dtype", [np.uint16, np.int32, np.int64])
+def test_misaligned_labels_take_the_numpy_route(dtype):
+    phase = _misaligned(np.random.default_rng(1).integers(0, 40, (1, 512, 520)).astype(dtype))
+    assert _native.host_labels(phase.reshape(-1)) is None
+    assert np.array_equal(inputs.used_labels(phase), np.unique(phase))
+    assert np.array_equal(pm.voxels_with_label(phase.reshape(-1), 7), np.flatnonzero(phase == 7))
+    assert _pack_labels(phase, {v: None for v in range(40)}) is None
+
+
+def test_misaligned_axes_take_the_numpy_route():
+    rng = np.random.default_rng(3)
+    shape = (4, 5, 6)
+    ori = {k: _misaligned(rng.normal(size=shape + (3,))) for k in ("axis1", "axis2")}
+    kept = tuple(np.empty((60, 3)) for _ in range(2))
+    sels = [np.arange(10, 70)]
+    assert not pm._native_axes((ori["axis1"], ori["axis2"]), shape, sels, 16, 2, kept)
+    got = pm.check_frames(ori, shape, sels, chunk=16, workers=2, keep=True)
+    assert all(np.array_equal(g, ori[k].reshape(-1, 3)[10:70]) for g, k in zip(got, ("axis1", "axis2")))

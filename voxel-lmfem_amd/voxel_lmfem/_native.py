@@ -114,8 +114,9 @@ def load():
 def host_labels(flat):
     """(library, pointer, item bytes, signed) for the host passes over a flat
     label array, or None when they do not take it: no library built, unsigned
-    64-bit, strided or byte-swapped labels."""
-    if (not flat.size or not flat.flags.c_contiguous or not flat.dtype.isnative or flat.dtype.kind not in "iu"
+    64-bit, strided, misaligned or byte-swapped labels."""
+    if (not flat.size or not (flat.flags.c_contiguous and flat.flags.aligned) or not flat.dtype.isnative
+            or flat.dtype.kind not in "iu"
             or (flat.dtype.kind == "u" and flat.dtype.itemsize == 8)):
         return None
     try:

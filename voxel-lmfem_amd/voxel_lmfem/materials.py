@@ -233,14 +233,14 @@ def frames(orientation, shape, flat_indices):
 
 
 def _native_axes(sources, shape, selections, chunk, workers, kept):
-    """The axis-pair checks of check_frames for full-grid C-ordered FP64 axes,
+    """The axis-pair checks of check_frames for full-grid C-ordered, aligned FP64 axes,
     by the library's threaded host pass (the same expressions in the same
     order, one read of the axes); fills kept and raises the first failing
     piece's error.  False when it does not apply."""
     import ctypes
     from . import _native
     full = tuple(shape) + (3,)
-    if any(s.shape != full or s.dtype != np.float64 or not s.flags.c_contiguous for s in sources):
+    if any(s.shape != full or s.dtype != np.float64 or not (s.flags.c_contiguous and s.flags.aligned) for s in sources):
         return False
     try:
         lib = _native.load()
