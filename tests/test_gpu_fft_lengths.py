@@ -70,3 +70,20 @@ def test_three_step_lengths(torch_gpu, n):
     tols = (("float64", 1e-11), ("float32", 5e-6)) if n <= 512 else (("float64", 1e-10), ("float32", 2e-5))
     for shape in ((3, 5, n), (3, n, 5), (n, 5, 3)):
         _check(torch_gpu, shape, h, 2, tols)
+
+
+@pytest.mark.parametrize("shape", [(16, 16, 16), (9, 10, 14), (37, 6, 34)])
+def test_denominators_past_the_largest_double(torch_gpu, shape):
+    """Entries of the C3D8R-HG symbol beyond 1.8e308 have reciprocal 0, not NaN: with
+    mu = 1e308 and h = 0.1 most wavevectors have one, and what is left is below
+    1e-300.  (The FI symbol subtracts two such terms, so that it has none.)"""
+    torch = torch_gpu
+    from voxel_lmfem.gpu import Cell, Preconditioner
+    field = pm.build_field(np.zeros(shape, dtype=np.int32), {0: dict(kind="isotropic", E=1.0, nu=0.3)})
+    cell = Cell(field, shape, np.full(3, 0.1), element="c3d8r_hg")
+    pc = Preconditioner(cell, 0.0, 1e308, precision="float64", nrhs_max=1)
+    r = torch.from_numpy(np.random.default_rng(4).normal(size=(1, 3, int(np.prod(shape))))).to("cuda")
+    z = pc.apply_planes(r)
+    assert bool(torch.isfinite(z).all()) and float(z.abs().max()) < 1e-300
+    pc.close()
+    cell.close()

@@ -290,13 +290,16 @@ struct Tables {
 
 // Reciprocal for the Green solve: the hardware estimate (<= 1 ulp) in FP32; in
 // FP64 the estimate with two Newton steps y += y (1 - x y), a third of the
-// instructions of a division.  x = 0 gives an infinity or NaN that the
-// callers discard.
+// instructions of a division.  Where the estimate is already 0, an infinity or
+// NaN (x infinite, 0 or NaN) it is the result, as a division gives it: the steps
+// would make NaN of each.
 __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ double rcp(double x) {
-  double y = __builtin_amdgcn_rcp(x);
+  const double y0 = __builtin_amdgcn_rcp(x);
+  constexpr int kNoSteps = 0x003 | 0x004 | 0x200 | 0x020 | 0x040;  // classes: NaN, -inf, +inf, -0, +0
+  double y = fma(y0, fma(-x, y0, 1.0), y0);
   y = fma(y, fma(-x, y, 1.0), y);
-  return fma(y, fma(-x, y, 1.0), y);
+  return __builtin_amdgcn_class(y0, kNoSteps) ? y0 : y;
 }
 
 // Per-axis factors of the Green symbol at one wavenumber: table columns 0-3
