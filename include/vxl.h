@@ -175,11 +175,11 @@ int vxl_tune_stencil(vxl_cell* cell, int precision, int nrhs, const void* u_dev,
 /* Full stencil configuration per precision: tile height (workgroup tile of
  * 32 x tile_y output nodes, 16 x 14 for VXL_F64's 6; VXL_F32: 14 (default),
  * 8 or 6; VXL_F64: 6 (default), 8 or 4), schedule (1-3, as above) and the
- * fewest z planes per workgroup chunk (2..64; each chunk recomputes one element
- * layer, and shallower chunks give small cells more workgroups; the default, 8,
- * leaves the depth to the launch, which may take any from 2).  Every
- * configuration computes the same element sums.  No reference counterpart (see
- * vxl_tune_stencil). */
+ * fewest z planes per workgroup chunk (2..64, or 0, the default; each chunk
+ * recomputes one element layer, and shallower chunks give small cells more
+ * workgroups; from that bound on the launch takes the depth with the least work,
+ * with 0 any from 2).  Every configuration computes the same element sums.  No
+ * reference counterpart (see vxl_tune_stencil). */
 int vxl_set_stencil_config(vxl_cell* cell, int precision, int tile_y, int variant, int zmin);
 /* Element of the cell's operator: VXL_ELEMENT_FI (default; fully integrated
  * HEX8, 2x2x2 Gauss) or VXL_ELEMENT_C3D8R_HG, the reference's reduced-
@@ -195,6 +195,18 @@ int vxl_set_stencil_config(vxl_cell* cell, int precision, int tile_y, int varian
  * while the matrix-core stencil or per-voxel frames are on (FI only). */
 int vxl_cell_set_element(vxl_cell* cell, int element, double hourglass_coefficient);
 int vxl_get_stencil_config(vxl_cell* cell, int precision, int* tile_y, int* variant, int* zmin);
+/* What an apply of nrhs fields would launch under the cell's configuration: the
+ * workgroup's output nodes tile_x x tile_y, the z planes per chunk and the kernel
+ * form, the sum of VXL_FORM_ORTHO (the table has no normal-shear or shear-shear
+ * entry; schedule 3 then leaves those products out), VXL_FORM_CUBIC (cubic
+ * voxels), VXL_FORM_HG, VXL_FORM_FRAMES and VXL_FORM_MFMA (FP32 only; tile_x and
+ * tile_y are then 0).  Outputs may be null.  No reference counterpart. */
+#define VXL_FORM_ORTHO 1
+#define VXL_FORM_CUBIC 2
+#define VXL_FORM_HG 4
+#define VXL_FORM_FRAMES 8
+#define VXL_FORM_MFMA 16
+int vxl_stencil_launch(vxl_cell* cell, int precision, int nrhs, int* tile_x, int* tile_y, int* depth, int* form);
 /* Matrix-core FP32 stencil (enable 1) or the modal VALU stencil (enable 0,
  * the default).  The matrix-core form is the label-grouped dense element
  * product f_e = K_L (u_e - u_e0) of the reference's grouped kernel

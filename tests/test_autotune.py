@@ -97,3 +97,36 @@ def test_default_ms_follows_the_cells_configuration(tmp_path):
                                       ("float32", (8, 2, 4), table[1, 1, 1])):
         assert autotune._table_ms(table, precision, *config) == expect
     assert np.isnan(autotune._table_ms(table, "float32", 16, 3, 8))
+
+
+class FormCell(FakeCell):
+    def __init__(self, form):
+        super().__init__()
+        self.form = form
+
+    def stencil_launch(self, precision="float32", nrhs=6):
+        return (32, 14), 2, self.form
+
+
+def test_entries_stay_with_their_kernel_form(tmp_path):
+    """A winner of one kernel form is not applied to another on the same grid."""
+    path = tmp_path / "t.json"
+    for form in ("", "cubic", "ortho", "ortho+cubic"):
+        assert autotune.tune(FormCell(form), "float32", 6, path=path)["tuned"], form
+        assert not autotune.tune(FormCell(form), "float32", 6, path=path)["tuned"], form
+    assert len(autotune.load(path)) == 4
+
+
+def test_entries_of_the_former_schema_are_dropped(tmp_path):
+    """Schema 1 entries were timed under other tiles and another chunk rule."""
+    path = tmp_path / "t.json"
+    cell = FakeCell()
+    entry = dict(tile_y=8, schedule=1, zmin=8)
+    path.write_text(json.dumps(dict(schema=1, entries={autotune.key(cell, "float32", 6): entry})))
+    assert autotune.load(path) == {}
+    assert autotune.tune(cell, "float32", 6, path=path)["tuned"]
+
+
+def test_automatic_depth_is_the_shallowest_of_the_table():
+    table = np.arange(27.0).reshape(3, 3, 3)
+    assert autotune._table_ms(table, "float32", 14, 3, 0) == table[0, 2, 2]

@@ -29,3 +29,35 @@ def test_chunk_rule_is_bitwise_neutral(torch_gpu, shape, nrhs):
             assert torch.equal(got, cell.apply_planes(u)), (count, precision)
             cell.set_stencil_config(precision, tile, schedule, depth)
         cell.close()
+
+
+@pytest.mark.parametrize("precision", ["float32", "float64"])
+@pytest.mark.parametrize("nrhs", [1, 6])
+def test_chunk_depth_is_a_lower_bound(torch_gpu, precision, nrhs):
+    """Depths 2 to 64 bound the planes per chunk from below (8 among them), 0 is
+    the automatic depth of a new cell, and the kernel form names the table."""
+    from voxel_lmfem import materials as pm
+    from voxel_lmfem.gpu import Cell
+    general = pm.isotropic_voigt(7.0, 0.3)
+    general[0, 3] = general[3, 0] = 0.4
+    rows = np.stack([pm.pack21(pm.isotropic_voigt(3.0, 0.35)), pm.pack21(general)])
+    shape = (40, 20, 24)
+    index = np.zeros(int(np.prod(shape)), dtype=np.uint8)
+    for count, h, form in ((1, (1.0, 1.0, 1.0), "ortho+cubic"), (1, (1.0, 1.0, 1.5), "ortho"),
+                           (2, (1.0, 1.0, 1.0), "cubic"), (2, (1.0, 1.0, 1.5), "")):
+        cell = Cell(pm.MaterialField(rows[:count], index, None, None, None), shape, h)
+        tile, schedule, zmin = cell.stencil_config(precision)
+        assert zmin == 0
+        _, automatic, got = cell.stencil_launch(precision, nrhs)
+        assert got == form and 2 <= automatic < 8   # a small grid: more chunks than depth 8 allows
+        for bound in (2, 4, 8, 16, 64):
+            cell.set_stencil_config(precision, tile, schedule, bound)
+            depth = cell.stencil_launch(precision, nrhs)[1]
+            assert min(bound, shape[0]) <= depth <= shape[0]
+            assert bound != 2 or depth == automatic
+        cell.set_stencil_config(precision, tile, schedule, 0)
+        assert cell.stencil_launch(precision, nrhs)[1] == automatic
+        for refused in (1, -1, 65):
+            with pytest.raises(ValueError):
+                cell.set_stencil_config(precision, tile, schedule, refused)
+        cell.close()

@@ -124,7 +124,7 @@ int cell_create_common(vxl_cell** out, int nz, int ny, int nx, double hx, double
   c->variant[1] = default_stencil_variant(VXL_F64);
   c->tile_y[0] = default_stencil_tile(VXL_F32);
   c->tile_y[1] = default_stencil_tile(VXL_F64);
-  c->zmin[0] = c->zmin[1] = kDefaultChunkPlanes;
+  c->zmin[0] = c->zmin[1] = 0;
   c->ortho = 0;
   c->element = VXL_ELEMENT_FI;
   c->hg_coef = 0.1;
@@ -532,7 +532,8 @@ int vxl_set_stencil_config(vxl_cell* cell, int precision, int tile_y, int varian
     return fail("vxl_set_stencil_config: invalid arguments");
   if (!stencil_tile_supported(precision, tile_y)) return fail("vxl_set_stencil_config: unsupported tile height");
   if (variant < 1 || variant > 3) return fail("vxl_set_stencil_config: schedule must be 1, 2 or 3");
-  if (zmin < kMinChunkPlanes || zmin > 64) return fail("vxl_set_stencil_config: chunk depth must lie in [2, 64]");
+  if (zmin != 0 && (zmin < kMinChunkPlanes || zmin > 64))
+    return fail("vxl_set_stencil_config: chunk depth must lie in [2, 64], or be 0 (the launch chooses)");
   const int slot = precision == VXL_F64 ? 1 : 0;
   cell->tile_y[slot] = tile_y;
   cell->variant[slot] = variant;
@@ -551,13 +552,20 @@ int vxl_get_stencil_config(vxl_cell* cell, int precision, int* tile_y, int* vari
   return VXL_OK;
 }
 
+int vxl_stencil_launch(vxl_cell* cell, int precision, int nrhs, int* tile_x, int* tile_y, int* depth, int* form) {
+  g_error.clear();
+  if (!cell || nrhs < 1 || (precision != VXL_F32 && precision != VXL_F64))
+    return fail("vxl_stencil_launch: invalid arguments");
+  return stencil_launch_info(cell, precision, nrhs, tile_x, tile_y, depth, form);
+}
+
 int vxl_autotune_stencil(vxl_cell* cell, int precision, int nrhs, const void* u_dev, void* out_dev, int reps,
                          int* tile_y, int* variant, int* zmin, double* ms_table) {
   g_error.clear();
   if (!cell || !u_dev || !out_dev || nrhs < 1 || reps < 1 || (precision != VXL_F32 && precision != VXL_F64))
     return fail("vxl_autotune_stencil: invalid arguments");
   const int slot = precision == VXL_F64 ? 1 : 0;
-  const int depths[3] = {kDefaultChunkPlanes, 4, kMinChunkPlanes};
+  const int depths[3] = {8, 4, kMinChunkPlanes};
   hipEvent_t e0, e1;
   VXL_HIP(hipEventCreate(&e0));
   VXL_HIP(hipEventCreate(&e1));

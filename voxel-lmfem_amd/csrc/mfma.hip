@@ -405,7 +405,7 @@ void mfma_grid(const vxl_cell* cell, int nrhs, int& tiles_x, int& tiles, int& ch
   const int nx = cell->grid.nx, ny = cell->grid.ny, nz = cell->grid.nz;
   tiles_x = (nx + kMX - 1) / kMX;
   tiles = tiles_x * ((ny + kMY - 1) / kMY);
-  const int zmin = std::max(kMinChunkPlanes, cell->zmin[0]);
+  const int zmin = cell->zmin[0] > 0 ? std::max(kMinChunkPlanes, cell->zmin[0]) : kMfmaChunkPlanes;
   chunks = (4096 + tiles * nrhs - 1) / (tiles * nrhs);
   chunks = std::max(1, std::min(chunks, nz / zmin));
   zchunk = (nz + chunks - 1) / chunks;

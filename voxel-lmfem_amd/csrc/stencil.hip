@@ -444,7 +444,7 @@ int launch_residual_apply(const vxl_cell* cell, int nrhs, const double* u, const
 
 int residual_apply_blocks(const vxl_cell* cell, int nrhs) {
   int tx, tiles, chunks, zc;
-  apply_grid<double, ResidTile::tx, ResidTile::ty>(cell, nrhs, tx, tiles, chunks, zc, kDefaultChunkPlanes);
+  apply_grid<double, ResidTile::tx, ResidTile::ty>(cell, nrhs, tx, tiles, chunks, zc, kMinChunkPlanes);
   return tiles * chunks;
 }
 
@@ -612,6 +612,50 @@ bool stencil_tile_supported(int precision, int tile_y) {
 }
 int default_stencil_tile(int precision) { return precision == VXL_F64 ? kTilesF64[0] : kTilesF32[0]; }
 int stencil_tile_option(int precision, int k) { return precision == VXL_F64 ? kTilesF64[k] : kTilesF32[k]; }
+
+template <typename T>
+int launch_info_t(const vxl_cell* cell, int nrhs, int (&out)[3]) {
+  int tx, tiles, chunks;
+  if constexpr (std::is_same<T, float>::value) {
+    if (cell->mfma) {
+      mfma_grid(cell, nrhs, tx, tiles, chunks, out[2]);
+      out[0] = out[1] = 0;
+      return VXL_OK;
+    }
+    if (cell->frame_index)
+      return frames_tile(cell, [&](auto ty) {
+        constexpr int TY = decltype(ty)::value;
+        apply_grid<T, 32, TY>(cell, nrhs, tx, tiles, chunks, out[2]);
+        out[0] = 32;
+        out[1] = TY;
+        return int(VXL_OK);
+      });
+  }
+  return with_tile<T>(cell, [&](auto t) {
+    using O = decltype(t);
+    apply_grid<T, O::tx, O::ty>(cell, nrhs, tx, tiles, chunks, out[2]);
+    out[0] = O::tx;
+    out[1] = O::ty;
+    return int(VXL_OK);
+  });
+}
+
+int stencil_launch_info(const vxl_cell* cell, int precision, int nrhs, int* tile_x, int* tile_y, int* depth,
+                        int* form) {
+  int v[3] = {0, 0, 0};
+  VXL_TRY(precision == VXL_F64 ? launch_info_t<double>(cell, nrhs, v) : launch_info_t<float>(cell, nrhs, v));
+  if (tile_x) *tile_x = v[0];
+  if (tile_y) *tile_y = v[1];
+  if (depth) *depth = v[2];
+  if (form) {
+    const bool hg = cell->element == VXL_ELEMENT_C3D8R_HG, f32 = precision == VXL_F32;
+    const bool frames = f32 && cell->frame_index, mfma = f32 && cell->mfma;
+    *form = (cell->ortho && !hg && !cell->mat.scale && !frames && !mfma ? VXL_FORM_ORTHO : 0) |
+            (cell->h[0] == cell->h[1] && cell->h[1] == cell->h[2] ? VXL_FORM_CUBIC : 0) | (hg ? VXL_FORM_HG : 0) |
+            (frames ? VXL_FORM_FRAMES : 0) | (mfma ? VXL_FORM_MFMA : 0);
+  }
+  return VXL_OK;
+}
 
 // One cell of a stacked cell: the same grid and rows, index block g.
 vxl_cell group_view(const vxl_cell* cell, int g) {

@@ -171,7 +171,7 @@ struct vxl_cell {
   int device;
   int variant[2];  // stencil schedule per precision (VXL_F32, VXL_F64): 1, 2 or 3
   int tile_y[2];   // stencil tile height (output nodes along y; the tile is 32 wide)
-  int zmin[2];     // fewest z planes per workgroup chunk (each chunk recomputes one layer)
+  int zmin[2];     // fewest z planes per workgroup chunk (each chunk recomputes one layer); 0: the launch chooses
   int ortho;       // every row has zeros outside the normal block and the shear diagonal
   int element;     // VXL_ELEMENT_FI (2x2x2 Gauss) or VXL_ELEMENT_C3D8R_HG (one point + hourglass)
   double hg_coef;  // hourglass coefficient of the C3D8R-HG element
@@ -208,8 +208,8 @@ int launch_apply_cg(const vxl_cell* cell, int nrhs, const T* p, T* q, const int*
                     int* blocks, hipStream_t s);
 template <typename T>
 int apply_cg_blocks(const vxl_cell* cell, int nrhs);
-constexpr int kDefaultChunkPlanes = 8;  // default fewest z planes per stencil chunk
-constexpr int kMinChunkPlanes = 2;      // smallest chunk depth a cell may be set to
+constexpr int kMinChunkPlanes = 2;   // fewest z planes of a stencil chunk
+constexpr int kMfmaChunkPlanes = 8;  // fewest of a matrix-core chunk where the cell's depth is automatic
 int apply_cg_blocks_max(const vxl_cell* cell, int nrhs, int precision);
 bool stencil_tile_supported(int precision, int tile_y);
 // Certification residual r = f - K u with the FP64 operator (r32 or r64
@@ -220,6 +220,8 @@ int launch_residual_apply(const vxl_cell* cell, int nrhs, const double* u, const
 int residual_apply_blocks(const vxl_cell* cell, int nrhs);
 int default_stencil_tile(int precision);
 int stencil_tile_option(int precision, int k);  // k = 0, 1, 2
+int stencil_launch_info(const vxl_cell* cell, int precision, int nrhs, int* tile_x, int* tile_y, int* depth, int* form);
+void mfma_grid(const vxl_cell* cell, int nrhs, int& tiles_x, int& tiles, int& chunks, int& zchunk);
 
 // C3D8R-HG hourglass penalty per element: s(C) = coef * max((I1 + 7 I2) / 60,
 // 1e-12) * V / hbar^2 with I1 = sum C_ii + 2 sum_{i<j<3} C_ij, I2 = sum_{i<3}

@@ -916,8 +916,8 @@ G9<T> cast_g(const ModalFactors& f) {
 // hides); workgroups run in rounds of two per CU, and a last round with at most
 // one per CU is shorter, but not half as long (six loads, default tiles: 2.2 us a
 // step with two, 1.7 with one).  The number of chunks with the least total is
-// taken, of those with at least `zmin` planes (under the default depth of 8 the
-// rule may go down to two).  Six loads, us, chunks as near eight planes as 4096
+// taken, of those with at least `zmin` planes (0: the cell's setting; automatic,
+// the default, is two).  Six loads, us, chunks as near eight planes as 4096
 // workgroups allow -> this rule: FP32 100 x 90 x 80 74 -> 61, 118 x 94 x 111
 // 123 -> 98, 160^3 346 -> 325, 256^3 1273 -> 1275; FP64 118 x 94 x 111 271 -> 243,
 // 160^3 700 -> 687.  One load: 160^3 FP32 59.6 -> 50.7, FP64 118 -> 110.
@@ -930,7 +930,7 @@ void apply_grid(const vxl_cell* cell, int nrhs, int& tiles_x, int& tiles, int& c
   const int tiles_y = (ny + TY - 1) / TY;
   tiles = tiles_x * tiles_y;
   if (zmin <= 0) zmin = cell->zmin[std::is_same<T, double>::value ? 1 : 0];
-  if (zmin == kDefaultChunkPlanes) zmin = kMinChunkPlanes;
+  zmin = std::max(zmin, kMinChunkPlanes);
   const int64_t columns = int64_t(tiles) * nrhs;
   const int limit = std::max(1, std::min(nz / kMinChunkPlanes, int((4096 + columns - 1) / columns)));
   if (most) {
@@ -1019,7 +1019,7 @@ int launch_apply_impl(const vxl_cell* cell, int nrhs, const T* u, T* out, hipStr
 }
 
 // Certification residual r = f - K u (FP64 operator, default FP64 tile,
-// schedule 3, chunks of kDefaultChunkPlanes planes): u FP64, r into r32 or
+// schedule 3, chunk depth by apply_grid's rule): u FP64, r into r32 or
 // r64, ||r||^2 partials per workgroup; systems with active == 0 are skipped.
 template <typename Idx, bool kScale, bool kOrtho = false>
 int launch_resid_impl(const vxl_cell* cell, int nrhs, const double* u, const double* f, float* r32, double* r64,
@@ -1044,7 +1044,7 @@ int launch_resid_impl(const vxl_cell* cell, int nrhs, const double* u, const dou
   a.ny = cell->grid.ny;
   a.nz = cell->grid.nz;
   int tiles = 0, chunks = 0;
-  apply_grid<double, TX, TY>(cell, nrhs, a.tiles_x, tiles, chunks, a.zchunk, kDefaultChunkPlanes);
+  apply_grid<double, TX, TY>(cell, nrhs, a.tiles_x, tiles, chunks, a.zchunk, kMinChunkPlanes);
   const ModalFactors mf = modal_factors(cell->h);
   a.g = cast_g<double>(mf);
   const bool hg = cell->element == VXL_ELEMENT_C3D8R_HG;

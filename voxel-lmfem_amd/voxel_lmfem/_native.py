@@ -50,6 +50,7 @@ SIGNATURES = {
     "vxl_set_stencil_config": (_I, [_P, _I, _I, _I, _I]),
     "vxl_cell_set_element": (_I, [_P, _I, _D]),
     "vxl_get_stencil_config": (_I, [_P, _I, _IP, _IP, _IP]),
+    "vxl_stencil_launch": (_I, [_P, _I, _I, _IP, _IP, _IP, _IP]),
     "vxl_cell_set_mfma": (_I, [_P, _I]),
     "vxl_cell_set_frames": (_I, [_P, _I, _DP, _IP, _P, _P]),
     "vxl_cell_set_groups": (_I, [_P, _I]),

@@ -1,13 +1,15 @@
 """Stencil autotuner with a persistent JSON cache.
 
 The stencil has three run-time knobs per precision (all compute the same
-element sums): the workgroup tile (32 x tile_y output nodes), the schedule
+element sums): the workgroup tile (tile_y output nodes high), the schedule
 (1: per-layer 8-node transform, 2: persistent face columns, 3: 2 with the
-plane after next prefetched) and the fewest z planes per workgroup chunk.
+plane after next prefetched) and the fewest z planes per workgroup chunk (8, 4
+or 2; the launch takes the depth with the least work from there on, and an
+untuned cell's automatic depth, 0, is 2).
 ``vxl_autotune_stencil`` times the 27 combinations on a cell; this module
 keeps the winners in a JSON file keyed by everything the timing depends on
-(grid, precision, load count, material index width, per-voxel scale, device
-name), so a shape is tuned once per machine.  The reference records its own
+(grid, precision, load count, material index width, per-voxel scale, kernel
+form, device name), so a shape is tuned once per machine.  The reference records its own
 operator-variant choice in ``_core/hybrid_operator/recommended.json:1-6``
 (written by ``hybrid_operator/study.py:64-82``); this is the measured
 counterpart for this build's stencil.
@@ -19,7 +21,7 @@ import os
 import tempfile
 from pathlib import Path
 
-SCHEMA = 1
+SCHEMA = 2   # 1: FP64 tile 6 always 32 x 6, another chunk rule, no kernel form in the key
 
 
 def cache_path(path=None):
@@ -78,19 +80,23 @@ def _table_ms(table, precision, tile_y, schedule, zmin):
     """Milliseconds of one configuration in the 3 x 3 x 3 autotune table
     (NaN if the configuration is not one of the tuned ones)."""
     tiles = TILES["fp64" if precision in ("float64", "fp64") else "fp32"]
+    zmin = zmin or DEPTHS[-1]   # automatic
     if tile_y not in tiles or zmin not in DEPTHS or not 1 <= schedule <= 3:
         return float("nan")
     return float(table[tiles.index(tile_y), schedule - 1, DEPTHS.index(zmin)])
 
 
 def key(cell, precision, nrhs):
-    """Cache key: device, precision, grid (z, y, x), loads, index width, scale."""
+    """Cache key: device, precision, grid (z, y, x), loads, index width, scale,
+    and the kernel form where the cell names one (Cell.stencil_launch)."""
     prec = "fp64" if precision in ("float64", "fp64") else "fp32"
     nz, ny, nx = cell.shape
     width = {1: "u8", 2: "u16", 4: "i32"}.get(int(cell.index.element_size()), "?")
     device = cell.torch.cuda.get_device_name(cell.device)
     scaled = "scaled" if cell.scale is not None else "plain"
-    return f"{device}|{prec}|{nz}x{ny}x{nx}|r{int(nrhs)}|{width}|{scaled}"
+    launch = getattr(cell, "stencil_launch", None)
+    form = f"|{launch(precision, nrhs)[2] or 'general'}" if launch else ""
+    return f"{device}|{prec}|{nz}x{ny}x{nx}|r{int(nrhs)}|{width}|{scaled}{form}"
 
 
 def tune(cell, precision="float32", nrhs=6, *, path=None, reps=3, refresh=False, entries=None):

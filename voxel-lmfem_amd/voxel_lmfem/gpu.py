@@ -209,11 +209,24 @@ class Cell:
         return _native.VXL_F64 if precision in ("float64", "fp64") else _native.VXL_F32
 
     def stencil_config(self, precision="float32"):
-        """(tile_y, schedule, fewest z planes per chunk) of the stencil."""
+        """(tile_y, schedule, fewest z planes per chunk; 0: the launch chooses) of the stencil."""
         t, v, z = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
         check(self.lib.vxl_get_stencil_config(self.handle, self._code(precision), ctypes.byref(t), ctypes.byref(v),
                                               ctypes.byref(z)), "vxl_get_stencil_config")
         return t.value, v.value, z.value
+
+    FORMS = ("ortho", "cubic", "hg", "frames", "mfma")
+
+    def stencil_launch(self, precision="float32", nrhs=6):
+        """What an apply of nrhs fields launches: (tile_x, tile_y) output nodes
+        of a workgroup, z planes per chunk, and the kernel form as names of
+        FORMS joined by "+" ("" for the general form on non-cubic voxels)."""
+        tx, ty, depth, form = (ctypes.c_int() for _ in range(4))
+        check(self.lib.vxl_stencil_launch(self.handle, self._code(precision), int(nrhs), ctypes.byref(tx),
+                                          ctypes.byref(ty), ctypes.byref(depth), ctypes.byref(form)),
+              "vxl_stencil_launch")
+        names = "+".join(n for k, n in enumerate(self.FORMS) if form.value >> k & 1)
+        return (tx.value, ty.value), depth.value, names
 
     def set_mfma(self, enable=True):
         """Run the cell's FP32 applies (plain and CG form) on the matrix cores:
