@@ -173,8 +173,9 @@ int vxl_get_stencil_variant(vxl_cell* cell, int precision);
 int vxl_tune_stencil(vxl_cell* cell, int precision, int nrhs, const void* u_dev, void* out_dev, int reps,
                      int* best, double* ms3);
 /* Full stencil configuration per precision: tile height (workgroup tile of
- * 32 x tile_y output nodes, 16 x 14 for VXL_F64's 6; VXL_F32: 14 (default),
- * 8 or 6; VXL_F64: 6 (default), 8 or 4), schedule (1-3, as above) and the
+ * 32 x tile_y output nodes, but VXL_F64's 6, which is 32 x 6 or 16 x 14 by the
+ * grid; VXL_F32: 14 (default), 8 or 6; VXL_F64: 6 (default), 8 or 4), schedule
+ * (1-3, as above) and the
  * fewest z planes per workgroup chunk (2..64, or 0, the default; each chunk
  * recomputes one element layer, and shallower chunks give small cells more
  * workgroups; from that bound on the launch takes the depth with the least work,

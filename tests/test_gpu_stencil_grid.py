@@ -61,3 +61,31 @@ def test_chunk_depth_is_a_lower_bound(torch_gpu, precision, nrhs):
             with pytest.raises(ValueError):
                 cell.set_stencil_config(precision, tile, schedule, refused)
         cell.close()
+
+
+@pytest.mark.parametrize("shape,tile", [((32, 32, 32), (32, 6)), ((72, 16, 84), (32, 6)), ((2, 3, 2), (32, 6)),
+                                        ((9, 13, 33), (32, 6)), ((64, 64, 64), (16, 14)), ((17, 56, 48), (16, 14))])
+def test_default_fp64_tile_by_grid(torch_gpu, shape, tile):
+    """FP64's option 6 is 32 x 6 or 16 x 14 by the grid; both give the sums of the
+    other options (1e-13 as for every configuration), in the general and the
+    orthotropic form and under the other schedules."""
+    torch = torch_gpu
+    from voxel_lmfem import materials as pm
+    from voxel_lmfem.gpu import Cell
+    rng = np.random.default_rng(5)
+    general = pm.isotropic_voigt(7.0, 0.3)
+    general[0, 3] = general[3, 0] = 0.4
+    rows = np.stack([pm.pack21(pm.isotropic_voigt(3.0, 0.35)), pm.pack21(general)])
+    n = int(np.prod(shape))
+    index = (rng.random(n) < 0.4).astype(np.uint8)
+    u = torch.from_numpy(rng.standard_normal((6, 3, n))).to("cuda")
+    for count in (1, 2):
+        cell = Cell(pm.MaterialField(rows[:count], index * (count - 1), None, None, None), shape, (1.0, 1.0, 1.5))
+        assert cell.stencil_launch("float64", 6)[0] == tile
+        cell.set_stencil_config("float64", 8, 3, 0)
+        want = cell.apply_planes(u).clone()
+        for schedule in (3, 2, 1):
+            cell.set_stencil_config("float64", 6, schedule, 0)
+            got = cell.apply_planes(u)
+            assert float((got - want).abs().max()) <= 1e-13 * float(want.abs().max()), (count, schedule)
+        cell.close()

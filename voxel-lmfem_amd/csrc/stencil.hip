@@ -451,10 +451,10 @@ int residual_apply_blocks(const vxl_cell* cell, int nrhs) {
 // Runtime tile choice -> template instance (the C3D8R-HG element runs the
 // default tile only).
 template <typename T, typename F>
-int with_tile(const vxl_cell* cell, F&& f) {
+int with_tile(const vxl_cell* cell, int nrhs, F&& f) {
   constexpr bool d = std::is_same<T, double>::value;
   const int ty = cell->element == VXL_ELEMENT_C3D8R_HG ? (d ? kTilesF64[0] : kTilesF32[0]) : cell->tile_y[d ? 1 : 0];
-  return with_tile_of<T>(ty, f);
+  return with_tile_of<T>(cell, nrhs, ty, f);
 }
 
 // The orthotropic form serves the FI element without a scale field (schedule
@@ -482,7 +482,7 @@ int launch_apply_t(const vxl_cell* cell, int nrhs, const T* u, T* out, hipStream
   if (cell->element == VXL_ELEMENT_C3D8R_HG)
     return dispatch_apply<T, DefaultTile<T>::tx, DefaultTile<T>::ty, true>(cell, nrhs, u, out, s);
   if (takes_ortho<T>(cell)) return launch_apply_ortho<T>(cell, nrhs, u, out, s, nullptr, nullptr, nullptr);
-  return with_tile<T>(cell, [&](auto t) {
+  return with_tile<T>(cell, nrhs, [&](auto t) {
     using O = decltype(t);
     return dispatch_apply<T, O::tx, O::ty>(cell, nrhs, u, out, s);
   });
@@ -500,7 +500,7 @@ int launch_apply_cg_t(const vxl_cell* cell, int nrhs, const T* p, T* q, const in
   if (cell->element == VXL_ELEMENT_C3D8R_HG)
     return dispatch_apply<T, DefaultTile<T>::tx, DefaultTile<T>::ty, true>(cell, nrhs, p, q, s, active, partial, blocks);
   if (takes_ortho<T>(cell)) return launch_apply_ortho<T>(cell, nrhs, p, q, s, active, partial, blocks);
-  return with_tile<T>(cell, [&](auto t) {
+  return with_tile<T>(cell, nrhs, [&](auto t) {
     using O = decltype(t);
     return dispatch_apply<T, O::tx, O::ty>(cell, nrhs, p, q, s, active, partial, blocks);
   });
@@ -516,7 +516,7 @@ int cg_blocks_t(const vxl_cell* cell, int nrhs, bool most) {
         return tiles * chunks;
       });
   }
-  return with_tile<T>(cell, [&](auto t) {
+  return with_tile<T>(cell, nrhs, [&](auto t) {
     using O = decltype(t);
     int tx, tiles, chunks, zc;
     apply_grid<T, O::tx, O::ty>(cell, nrhs, tx, tiles, chunks, zc, 0, most);
@@ -631,7 +631,7 @@ int launch_info_t(const vxl_cell* cell, int nrhs, int (&out)[3]) {
         return int(VXL_OK);
       });
   }
-  return with_tile<T>(cell, [&](auto t) {
+  return with_tile<T>(cell, nrhs, [&](auto t) {
     using O = decltype(t);
     apply_grid<T, O::tx, O::ty>(cell, nrhs, tx, tiles, chunks, out[2]);
     out[0] = O::tx;

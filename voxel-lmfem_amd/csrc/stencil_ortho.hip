@@ -20,7 +20,7 @@ int by_index(const vxl_cell* cell, F&& f) {
 template <typename T>
 int launch_apply_ortho(const vxl_cell* cell, int nrhs, const T* u, T* out, hipStream_t s, const int* active,
                        double* partial, int* blocks) {
-  return with_tile_of<T>(cell->tile_y[std::is_same<T, double>::value ? 1 : 0], [&](auto t) {
+  return with_tile_of<T>(cell, nrhs, cell->tile_y[std::is_same<T, double>::value ? 1 : 0], [&](auto t) {
     using O = decltype(t);
     return by_index(cell, [&](auto tag) {
       return launch_apply_impl<T, decltype(tag), false, O::tx, O::ty, false, true>(cell, nrhs, u, out, s, active,

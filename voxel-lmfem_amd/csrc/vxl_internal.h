@@ -170,7 +170,7 @@ struct vxl_cell {
   hipStream_t stream;
   int device;
   int variant[2];  // stencil schedule per precision (VXL_F32, VXL_F64): 1, 2 or 3
-  int tile_y[2];   // stencil tile height (output nodes along y; the tile is 32 wide)
+  int tile_y[2];   // stencil tile option (see kTilesF32, kTilesF64: output nodes along y, 32 wide but for FP64's 6)
   int zmin[2];     // fewest z planes per workgroup chunk (each chunk recomputes one layer); 0: the launch chooses
   int ortho;       // every row has zeros outside the normal block and the shear diagonal
   int element;     // VXL_ELEMENT_FI (2x2x2 Gauss) or VXL_ELEMENT_C3D8R_HG (one point + hourglass)

@@ -305,17 +305,16 @@ __device__ __forceinline__ BlockId xcd_block() {
 // FP32 32 x 14 nodes = 33 x 15 elements = 8 waves, so two workgroups (16
 // waves, 4 per SIMD) share a CU at up to 128 VGPRs; 32 x 16 (9 waves) fits
 // only one at the 96 VGPRs that pairing would need, and ran 1.55x slower.
-// Smaller tiles give small cells more workgroups.  FP64 default 32 x 6
-// (4 waves): measured 2.90 ms against 3.66 ms for 32 x 8 per six-RHS launch
-// at 256^3 (schedule 3).
+// Smaller tiles give small cells more workgroups.  FP64's default, 6, is four
+// waves (256^3, six loads, schedule 3: 2.68 ms against 3.66 for 32 x 8).
 constexpr int kTilesF32[3] = {14, 8, 6};
 constexpr int kTilesF64[3] = {6, 8, 4};
 
 // Nodes of a tile option.  All are 32 wide and as high as their name but FP64's
-// default, 6, which is 16 x 14: its 17 x 15 elements fill four waves, and it
-// computes 1.14 elements per output node against 1.20 for 32 x 6 (six loads,
-// 64^3 54.9 -> 44.6 us, 100 x 90 x 80 141 -> 121, 118 x 94 x 111 243 -> 218, 192 x
-// 160 x 144 815 -> 719, 256^3 2835 -> 2682; 32^3, where 32 fits, 13.3 -> 14.0).
+// default, 6, which is 16 x 14 or 32 x 6 by the grid (wide_f64): the 17 x 15 elements
+// of the former fill four waves, and it computes 1.14 elements per output node
+// against 1.20 (six loads, 64^3 54.9 -> 44.6 us, 100 x 90 x 80 141 -> 121, 118 x 94 x
+// 111 243 -> 218, 192 x 160 x 144 815 -> 719, 256^3 2835 -> 2682).
 // FP32 gains nothing from 16 x 14 (160^3 347 -> 344 us, 256^3
 // 1289 -> 1334).
 template <typename T, int OPT>
@@ -324,6 +323,9 @@ struct TileOption {
   static constexpr int tx = kSquare ? 16 : 32, ty = kSquare ? 14 : OPT;
 };
 using ResidTile = TileOption<double, kTilesF64[0]>;
+struct WideTile {  // FP64's option 6 where wide_f64 holds
+  static constexpr int tx = 32, ty = 6;
+};
 
 template <int TX, int TY>
 struct Tile {
@@ -921,23 +923,9 @@ G9<T> cast_g(const ModalFactors& f) {
 // workgroups allow -> this rule: FP32 100 x 90 x 80 74 -> 61, 118 x 94 x 111
 // 123 -> 98, 160^3 346 -> 325, 256^3 1273 -> 1275; FP64 118 x 94 x 111 271 -> 243,
 // 160^3 700 -> 687.  One load: 160^3 FP32 59.6 -> 50.7, FP64 118 -> 110.
-// most: the largest number of chunks any depth setting can give.
-template <typename T, int TX, int TY>
-void apply_grid(const vxl_cell* cell, int nrhs, int& tiles_x, int& tiles, int& chunks, int& zchunk,
-                int zmin = 0, bool most = false) {
-  const int nx = cell->grid.nx, ny = cell->grid.ny, nz = cell->grid.nz;
-  tiles_x = (nx + TX - 1) / TX;
-  const int tiles_y = (ny + TY - 1) / TY;
-  tiles = tiles_x * tiles_y;
-  if (zmin <= 0) zmin = cell->zmin[std::is_same<T, double>::value ? 1 : 0];
-  zmin = std::max(zmin, kMinChunkPlanes);
-  const int64_t columns = int64_t(tiles) * nrhs;
-  const int limit = std::max(1, std::min(nz / kMinChunkPlanes, int((4096 + columns - 1) / columns)));
-  if (most) {
-    chunks = limit;
-    zchunk = (nz + chunks - 1) / chunks;
-    return;
-  }
+// Planes per chunk of `columns` workgroup columns (at most `limit` chunks), and the
+// total in those units.
+inline int64_t chunk_rule(int64_t columns, int nz, int zmin, int limit, int& zchunk) {
   constexpr int kCu = 256;
   int64_t best = -1;
   for (int c = 1; c <= limit; ++c) {
@@ -951,6 +939,47 @@ void apply_grid(const vxl_cell* cell, int nrhs, int& tiles_x, int& tiles, int& c
       zchunk = depth;
     }
   }
+  return best;
+}
+inline int chunk_limit(int64_t columns, int nz) {
+  return std::max(1, std::min(nz / kMinChunkPlanes, int((4096 + columns - 1) / columns)));
+}
+
+// Whether FP64's tile option 6 is 32 x 6 on this grid: where the rule gives it no more
+// steps than 16 x 14 (grids that 32 or 6 fit better, and launches of one round), since a
+// step of it costs up to a twentieth less (231 elements instead of 255).  General form,
+// six loads, us, x last, 16 x 14 -> 32 x 6: 32^3 13.5 -> 12.9, 72 x 16 x 84 30.8 -> 23.5, 64 x 18 x
+// 256 68.0 -> 53.3, 20 x 200 x 20 28.6 -> 26.9; with a twentieth more steps 40 x 185 x 149
+// 202 -> 205.
+inline bool wide_f64(const vxl_cell* cell, int nrhs) {
+  const Grid& g = cell->grid;
+  int depth;
+  auto steps = [&](int tx, int ty) {
+    const int64_t columns = int64_t((g.nx + tx - 1) / tx) * ((g.ny + ty - 1) / ty) * nrhs;
+    return chunk_rule(columns, g.nz, kMinChunkPlanes, chunk_limit(columns, g.nz), depth);
+  };
+  return cell->element == VXL_ELEMENT_FI &&
+         steps(WideTile::tx, WideTile::ty) <= steps(ResidTile::tx, ResidTile::ty);
+}
+
+// most: the largest number of chunks any depth setting can give.
+template <typename T, int TX, int TY>
+void apply_grid(const vxl_cell* cell, int nrhs, int& tiles_x, int& tiles, int& chunks, int& zchunk,
+                int zmin = 0, bool most = false) {
+  const int nx = cell->grid.nx, ny = cell->grid.ny, nz = cell->grid.nz;
+  tiles_x = (nx + TX - 1) / TX;
+  const int tiles_y = (ny + TY - 1) / TY;
+  tiles = tiles_x * tiles_y;
+  if (zmin <= 0) zmin = cell->zmin[std::is_same<T, double>::value ? 1 : 0];
+  zmin = std::max(zmin, kMinChunkPlanes);
+  const int64_t columns = int64_t(tiles) * nrhs;
+  const int limit = chunk_limit(columns, nz);
+  if (most) {
+    chunks = limit;
+    zchunk = (nz + chunks - 1) / chunks;
+    return;
+  }
+  chunk_rule(columns, nz, zmin, limit, zchunk);
   chunks = (nz + zchunk - 1) / zchunk;
 }
 
@@ -1078,8 +1107,11 @@ int launch_resid_impl(const vxl_cell* cell, int nrhs, const double* u, const dou
 
 // Runtime tile choice -> template instance.
 template <typename T, typename F>
-int with_tile_of(int ty, F&& f) {
+int with_tile_of(const vxl_cell* cell, int nrhs, int ty, F&& f) {
   constexpr bool d = std::is_same<T, double>::value;
+  if constexpr (d) {
+    if (ty == kTilesF64[0] && wide_f64(cell, nrhs)) return f(WideTile());
+  }
   const auto& list = d ? kTilesF64 : kTilesF32;
   if (ty == list[0]) return f(TileOption<T, (d ? kTilesF64[0] : kTilesF32[0])>());
   if (ty == list[1]) return f(TileOption<T, (d ? kTilesF64[1] : kTilesF32[1])>());
