@@ -84,3 +84,12 @@ def test_rhs(torch_gpu, shape, kind, scale, nload):
     top = s.abs().max() * H[0] * H[1] * H[2] * sum(abs(x) for x in _grad(7)) * 8
     assert (got - f).abs().max() <= 64 * 2.3e-16 * top
     cell.close()
+
+
+# More than 1024 single planes of 256 columns: chunks of two planes and more, the last one short.
+@pytest.mark.parametrize("shape", [(3, 190, 200), (7, 120, 101), (35, 150, 160)])
+@pytest.mark.parametrize("kind,scale,nload", [(np.uint8, False, 6), (np.uint16, True, 3)])
+def test_chunks_of_several_planes(torch_gpu, shape, kind, scale, nload):
+    assert (shape[1] * shape[2] + 255) // 256 * nload * shape[0] > 1024 or nload == 3
+    test_center_fields(torch_gpu, shape, kind, scale, nload)
+    test_rhs(torch_gpu, shape, kind, scale, nload)

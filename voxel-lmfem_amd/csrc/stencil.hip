@@ -240,12 +240,17 @@ rhs_kernel(const void* index, const double* __restrict__ sig, const float* __res
 }
 
 // Planes per block of the kernels that march columns: about 4096 blocks for all
-// columns and loads, chunks of 2 to 16 planes (each reads one plane twice).
+// columns and loads, chunks of 2 to 16 planes (each reads one plane twice); single
+// planes where those are at most 1024 blocks, all resident at once, since a second
+// plane then only lengthens each thread's chain (32^3, one load, with the launch: centre
+// fields 30.2 -> 28.3 us, right-hand side 27.5 -> 26.4; 64^3, six loads, 6144 single
+// planes: 62.5 against 64.5, 47.1 against 52.8).
 inline dim3 column_grid(int nx, int ny, int nz, int nload, int& depth) {
   const int64_t columns = (int64_t(nx) * ny + 255) / 256;
   const int loads = std::max(1, std::min(nload, 65535));
   const int64_t chunks = std::max<int64_t>(1, 4096 / (columns * loads));
-  depth = int(std::max<int64_t>({2, std::min<int64_t>(16, nz / chunks), (int64_t(nz) + 65534) / 65535}));
+  const int64_t least = columns * loads * nz <= 1024 ? 1 : 2;
+  depth = int(std::max<int64_t>({least, std::min<int64_t>(16, nz / chunks), (int64_t(nz) + 65534) / 65535}));
   return dim3(unsigned(columns), unsigned((nz + depth - 1) / depth), unsigned(loads));
 }
 
@@ -467,8 +472,14 @@ bool takes_ortho(const vxl_cell* cell) {
          cell->variant[std::is_same<T, double>::value ? 1 : 0] == 3;
 }
 
-template <typename T>
-using DefaultTile = TileOption<T, (std::is_same<T, double>::value ? kTilesF64[0] : kTilesF32[0])>;
+// The default option's tile (the C3D8R-HG element has no other).
+template <typename T, typename F>
+int with_default_tile(const vxl_cell* cell, int nrhs, F&& f) {
+  if constexpr (std::is_same<T, double>::value)
+    return wide_f64(cell, nrhs) ? f(WideTile()) : f(ResidTile());
+  else
+    return f(TileOption<float, kTilesF32[0]>());
+}
 
 template <typename T>
 int launch_apply_t(const vxl_cell* cell, int nrhs, const T* u, T* out, hipStream_t s) {
@@ -480,7 +491,10 @@ int launch_apply_t(const vxl_cell* cell, int nrhs, const T* u, T* out, hipStream
       });
   }
   if (cell->element == VXL_ELEMENT_C3D8R_HG)
-    return dispatch_apply<T, DefaultTile<T>::tx, DefaultTile<T>::ty, true>(cell, nrhs, u, out, s);
+    return with_default_tile<T>(cell, nrhs, [&](auto t) {
+      using O = decltype(t);
+      return dispatch_apply<T, O::tx, O::ty, true>(cell, nrhs, u, out, s);
+    });
   if (takes_ortho<T>(cell)) return launch_apply_ortho<T>(cell, nrhs, u, out, s, nullptr, nullptr, nullptr);
   return with_tile<T>(cell, nrhs, [&](auto t) {
     using O = decltype(t);
@@ -498,7 +512,10 @@ int launch_apply_cg_t(const vxl_cell* cell, int nrhs, const T* p, T* q, const in
       });
   }
   if (cell->element == VXL_ELEMENT_C3D8R_HG)
-    return dispatch_apply<T, DefaultTile<T>::tx, DefaultTile<T>::ty, true>(cell, nrhs, p, q, s, active, partial, blocks);
+    return with_default_tile<T>(cell, nrhs, [&](auto t) {
+      using O = decltype(t);
+      return dispatch_apply<T, O::tx, O::ty, true>(cell, nrhs, p, q, s, active, partial, blocks);
+    });
   if (takes_ortho<T>(cell)) return launch_apply_ortho<T>(cell, nrhs, p, q, s, active, partial, blocks);
   return with_tile<T>(cell, nrhs, [&](auto t) {
     using O = decltype(t);

@@ -958,8 +958,7 @@ inline bool wide_f64(const vxl_cell* cell, int nrhs) {
     const int64_t columns = int64_t((g.nx + tx - 1) / tx) * ((g.ny + ty - 1) / ty) * nrhs;
     return chunk_rule(columns, g.nz, kMinChunkPlanes, chunk_limit(columns, g.nz), depth);
   };
-  return cell->element == VXL_ELEMENT_FI &&
-         steps(WideTile::tx, WideTile::ty) <= steps(ResidTile::tx, ResidTile::ty);
+  return steps(WideTile::tx, WideTile::ty) <= steps(ResidTile::tx, ResidTile::ty);
 }
 
 // most: the largest number of chunks any depth setting can give.
