@@ -956,10 +956,10 @@ struct CgHooks {
 
 enum Stages { kForwardX = 1, kRest = 2, kAllStages = 3 };
 
-// Runs the x forward pass (kForwardX, optionally fused with the CG update upd,
-// four-step x passes only) and/or the remaining passes (kRest).
+// Runs the x forward pass (kForwardX, optionally fused with the CG update upd)
+// and/or the remaining passes (kRest).
 // SC is the spectrum storage type: CT<T>::type, or bf16x2 (four-step passes only).
-// sr (spectral residual; FP32 storage, four-step x and y passes): the CG
+// sr (spectral residual; full-precision storage): the CG
 // residual lives as its x spectrum in im->rhat.  The forward pass writes the
 // x spectrum of r there (no upd) or updates it, R^ -= alpha q^, from the
 // transform of upd->q (with upd); the y forward pass reads R^ and writes the

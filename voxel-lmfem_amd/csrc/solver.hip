@@ -156,7 +156,7 @@ int upload_control(vxl_solver* s, const double* macro_host, hipStream_t st) {
 // One iteration: [stencil: q = K p, p.q] [alpha] [x += alpha p, r -= alpha q,
 // ||r||^2] [latch] (host check / FP64 certification) [FFT passes of M r; the
 // z pass reduces r.z] [beta] [last pass: p = M r + beta p].  With the fused
-// four-step forward pass the x/r update and ||r||^2 ride on the forward x
+// forward pass the x/r update and ||r||^2 ride on the forward x
 // pass of the next preconditioner apply (its input is the updated r); a
 // certification that replaces r repeats that pass on the new r.
 template <typename T>
@@ -262,10 +262,10 @@ struct Steps {
 };
 
 // Whether a solve with these steps keeps the residual as its x spectrum: mixed
-// mode (FP32 spectra), direction ring, fused forward pass, four-step x and y
-// passes, and room for the R^ buffer (allocated here, once; if it does not
-// fit, the solver keeps the real-space residual from then on, so eager runs
-// and captured blocks always agree).  At 256^3 x 6 this takes the forward
+// mode (FP32 spectra), direction ring, fused forward pass, and room for the
+// R^ buffer (allocated here, once; if it does not fit, the solver keeps the
+// real-space residual from then on, so eager runs and captured blocks always
+// agree).  At 256^3 x 6 this takes the forward
 // pass from 4.8 to 3.6 GB.
 template <typename T>
 bool spectral_on(vxl_solver* s, const Steps<T>& steps) {
@@ -772,6 +772,8 @@ int run_impl(vxl_solver* s, const double* macro_host, double tol, int max_iter, 
 }
 
 // ---- block CG over the load cases ---------------------------------------------
+// (Its FP32 residuals are not scaled by powers of two as run_impl's are: a load
+// whose right-hand side is rounding noise can stop before its certificate.)
 // Y[idx][j] = G[idx][idx]^-1 B[idx][j] for the columns j with cols[j] != 0 (G
 // symmetric, R x R row major; other entries of Y are 0).  idx starts as the
 // kept directions and loses every direction whose Cholesky pivot falls below

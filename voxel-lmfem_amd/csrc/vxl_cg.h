@@ -208,8 +208,8 @@ template <typename T>
 int precond_cg_rest(vxl_precond* pc, int nrhs, T* p, double* rz_partial, const double* beta,
                     const std::function<int()>& mid, const int* active, hipStream_t s, const T* p_old = nullptr,
                     bool sr = false, const BetaFold* fold = nullptr);
-// Whether the spectral-residual form is available (FP32 spectrum storage,
-// four-step x and y passes; VXL_SPECTRAL_RESIDUAL=0 turns it off), and the
+// Whether the spectral-residual form is available (FP32 spectrum storage;
+// VXL_SPECTRAL_RESIDUAL=0 turns it off), and the
 // allocation of its R^ buffer (nrhs_max spectra; once, outside any capture).
 bool precond_spectral_residual_ok(const vxl_precond* pc);
 int precond_residual_spectrum(vxl_precond* pc);
@@ -238,7 +238,7 @@ struct vxl_solver {
   double* partial;
   double* partial_st;  // stencil p.q partials
   double* partial_rz;  // FFT z-pass r.z partials (Parseval)
-  double* partial_fx;  // ||r||^2 partials of the fused forward x pass (four-step x only)
+  double* partial_fx;  // ||r||^2 partials of the fused forward x pass
   int precond_kind;    // VXL_PRECOND_FFT or VXL_PRECOND_JACOBI
   int element;         // element of the cell when the preconditioner was built
   double* dinv64;      // Jacobi: 1 / diag K (3N FP64)
