@@ -112,3 +112,14 @@ def test_misaligned_axes_take_the_numpy_route():
     assert not pm._native_axes((ori["axis1"], ori["axis2"]), shape, sels, 16, 2, kept)
     got = pm.check_frames(ori, shape, sels, chunk=16, workers=2, keep=True)
     assert all(np.array_equal(g, ori[k].reshape(-1, 3)[10:70]) for g, k in zip(got, ("axis1", "axis2")))
+
+
+@pytest.mark.parametrize("label", [2 ** 64 + 1, -2 ** 64 + 1, 2 ** 63])
+def test_labels_past_64_bits_match_nothing(label):
+    """They must not wrap to a label that is there."""
+    flat = np.array([1, 2, 1, -2 ** 31], dtype=np.int32)
+    try:
+        got = pm.voxels_with_label(flat, label)
+    except OverflowError:   # what NumPy's comparison raises in some versions
+        return
+    assert len(got) == 0

@@ -147,7 +147,7 @@ def voxels_with_label(flat, label):
     piece by piece on a thread pool."""
     from . import _native
     native = _native.host_labels(flat)
-    if native is not None:
+    if native is not None and -(1 << 63) <= label < 1 << 63:   # what the library's argument holds
         import ctypes
         lib, ptr, size, signed = native
         out, found = np.empty(flat.size, dtype=np.int64), ctypes.c_int64()
