@@ -1,5 +1,5 @@
 // FFT passes for axes of any length (instantiated per precision by
-// fftgen_f32.hip and fftgen_f64.hip).
+// fftgen_f32.hip and fftgen_f64.hip, and fftgen_z32.hip and fftgen_z64.hip).
 //
 // An axis of n = n1 * n2 runs as two steps over columns ("pencils") whose
 // entries sit in LDS as L[entry][column]:
@@ -1134,9 +1134,10 @@ int launch_gen_z(const AxisPlan& plan, const GenShape& sh, const Tables<T>& tb, 
   return VXL_OK;
 }
 
-// Explicit instantiation of every launcher for one precision.
+// Explicit instantiation for one precision: the plans with the x and y launchers,
+// and the z launcher, whose kernels take as long to compile as all the others.
 #define VXL_FFTGEN_INSTANCES(T)                                                                                       \
-  template AxisPlan make_axis_plan<T>(int, bool);                                                                         \
+  template AxisPlan make_axis_plan<T>(int, bool);                                                                     \
   template GenShape gen_shape_y<T>(const AxisPlan&);                                                                  \
   template GenShape gen_shape_z<T>(const AxisPlan&);                                                                  \
   template GenShape gen_shape_x<T>(const AxisPlan&, int);                                                             \
@@ -1146,7 +1147,8 @@ int launch_gen_z(const AxisPlan& plan, const GenShape& sh, const Tables<T>& tb, 
   template int launch_gen_c2r<T>(const GenX<T>&, int, const CT<T>::type*, T*, const double*, const T*,                   \
                                  const BetaFold&, hipStream_t);                                                     \
   template int launch_gen_y<T>(const AxisPlan&, const GenShape&, const CT<T>::type*, bool, int, CT<T>::type*,         \
-                               const CT<T>::type*, int, int, int64_t, const int*, hipStream_t);                       \
+                               const CT<T>::type*, int, int, int64_t, const int*, hipStream_t);
+#define VXL_FFTGEN_Z_INSTANCES(T)                                                                                     \
   template int launch_gen_z<T>(const AxisPlan&, const GenShape&, const Tables<T>&, int, CT<T>::type*, int, int, T, T,  \
                                T, int64_t, const int*, int, double*, const double*, int, hipStream_t);
 
