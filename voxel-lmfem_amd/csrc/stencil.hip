@@ -433,24 +433,24 @@ int launch_residual_apply(const vxl_cell* cell, int nrhs, const double* u, const
   const bool sc = cell->mat.scale != nullptr;
   if (cell->ortho && !sc && cell->element == VXL_ELEMENT_FI)
     return launch_residual_ortho(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale, s);
-  switch (cell->mat.index_kind) {
-    case VXL_INDEX_U8:
-      return sc ? launch_resid_impl<uint8_t, true>(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale, s)
-                : launch_resid_impl<uint8_t, false>(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale, s);
-    case VXL_INDEX_U16:
-      return sc ? launch_resid_impl<uint16_t, true>(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale, s)
-                : launch_resid_impl<uint16_t, false>(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale, s);
-    case VXL_INDEX_I32:
-      return sc ? launch_resid_impl<int32_t, true>(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale, s)
-                : launch_resid_impl<int32_t, false>(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale, s);
-  }
-  return fail("unknown material index kind");
+  return with_default_tile<double>(cell, nrhs, [&](auto t) {
+    using O = decltype(t);
+    return by_index(cell, [&](auto tag) {
+      using Idx = decltype(tag);
+      return sc ? launch_resid_impl<Idx, true, O::tx, O::ty>(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale, s)
+                : launch_resid_impl<Idx, false, O::tx, O::ty>(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale,
+                                                              s);
+    });
+  });
 }
 
 int residual_apply_blocks(const vxl_cell* cell, int nrhs) {
-  int tx, tiles, chunks, zc;
-  apply_grid<double, ResidTile::tx, ResidTile::ty>(cell, nrhs, tx, tiles, chunks, zc, kMinChunkPlanes);
-  return tiles * chunks;
+  return with_default_tile<double>(cell, nrhs, [&](auto t) {
+    using O = decltype(t);
+    int tx, tiles, chunks, zc;
+    apply_grid<double, O::tx, O::ty>(cell, nrhs, tx, tiles, chunks, zc, kMinChunkPlanes);
+    return tiles * chunks;
+  });
 }
 
 // Runtime tile choice -> template instance (the C3D8R-HG element runs the
@@ -470,15 +470,6 @@ template <typename T>
 bool takes_ortho(const vxl_cell* cell) {
   return cell->ortho && cell->element == VXL_ELEMENT_FI && !cell->mat.scale &&
          cell->variant[std::is_same<T, double>::value ? 1 : 0] == 3;
-}
-
-// The default option's tile (the C3D8R-HG element has no other).
-template <typename T, typename F>
-int with_default_tile(const vxl_cell* cell, int nrhs, F&& f) {
-  if constexpr (std::is_same<T, double>::value)
-    return wide_f64(cell, nrhs) ? f(WideTile()) : f(ResidTile());
-  else
-    return f(TileOption<float, kTilesF32[0]>());
 }
 
 template <typename T>

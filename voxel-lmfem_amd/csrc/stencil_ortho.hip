@@ -35,9 +35,12 @@ template int launch_apply_ortho<double>(const vxl_cell*, int, const double*, dou
 
 int launch_residual_ortho(const vxl_cell* cell, int nrhs, const double* u, const double* f, float* r32, double* r64,
                           const int* active, double* partial, int* blocks, const double* rscale, hipStream_t s) {
-  return by_index(cell, [&](auto tag) {
-    return launch_resid_impl<decltype(tag), false, true>(cell, nrhs, u, f, r32, r64, active, partial, blocks, rscale,
-                                                         s);
+  return with_default_tile<double>(cell, nrhs, [&](auto t) {
+    using O = decltype(t);
+    return by_index(cell, [&](auto tag) {
+      return launch_resid_impl<decltype(tag), false, O::tx, O::ty, true>(cell, nrhs, u, f, r32, r64, active, partial,
+                                                                         blocks, rscale, s);
+    });
   });
 }
 

@@ -322,7 +322,7 @@ struct TileOption {
   static constexpr bool kSquare = std::is_same<T, double>::value && OPT == kTilesF64[0];
   static constexpr int tx = kSquare ? 16 : 32, ty = kSquare ? 14 : OPT;
 };
-using ResidTile = TileOption<double, kTilesF64[0]>;
+using SquareTile = TileOption<double, kTilesF64[0]>;
 struct WideTile {  // FP64's option 6 where wide_f64 holds
   static constexpr int tx = 32, ty = 6;
 };
@@ -958,7 +958,7 @@ inline bool wide_f64(const vxl_cell* cell, int nrhs) {
     const int64_t columns = int64_t((g.nx + tx - 1) / tx) * ((g.ny + ty - 1) / ty) * nrhs;
     return chunk_rule(columns, g.nz, kMinChunkPlanes, chunk_limit(columns, g.nz), depth);
   };
-  return steps(WideTile::tx, WideTile::ty) <= steps(ResidTile::tx, ResidTile::ty);
+  return steps(WideTile::tx, WideTile::ty) <= steps(SquareTile::tx, SquareTile::ty);
 }
 
 // most: the largest number of chunks any depth setting can give.
@@ -1046,13 +1046,12 @@ int launch_apply_impl(const vxl_cell* cell, int nrhs, const T* u, T* out, hipStr
   return VXL_OK;
 }
 
-// Certification residual r = f - K u (FP64 operator, default FP64 tile,
+// Certification residual r = f - K u (FP64 operator, default FP64 option,
 // schedule 3, chunk depth by apply_grid's rule): u FP64, r into r32 or
 // r64, ||r||^2 partials per workgroup; systems with active == 0 are skipped.
-template <typename Idx, bool kScale, bool kOrtho = false>
+template <typename Idx, bool kScale, int TX, int TY, bool kOrtho = false>
 int launch_resid_impl(const vxl_cell* cell, int nrhs, const double* u, const double* f, float* r32, double* r64,
                       const int* active, double* partial, int* blocks, const double* rscale, hipStream_t s) {
-  constexpr int TX = ResidTile::tx, TY = ResidTile::ty;
   using TL = Tile<TX, TY>;
   ApplyArgs<double> a{};
   set_groups(a, cell, nrhs);
@@ -1102,6 +1101,15 @@ int launch_resid_impl(const vxl_cell* cell, int nrhs, const double* u, const dou
 #undef VXL_R
   VXL_HIP(hipGetLastError());
   return VXL_OK;
+}
+
+// The default option's tile (the C3D8R-HG element and the certification have no other).
+template <typename T, typename F>
+int with_default_tile(const vxl_cell* cell, int nrhs, F&& f) {
+  if constexpr (std::is_same<T, double>::value)
+    return wide_f64(cell, nrhs) ? f(WideTile()) : f(SquareTile());
+  else
+    return f(TileOption<float, kTilesF32[0]>());
 }
 
 // Runtime tile choice -> template instance.
